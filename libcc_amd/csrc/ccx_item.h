@@ -68,6 +68,11 @@ __host__ __device__ constexpr int wsrc_comp(int p, int s, int t)
     return wsrc(p, pi);
 }
 
+// Even orderings 0, 3, 4 and odd ones 1, 2, 5, and the rank of an ordering among its parity.
+__device__ constexpr int EVEN[3] = {0, 3, 4}, ODD[3] = {1, 2, 5};
+__host__ __device__ constexpr bool is_even(int q) { return q == 0 || q == 3 || q == 4; }
+__host__ __device__ constexpr int parity_rank(int q) { return q <= 1 ? 0 : q <= 3 ? 1 : 2; }
+
 // Item modes: which orderings are accumulated.  Equal blocks of the orbit (AAC: A = B, ACC:
 // B = C, AAA) relate orderings by transposes inside the cube, equal occupied indices of the tuple
 // ((i,j,j), (i,i,j)) pointwise; a degenerate tuple on an orbit with two equal blocks uses both.
@@ -324,19 +329,48 @@ __device__ __forceinline__ void run_phase(const TriplesArgs &g, const ItemCtx &i
     });
 }
 
-__device__ __forceinline__ double wave_sum(double v)
+// Sums over groups of lanes, every lane of the group getting the sum.  Within a row of 16 lanes by
+// row rotations (DPP), across rows by the row-swap instructions: no LDS access, where a
+// ds_bpermute-based shuffle made the reductions of an item's epilogue 15.6 kcycles (of 475 per item
+// at no=24, nu=216).  The additions are those of an xor butterfly, bit for bit: after the step of
+// distance d the values repeat every d lanes, so lane l + d/2 (mod 16) holds what lane l ^ d/2 does.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v)
 {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
 }
 
 __device__ __forceinline__ double group16_sum(double v)
 {
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+    v += dpp_f64<0x128>(v);   // row_ror:8
+    v += dpp_f64<0x124>(v);   // row_ror:4
+    v += dpp_f64<0x122>(v);   // row_ror:2
+    v += dpp_f64<0x121>(v);   // row_ror:1
     return v;
 }
+
+// v of this lane plus v of lane ^ 16 / lane ^ 32
+__device__ __forceinline__ double add_xor16(double v)
+{
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)u, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
+    return __builtin_bit_cast(double, (unsigned long long)hi[0] << 32 | lo[0]) +
+           __builtin_bit_cast(double, (unsigned long long)hi[1] << 32 | lo[1]);
+}
+__device__ __forceinline__ double add_xor32(double v)
+{
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
+    return __builtin_bit_cast(double, (unsigned long long)hi[0] << 32 | lo[0]) +
+           __builtin_bit_cast(double, (unsigned long long)hi[1] << 32 | lo[1]);
+}
+
+__device__ __forceinline__ double wave_sum(double v) { return group16_sum(add_xor16(add_xor32(v))); }
 
 // Element (a,b,c) of a 16^3 cube in LDS.
 __device__ __forceinline__ int cidx(int a, int b, int c) { return a * CSTR_A + b * CSTR_B + c; }

@@ -290,19 +290,19 @@ __global__ void pack_split_kernel(const double *__restrict__ src, unsigned char 
 // ---------------------------------------------------------------------------------
 namespace {
 
-// FK: 0 FP64 slabs, 1 FP32 slabs (16 K per fragment load), 2-4 split slices (SplitCfg).  Always
-// inlined: as a called function every item paid a call frame and callee-saved register
-// spills in scratch memory (0.06 TB of writes per launch at no=24, nu=216).
-template <int MODE, class T, int FK>
-__device__ __forceinline__ void do_item(const TriplesArgs &g, double *lds, double (*red)[112], const ItemCtx &it, long long item,
-                        int tkind, int mult, bool swap_bc, int wave, int lane, int tid)
+// Energy, v1 partials and the optional W store of one item from its six w (layout L).  One copy for
+// every mode: the modes differ in the sweeps only (dispatch in triples_kernel), and the FP64 kernel
+// is 80 KB of code instead of 324 KB.  Bound by the FP64 VALU and, before the reductions went to DPP
+// and row swaps, by their LDS shuffles.  Of 475 kcycles per item at no=24, nu=216 the point loop took
+// 15.8 and now takes 10.4 (two multiply-adds per v1 term instead of five operations), the
+// reductions 15.9 and now 7.5; the kernel went from 1137 to 1109 ms there, from 4.79 to 4.49 ms
+// at no=8, nu=120, where an item's sweeps are half as long, and FP32 from 783 to 753 ms.
+template <class T, int FK>
+__device__ __forceinline__ void item_epilogue(const TriplesArgs &g, double *lds, double (*red)[112], const ItemCtx &it,
+                                              const typename Mfma<T>::acc_t (&acc)[6][BPW],
+                                              const f4 (&acc1)[FK == 4 ? 6 : 1][BPW], long long item, int tkind,
+                                              int mult, bool swap_bc, int wave, int lane, int tid)
 {
-    typename Mfma<T>::acc_t acc[6][BPW];
-    f4 acc1[FK == 4 ? 6 : 1][BPW];   // two-accumulator split form: the levels above 0
-    if constexpr (FK >= 2) item_w_split<MODE, FK>(g, lds, it, acc, acc1, wave, lane);
-    else if constexpr (FK == 1) item_w_f32v<MODE>(g, lds, it, acc, wave, lane);
-    else item_w<MODE, T>(g, lds, it, acc, wave, lane);
-
     const int A = it.blk[0], B = it.blk[1], C = it.blk[2];
     // ---- stage the 36 VOE sub-blocks: [ordered tuple-position pair][ordered block pair]
     for (int idx = tid; idx < 36 * 16 * 4; idx += NTHR) {
@@ -353,6 +353,14 @@ __device__ __forceinline__ void do_item(const TriplesArgs &g, double *lds, doubl
             const double ev = w[0] + w[3] + w[4], od = w[1] + w[2] + w[5];
             const double sq = w[0] * w[0] + w[1] * w[1] + w[2] * w[2] + w[3] * w[3] + w[4] * w[4] + w[5] * w[5];
             esum += (6.0 * sq + 2.0 * ev * ev + 2.0 * od * od - 8.0 * ev * od) * inv;
+            // Z = 2 w[q0] - 2 w[q1] - w[q2] + w[q3] is a combination of two differences of an even and
+            // an odd ordering, so with the nine differences over D at hand each of the 36 terms is
+            // two multiply-adds.
+            double d[3][3];
+#pragma unroll
+            for (int x = 0; x < 3; ++x)
+#pragma unroll
+                for (int y = 0; y < 3; ++y) d[x][y] = (w[EVEN[x]] - w[ODD[y]]) * inv;
             const int el[3] = {al, bl, cl};
             static_for<6>([&](auto S) __attribute__((always_inline)) {
                 constexpr int s = decltype(S)::value;
@@ -364,13 +372,17 @@ __device__ __forceinline__ void do_item(const TriplesArgs &g, double *lds, doubl
                     constexpr int q1 = wsrc_comp(p, s, 2);   // sigma o (1,0,2)
                     constexpr int q2 = wsrc_comp(p, s, 1);   // sigma o (0,2,1)
                     constexpr int q3 = wsrc_comp(p, s, 3);   // sigma o (1,2,0)
+                    static_assert(is_even(q0) == is_even(q3) && is_even(q1) == is_even(q2) && is_even(q0) != is_even(q1),
+                                  "parities of a Z term");
+                    constexpr int e0 = parity_rank(is_even(q0) ? q0 : q1), o0 = parity_rank(is_even(q0) ? q1 : q0);
+                    constexpr int e1 = parity_rank(is_even(q0) ? q3 : q2), o1 = parity_rank(is_even(q0) ? q2 : q3);
                     constexpr int qr = pair_index(PERM[p][1], PERM[p][2]);
-                    const double z = 2.0 * w[q0] - 2.0 * w[q1] - w[q2] + w[q3];
+                    const double za = fma(2.0, d[e0][o0], d[e1][o1]);
+                    const double z = is_even(q0) ? za : -za;
                     const double vv = lds[(qr * 6 + bpair) * VBLK + el[r1] * VSTR + el[r2]];
-                    const double c = z * vv * inv;
-                    if constexpr (r0 == 0) va[v][PERM[p][0]] += c;
-                    else if constexpr (r0 == 1) vb[bb][PERM[p][0]] += c;
-                    else vc[PERM[p][0]] += c;
+                    if constexpr (r0 == 0) va[v][PERM[p][0]] = fma(z, vv, va[v][PERM[p][0]]);
+                    else if constexpr (r0 == 1) vb[bb][PERM[p][0]] = fma(z, vv, vb[bb][PERM[p][0]]);
+                    else vc[PERM[p][0]] = fma(z, vv, vc[PERM[p][0]]);
                 });
             });
             if (g.wout != nullptr) {
@@ -402,9 +414,7 @@ __device__ __forceinline__ void do_item(const TriplesArgs &g, double *lds, doubl
         }
 #pragma unroll
     for (int p = 0; p < 3; ++p) {        // role c: rows lane&15
-        double s = vc[p];
-        s += __shfl_xor(s, 16, 64);
-        s += __shfl_xor(s, 32, 64);
+        const double s = add_xor32(add_xor16(vc[p]));
         if (lane < 16) rw[54 + lane * 3 + p] = s;
     }
     {
@@ -445,10 +455,14 @@ __global__ void __launch_bounds__(NTHR, 1) triples_kernel(TriplesArgs g)
     extern __shared__ double lds[];
     __shared__ double red[NWAVE][112];
     __shared__ long long next_item;
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     for (;;) {
+        // The lane number is made new for every item: the LDS addresses that follow from it are then
+        // computed where they are used, not kept through the sweeps (that is, in scratch).
+        int lane = tid & 63;
+        asm volatile("" : "+v"(lane));
         // Work order: block triple major (default), so the tuples of one block triple run
         // together and the operand panels they share stay in the last-level cache (34% less
         // L2 miss traffic than tuple major at no=24, nu=216); tuple major on request.
@@ -468,18 +482,25 @@ __global__ void __launch_bounds__(NTHR, 1) triples_kernel(TriplesArgs g)
         int tkind, mult;
         ItemCtx it = make_item_ctx(g.tuples, g.blocks, t, q, tkind, mult);
         const bool swap_bc = ragged_block_to_b(g, it, mult);
+        typename Mfma<T>::acc_t acc[6][BPW];
+        f4 acc1[FK == 4 ? 6 : 1][BPW];   // two-accumulator split form: the levels above 0
+        auto sweeps = [&](auto M) __attribute__((always_inline)) {
+            constexpr int MODE = decltype(M)::value;
+            if constexpr (FK >= 2) item_w_split<MODE, FK>(g, lds, it, acc, acc1, wave, lane);
+            else if constexpr (FK == 1) item_w_f32v<MODE>(g, lds, it, acc, wave, lane);
+            else item_w<MODE, T>(g, lds, it, acc, wave, lane);
+        };
         if constexpr (pair_modes(FK)) {
-            dispatch_mode(tkind, mult, it, [&](auto M) __attribute__((always_inline)) {
-                do_item<decltype(M)::value, T, FK>(g, lds, red, it, item, tkind, mult, swap_bc, wave, lane, tid);
-            });
+            dispatch_mode(tkind, mult, it, sweeps);
         } else {
-            if (tkind == 2) do_item<M_IJJ, T, FK>(g, lds, red, it, item, tkind, mult, swap_bc, wave, lane, tid);
-            else if (tkind == 3) do_item<M_IIJ, T, FK>(g, lds, red, it, item, tkind, mult, swap_bc, wave, lane, tid);
-            else if (mult == 1) do_item<M_FULL, T, FK>(g, lds, red, it, item, tkind, mult, swap_bc, wave, lane, tid);
-            else if (mult == 6) do_item<M_AAA, T, FK>(g, lds, red, it, item, tkind, mult, swap_bc, wave, lane, tid);
-            else if (it.blk[0] == it.blk[1]) do_item<M_AAC, T, FK>(g, lds, red, it, item, tkind, mult, swap_bc, wave, lane, tid);
-            else do_item<M_ACC, T, FK>(g, lds, red, it, item, tkind, mult, swap_bc, wave, lane, tid);
+            if (tkind == 2) sweeps(std::integral_constant<int, M_IJJ>{});
+            else if (tkind == 3) sweeps(std::integral_constant<int, M_IIJ>{});
+            else if (mult == 1) sweeps(std::integral_constant<int, M_FULL>{});
+            else if (mult == 6) sweeps(std::integral_constant<int, M_AAA>{});
+            else if (it.blk[0] == it.blk[1]) sweeps(std::integral_constant<int, M_AAC>{});
+            else sweeps(std::integral_constant<int, M_ACC>{});
         }
+        item_epilogue<T, FK>(g, lds, red, it, acc, acc1, item, tkind, mult, swap_bc, wave, lane, tid);
     }
 }
 
