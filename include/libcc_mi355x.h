@@ -113,7 +113,7 @@ int ccx_w_abc(ccx_ctx *ctx, int64_t a, int64_t b, int64_t c, double *v3);
 /* E[T] (etd) re-summed over virtual triples: sum over a>b>c of X_abc plus half the sum of
  * X_abb and X_aab, X_abc = sum_ijk W [8W - 4(W_ikj + W_kji + W_jik) + 2(W_kij + W_jki)] / D
  * on the cubes of ccx_w_abc.  Equal to the etd of ccx_energy up to summation order; a
- * cross-check route (FP64 FMA, not the matrix cores), not the fast path. */
+ * cross-check route, not the fast path. */
 int ccx_energy_abc(ccx_ctx *ctx, double *etd);
 
 /* Timing of the last ccx_energy call in milliseconds (HIP events around the

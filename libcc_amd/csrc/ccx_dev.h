@@ -47,6 +47,12 @@ int ccx_hip_t1wt3(const double *w, const double *voe6, double dijk, const double
 /* virtual-triple view (ccx_abc.hip): trip holds (a, b, c, kind) per triple, 0-based */
 int ccx_hip_w_abc(const void *axr, const void *bx, const int *trip, int ntrip, int no, int nu, int nb, int kp,
                   double *w, void *stream);
+size_t ccx_hip_abc_a_doubles(int no, int nu, int kp);
+size_t ccx_hip_abc_b_doubles(int no, int nu, int kp);
+int ccx_hip_abc_pack(const void *axr, const void *bx, double *axt, double *bxt, int no, int nu, int nb, int kp,
+                     void *stream);
+int ccx_hip_w_abc_packed(const double *axt, const double *bxt, const int *trip, int ntrip, int no, int nu, int kp,
+                         double *w, void *stream);
 int ccx_hip_x_abc(const double *w, const int *trip, int ntrip, int no, const double *eh, const double *ep,
                   double *x, void *stream);
 

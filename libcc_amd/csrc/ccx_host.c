@@ -574,7 +574,7 @@ int ccx_energy_abc(ccx_ctx *c, double *etd)
     if (batch > ntrip) batch = ntrip;
     int rc = CCX_OK;
     int *h_trip = NULL, *d_trip = NULL;
-    double *d_w = NULL, *d_x = NULL, *h_x = NULL;
+    double *d_w = NULL, *d_x = NULL, *h_x = NULL, *d_axt = NULL, *d_bxt = NULL;
     double sum = 0.0;
     if (ntrip > 0) {
         h_trip = (int *)malloc(sizeof(int) * 4 * (size_t)batch);
@@ -583,14 +583,28 @@ int ccx_energy_abc(ccx_ctx *c, double *etd)
         DALLOC(d_trip, 4 * batch);
         DALLOC(d_w, no3 * batch);
         DALLOC(d_x, batch);
+        /* the packed copies of the matrix-core route (axt has the size of a slab, its occupied index
+         * padded to 16); without room for them the triples go through w_abc_kernel */
+        if (ccx_hip_malloc((void **)&d_axt, sizeof(double) * ccx_hip_abc_a_doubles((int)c->no, (int)c->nu, (int)c->kp)) != 0 ||
+            ccx_hip_malloc((void **)&d_bxt, sizeof(double) * ccx_hip_abc_b_doubles((int)c->no, (int)c->nu, (int)c->kp)) != 0) {
+            (void)ccx_hip_last_error();   /* handled here: clears it for the launches below */
+            ccx_hip_free(d_axt);
+            d_axt = d_bxt = NULL;
+        }
+        if (d_axt && ccx_hip_abc_pack(c->d_axr, c->d_bx, d_axt, d_bxt, (int)c->no, (int)c->nu, (int)c->nb, (int)c->kp,
+                                      c->stream) != 0) {
+            rc = CCX_ERR_DEVICE;
+            goto fail;
+        }
     }
     /* batches in list order; the partials of each batch are added on the host in order */
     for (int64_t first = 0; first < ntrip; first += batch) {
         const int64_t n = ntrip - first < batch ? ntrip - first : batch;
         abc_triples(c->nu, first, n, h_trip);
         if (ccx_hip_memcpy_h2d(d_trip, h_trip, sizeof(int) * 4 * (size_t)n, c->stream) != 0 ||
-            ccx_hip_w_abc(c->d_axr, c->d_bx, d_trip, (int)n, (int)c->no, (int)c->nu, (int)c->nb, (int)c->kp, d_w,
-                          c->stream) != 0 ||
+            (d_axt ? ccx_hip_w_abc_packed(d_axt, d_bxt, d_trip, (int)n, (int)c->no, (int)c->nu, (int)c->kp, d_w, c->stream)
+                   : ccx_hip_w_abc(c->d_axr, c->d_bx, d_trip, (int)n, (int)c->no, (int)c->nu, (int)c->nb, (int)c->kp, d_w,
+                                   c->stream)) != 0 ||
             ccx_hip_x_abc(d_w, d_trip, (int)n, (int)c->no, c->d_eh, c->d_ep, d_x, c->stream) != 0 ||
             ccx_hip_memcpy_d2h(h_x, d_x, sizeof(double) * (size_t)n, c->stream) != 0) {
             rc = CCX_ERR_DEVICE;
@@ -601,7 +615,7 @@ int ccx_energy_abc(ccx_ctx *c, double *etd)
     *etd = sum;
 fail:
     free(h_trip); free(h_x);
-    ccx_hip_free(d_trip); ccx_hip_free(d_w); ccx_hip_free(d_x);
+    ccx_hip_free(d_trip); ccx_hip_free(d_w); ccx_hip_free(d_x); ccx_hip_free(d_axt); ccx_hip_free(d_bxt);
     return rc;
 }
 

@@ -66,6 +66,21 @@ def test_energy_abc_matches_ijk(no, nu, seed):
     ctx.close()
 
 
+# Edges of the matrix-core route's tiles: no^2 below, at and above multiples of 16 pair tiles (one to
+# four tiles per wave, one or four waves per triple), no below, at and above one row tile.
+@pytest.mark.parametrize("no,nu", [(2, 7), (4, 16), (5, 18), (7, 12), (8, 17), (9, 10), (12, 6), (16, 5), (17, 4)],
+                         ids=lambda v: str(v))
+def test_energy_abc_tile_edges(no, nu):
+    inp = synth.make_inputs(no, nu, 40 + no)
+    ctx = TriplesContext(no, nu)
+    ctx.load(inp)
+    print(f"energy_abc no={no} nu={nu}", flush=True)
+    want = dense.energies(inp)["etd"] if no <= 9 else ctx.energy()["etd"]
+    # sums of about no^3 nu^3 FP64 terms of both signs in another order
+    assert abs(ctx.energy_abc() - want) <= 1e-12 * abs(want)
+    ctx.close()
+
+
 def test_abc_errors():
     ctx = TriplesContext(2, 5)
     v3 = np.zeros(8)
