@@ -17,16 +17,16 @@ int ccx_hip_cu_count(int *n);
 const char *ccx_hip_last_error(void);
 int ccx_hip_lds_bytes(void);
 
-int ccx_hip_unpack_vvvo(const double *packed, double *full, int no, int nu, void *stream);
+int ccx_hip_zero_flag(unsigned int *d_flag, void *stream);
 int ccx_hip_nonfinite(const double *const *p, const size_t *n, int narr, unsigned int *d_flag, int *nonfinite,
                       void *stream);
-int ccx_hip_pack(int form, const double *vvvo, const double *t2, const double *vm, const double *voe, void *axr,
-                 void *axc, void *bx, double *voep, int no, int nu, int nup, int kp, void *stream);
-int ccx_hip_pack_ax_one(const double *vvvo_x, const double *t2_x, double *axr_x, double *axc_x, int no, int nu,
-                        int nup, int kp, void *stream);
+int ccx_hip_pack(int vvvo_layout, const double *vvvo, const double *t2, const double *vm, const double *voe,
+                 const double *eh, const double *ep, const double *t1, double *axr, double *axc, double *bx,
+                 double *voep, double *ehp, double *epp, double *t1p, int no, int nu, int nup, int kp, void *stream);
+int ccx_hip_pack_ax_one(int layout, const double *cube, const double *t2_x, double *axr_x, double *axc_x, int no,
+                        int nu, int nup, int kp, void *stream);
 int ccx_hip_pack_pair(const double *t2_yz, const double *vm_zy, const double *voe_yz, double *bx_yz,
                       double *voep_yz, int no, int nu, int nup, int kp, void *stream);
-int ccx_hip_ve_to_vvvo(const double *ve, double *vvvo_x, int nu, void *stream);
 int ccx_hip_triples(int form, const void *axr, const void *axc, const void *bx, const double *voep,
                     const double *eh, const double *ep, const int *tuples, const int *blocks, double *e_part,
                     double *v1_part, double *wout, unsigned int *counter, int no, int nu, int nup, int kp,
@@ -37,9 +37,8 @@ int ccx_hip_pack_split(int form, const double *axr, const double *axc, const dou
                        unsigned long long *dmax, int no, int nb, int kp, int kps, double *wscale, void *stream);
 int ccx_hip_pack_f32v(const double *axr, const double *axc, const double *bx, float *axr32, float *axc32,
                       float *bx32, int no, int nb, int kp, int kpf, void *stream);
-int ccx_hip_finalize(const double *e_part, const double *v1_part, const int *tuples, const int *blocks,
-                     const double *t1, double *v1t, double *v1, double *out, int no, int nu, int ntup, int nblk,
-                     void *stream);
+int ccx_hip_finalize(double *e_part, const double *v1_part, const int *tuples, const double *t1, double *v1t,
+                     double *v1, double *out, int no, int nu, int ntup, int nblk, void *stream);
 
 int ccx_hip_t1wt3(const double *w, const double *voe6, double dijk, const double *ep, int nu, double *x3,
                   double *v1p, void *stream);

@@ -199,12 +199,11 @@ static int finite_all(const double *p, size_t n)
 /* Build the packed operand slabs and small arrays from device-resident raw inputs. */
 static int build_from_device(ccx_ctx *c, const double *d_eh, const double *d_ep_raw, const double *d_t1,
                              const double *d_t2, const double *d_vm, const double *d_voe,
-                             const double *d_vvvo_full)
+                             const double *d_vvvo, int vvvo_layout)
 {
     int rc = CCX_OK;
     const int64_t no = c->no, nu = c->nu, nup = c->nup, nb = c->nb, kp = c->kp;
     const int64_t nitems = c->ntup * c->nblk;
-    double *h_ep = NULL;
     if (c->d_axr) goto allocated; /* buffers depend only on the dimensions: reuse */
     DALLOC(c->d_axr, no * nb * nb * kp * 256);
     DALLOC(c->d_axc, no * nb * nb * kp * 256);
@@ -225,24 +224,14 @@ allocated:
     c->loaded = 0;
     c->f32_ready = 0;
     c->split_ready = 0;
-    if (ccx_hip_pack(0, d_vvvo_full, d_t2, d_vm, d_voe, c->d_axr, c->d_axc, c->d_bx, c->d_voep, (int)no, (int)nu,
-                     (int)nup, (int)kp, c->stream) != 0) { rc = CCX_ERR_DEVICE; goto fail; }
-    /* eps_virtual padded to nup with finite values (padded elements carry W = 0) */
-    h_ep = (double *)malloc(sizeof(double) * (size_t)nup);
-    if (!h_ep) { rc = CCX_ERR_ALLOC; goto fail; }
-    if (ccx_hip_memcpy_d2h(h_ep, d_ep_raw, sizeof(double) * (size_t)nu, c->stream) != 0) { rc = CCX_ERR_DEVICE; goto fail; }
-    for (int64_t a = nu; a < nup; ++a) h_ep[a] = 1.0e3;
-    if (ccx_hip_memcpy_h2d(c->d_ep, h_ep, sizeof(double) * (size_t)nup, c->stream) != 0 ||
-        ccx_hip_memcpy_d2d(c->d_eh, d_eh, sizeof(double) * (size_t)no, c->stream) != 0 ||
-        ccx_hip_memcpy_d2d(c->d_t1, d_t1, sizeof(double) * (size_t)(no * nu), c->stream) != 0 ||
+    if (ccx_hip_pack(vvvo_layout, d_vvvo, d_t2, d_vm, d_voe, d_eh, d_ep_raw, d_t1, c->d_axr, c->d_axc, c->d_bx,
+                     c->d_voep, c->d_eh, c->d_ep, c->d_t1, (int)no, (int)nu, (int)nup, (int)kp, c->stream) != 0 ||
         ccx_hip_memcpy_h2d(c->d_tuples, c->h_tuples, sizeof(int) * 4 * (size_t)c->ntup, c->stream) != 0 ||
         ccx_hip_memcpy_h2d(c->d_blocks, c->h_blocks, sizeof(int) * 4 * (size_t)c->nblk, c->stream) != 0 ||
         ccx_hip_sync(c->stream) != 0) { rc = CCX_ERR_DEVICE; goto fail; }
-    free(h_ep);
     c->loaded = 1;
     return CCX_OK;
 fail:
-    free(h_ep);
     free_dev(c);
     return rc;
 }
@@ -260,18 +249,11 @@ int ccx_load_device(ccx_ctx *c, const double *eh, const double *ep, const double
                              vvvo_layout == 0 ? (size_t)(nu * nu * nu * no) : (size_t)(nu * (nu + 1) / 2 * nu * no)};
         int bad = 0;
         if (!c->d_flag && ccx_hip_malloc((void **)&c->d_flag, sizeof(unsigned int)) != 0) return CCX_ERR_ALLOC;
+        if (ccx_hip_zero_flag(c->d_flag, c->stream) != 0) return CCX_ERR_DEVICE;
         if (ccx_hip_nonfinite(arr, n, 7, c->d_flag, &bad, c->stream) != 0) return CCX_ERR_DEVICE;
         if (bad) return CCX_ERR_INPUT;
     }
-    if (vvvo_layout == 0) return build_from_device(c, eh, ep, t1, t2, vm, voe, vvvo);
-    double *full = NULL;
-    if (ccx_hip_malloc((void **)&full, sizeof(double) * (size_t)(c->nu * c->nu * c->nu * c->no)) != 0)
-        return CCX_ERR_ALLOC;
-    int rc = ccx_hip_unpack_vvvo(vvvo, full, (int)c->no, (int)c->nu, c->stream) != 0 ? CCX_ERR_DEVICE : CCX_OK;
-    if (rc == CCX_OK) rc = build_from_device(c, eh, ep, t1, t2, vm, voe, full);
-    ccx_hip_sync(c->stream);
-    ccx_hip_free(full);
-    return rc;
+    return build_from_device(c, eh, ep, t1, t2, vm, voe, vvvo, vvvo_layout);
 }
 
 int ccx_load_host(ccx_ctx *c, const double *eh, const double *ep, const double *t1, const double *t2,
@@ -420,7 +402,7 @@ static int energy_run(ccx_ctx *c, int form, const int *d_tup, int64_t ntup, doub
                         form == CCX_FORM_FP32 ? (int)c->kpf : (int)c->kps, c->split_scale, c->stream) != 0)
         return CCX_ERR_DEVICE;
     if (ccx_hip_event_record(c->ev[2], c->stream) != 0) return CCX_ERR_DEVICE;
-    if (ccx_hip_finalize(c->d_epart, c->d_v1part, d_tup, c->d_blocks, c->d_t1, c->d_v1t, c->d_v1, c->d_out,
+    if (ccx_hip_finalize(c->d_epart, c->d_v1part, d_tup, c->d_t1, c->d_v1t, c->d_v1, c->d_out,
                          (int)c->no, (int)c->nu, (int)ntup, (int)c->nblk, c->stream) != 0)
         return CCX_ERR_DEVICE;
     if (ccx_hip_event_record(c->ev[3], c->stream) != 0) return CCX_ERR_DEVICE;
@@ -837,7 +819,7 @@ int ccx_gradient_form(ccx_ctx *c, int form, double *ets, double *etd, double *dt
             goto fail;
         }
     }
-    if (ccx_hip_finalize(c->d_epart, c->d_v1part, c->d_tuples, c->d_blocks, c->d_t1, c->d_v1t, c->d_v1, c->d_out,
+    if (ccx_hip_finalize(c->d_epart, c->d_v1part, c->d_tuples, c->d_t1, c->d_v1t, c->d_v1, c->d_out,
                          (int)no, (int)nu, (int)ntup, (int)nblk, c->stream) != 0) { rc = CCX_ERR_DEVICE; goto fail; }
     {
         double *outs[5] = {dvvvo, dt2, dvm, dvoe, dt1};
@@ -1007,7 +989,7 @@ void cc_triples_(double *eh, double *ep, double *v1, double *t1, double *t2, dou
 static struct {
     int64_t no, nu, nup, nb, kp, nblk;
     double *axr, *axc, *bx, *voep, *eh, *ep, *t1, *epart, *v1part, *v1t, *v1, *out;
-    double *vvvox, *t2x, *vmb, *voeb, *in, *x3, *v1p;
+    double *t2x, *vmb, *voeb, *in, *x3, *v1p;
     int *tup, *blocks;
     unsigned int *counter;
     double *h_ep;
@@ -1017,7 +999,7 @@ static struct {
 static void te_free(void)
 {
     double *d[] = {g_te.axr, g_te.axc, g_te.bx, g_te.voep, g_te.eh, g_te.ep, g_te.t1, g_te.epart, g_te.v1part,
-                   g_te.v1t, g_te.v1, g_te.out, g_te.vvvox, g_te.t2x, g_te.vmb, g_te.voeb, g_te.in, g_te.x3,
+                   g_te.v1t, g_te.v1, g_te.out, g_te.t2x, g_te.vmb, g_te.voeb, g_te.in, g_te.x3,
                    g_te.v1p};
     for (size_t q = 0; q < sizeof(d) / sizeof(d[0]); ++q) ccx_hip_free(d[q]);
     ccx_hip_free(g_te.tup);
@@ -1052,7 +1034,6 @@ static int te_ensure(int64_t no, int64_t nu)
     DALLOC(g_te.v1t, 3 * nu);
     DALLOC(g_te.v1, S * nu);
     DALLOC(g_te.out, 4);
-    DALLOC(g_te.vvvox, S * nu3);
     DALLOC(g_te.t2x, S * nu * nu * no);
     DALLOC(g_te.vmb, S * S * no * nu);
     DALLOC(g_te.voeb, S * S * nu * nu);
@@ -1121,20 +1102,12 @@ static int te_tuple(int64_t no, int64_t nu, const int64_t x[3], int kind, const 
             if (x[q] == x[p]) first = 0;
         if (!first) continue;
         if (!vvvo_src[p] || !t2x[p]) return CCX_ERR_ARG;
-        double *vx = g_te.vvvox + sl[p] * nu3;
-        if (src_kind == 0) {
-            if (ccx_hip_memcpy_h2d(g_te.in, vvvo_src[p], sizeof(double) * (size_t)nu3, NULL) != 0 ||
-                ccx_hip_ve_to_vvvo(g_te.in, vx, (int)nu, NULL) != 0)
-                return CCX_ERR_DEVICE;
-        } else {
-            if (ccx_hip_memcpy_h2d(g_te.in, vvvo_src[p], sizeof(double) * (size_t)(nutr * nu), NULL) != 0 ||
-                ccx_hip_unpack_vvvo(g_te.in, vx, 1, (int)nu, NULL) != 0)
-                return CCX_ERR_DEVICE;
-        }
+        const size_t cube = sizeof(double) * (size_t)(src_kind == 0 ? nu3 : nutr * nu);
         double *tx = g_te.t2x + sl[p] * nu2 * no;
-        if (ccx_hip_memcpy_h2d(tx, t2x[p], sizeof(double) * (size_t)(nu2 * no), NULL) != 0 ||
-            ccx_hip_pack_ax_one(vx, tx, g_te.axr + sl[p] * panel, g_te.axc + sl[p] * panel, (int)no, (int)nu,
-                                (int)nup, (int)kp, NULL) != 0)
+        if (ccx_hip_memcpy_h2d(g_te.in, vvvo_src[p], cube, NULL) != 0 ||
+            ccx_hip_memcpy_h2d(tx, t2x[p], sizeof(double) * (size_t)(nu2 * no), NULL) != 0 ||
+            ccx_hip_pack_ax_one(src_kind, g_te.in, tx, g_te.axr + sl[p] * panel, g_te.axc + sl[p] * panel, (int)no,
+                                (int)nu, (int)nup, (int)kp, NULL) != 0)
             return CCX_ERR_DEVICE;
     }
     /* BX panels and VOE blocks of the ordered position pairs (y,z), y != z, at slot pair (sy,sz) */
@@ -1176,7 +1149,7 @@ static int te_tuple(int64_t no, int64_t nu, const int64_t x[3], int kind, const 
         double out[2];
         double *hv = (double *)malloc(sizeof(double) * (size_t)(TE_SLOTS * nu));
         if (!hv) return CCX_ERR_ALLOC;
-        if (ccx_hip_finalize(g_te.epart, g_te.v1part, g_te.tup, g_te.blocks, g_te.t1, g_te.v1t, g_te.v1, g_te.out,
+        if (ccx_hip_finalize(g_te.epart, g_te.v1part, g_te.tup, g_te.t1, g_te.v1t, g_te.v1, g_te.out,
                              TE_SLOTS, (int)nu, 1, (int)g_te.nblk, NULL) != 0 ||
             ccx_hip_memcpy_d2h(out, g_te.out, sizeof(out), NULL) != 0 ||
             ccx_hip_memcpy_d2h(hv, g_te.v1, sizeof(double) * (size_t)(TE_SLOTS * nu), NULL) != 0) {

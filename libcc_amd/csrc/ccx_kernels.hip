@@ -38,66 +38,134 @@
 // ---------------------------------------------------------------------------------
 // packing kernels (once per problem)
 // ---------------------------------------------------------------------------------
-__device__ __forceinline__ double ax_value(const double *__restrict__ vvvo, const double *__restrict__ t2,
-                                           int no, int nu, int x, int ag, int bg, long long K)
-{
-    if (ag >= nu || bg >= nu) return 0.0;
-    if (K < nu) return vvvo[K + (long long)nu * (bg + (long long)nu * (ag + (long long)nu * x))];
-    if (K < nu + no) return t2[ag + (long long)nu * (bg + (long long)nu * ((K - nu) + (long long)no * x))];
-    return 0.0;
-}
+// Layouts VVVO comes in; (K, b, a, x) is the element VVVO(K,b,a,x), 0-based.
+enum VvvoLayout {
+    V_FULL = 0,     // (nu, nu, nu, no)
+    V_PACKED = 1,   // distributed (nutr, nu no): column a + nu x holds the lower-packed symmetric (K,b)
+                    // block, row p (p+1)/2 + q for q <= p, as DDCC_T_GETVE / CPYTSQ expand it
+                    // (src/triples-ijk/common_functions.f:43-60,106-125)
+    V_VE = 2        // VE_x(K,a,b), the cube the reference's per-tuple routines take
+};
 
-// COLS = 0: row layout [..][alpha][kb][k4][beta]; COLS = 1: column layout [..][beta][kb][k4][alpha].
-// Packs the panels of nx occupied indices x = 0..nx-1 from vvvo + x nu^3 and t2 + x nu^2 no (nx = no
-// for the whole slab; 1 for one index, with the pointers at that index).
-template <int COLS, class T>
-__global__ void pack_ax_kernel(const double *__restrict__ vvvo, const double *__restrict__ t2,
-                               T *__restrict__ ax, int no, int nu, int nb, int kp, int nx)
+template <int LAYOUT>
+__device__ __forceinline__ double vvvo_at(const double *__restrict__ v, int nu, int x, int a, int b, int K)
 {
-    const long long per_panel = 256LL * kp;
-    const long long total = (long long)nx * nb * nb * per_panel;
-    for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
-         idx += (long long)gridDim.x * blockDim.x) {
-        long long r = idx % per_panel;
-        long long pnl = idx / per_panel;
-        // [outer/2][kp/4][64 lanes][2]: the fragments of the two batches (outer indices 2w,
-        // 2w+1) a wave owns interleave per lane, so one 2-wide load fetches both
-        const int bbit = (int)(r & 1);
-        const int lane = (int)((r >> 1) & 63);
-        const long long rr = r >> 7;
-        const long long K = (rr % (kp / 4)) * 4 + (lane >> 4);   // kb*4 + k4
-        const int outer = (int)(rr / (kp / 4)) * 2 + bbit;       // alpha (rows) / beta (columns)
-        const int inner = lane & 15;                              // beta (rows) / alpha (columns)
-        const int q = pnl % nb; pnl /= nb;
-        const int pblk = pnl % nb; pnl /= nb;
-        const int x = (int)pnl;
-        const int al = COLS ? inner : outer, be = COLS ? outer : inner;
-        ax[idx] = (T)ax_value(vvvo, t2, no, nu, x, pblk * TB + al, q * TB + be, K);
+    if constexpr (LAYOUT == V_FULL) {
+        return v[K + (long long)nu * (b + (long long)nu * (a + (long long)nu * x))];
+    } else if constexpr (LAYOUT == V_PACKED) {
+        const int hi = K > b ? K : b, lo = K > b ? b : K;
+        return v[(long long)hi * (hi + 1) / 2 + lo + ((long long)nu * (nu + 1) / 2) * (a + (long long)nu * x)];
+    } else {
+        return v[K + (long long)nu * (a + (long long)nu * (b + (long long)nu * x))];
     }
 }
 
-template <class T>
-__global__ void pack_bx_kernel(const double *__restrict__ t2, const double *__restrict__ vm,
-                               T *__restrict__ bx, int no, int nu, int nb, int kp)
+// Both orientations of the AX slab from VVVO and T2, for nx occupied indices from those the pointers
+// stand at.  Bound by HBM: VVVO and T2 read once, the two slabs written once.  A work group takes
+// PK_K K of one 16 x 16 panel through LDS, because no thread order is good for both ends: VVVO runs
+// along K (packed, above the diagonal: along b), T2 along a, and the slabs' fragments are
+// [outer/2][K/4][lane: K%4, inner][outer%2].  At no=8, nu=120 the two slabs took 144 us as two
+// kernels with an index chain of 64-bit divisions per element and strided reads, and the packed
+// layout first went through an unpacked copy.
+constexpr int PK_K = 16;
+
+template <int LAYOUT>
+__global__ void __launch_bounds__(256) pack_ax_kernel(const double *__restrict__ vvvo, const double *__restrict__ t2,
+                                                      double *__restrict__ axr, double *__restrict__ axc, int no,
+                                                      int nu, int nb, int kp, int nkc)
+{
+    constexpr int STR = 273, STR_A = 17;
+    __shared__ double tile[PK_K * STR];   // [K][a][b], padded for reads along a and writes along K
+    const int tid = threadIdx.x;
+    unsigned int u = blockIdx.x;
+    const int kc = u % nkc; u /= nkc;
+    const int Q = u % nb; u /= nb;
+    const int P = u % nb;
+    const int x = u / nb;
+    const int K0 = kc * PK_K;
+    if (K0 < nu) {
+        const bool along_b = LAYOUT == V_PACKED && K0 + PK_K - 1 > Q * TB;
+        for (int i = tid; i < PK_K * 256; i += 256) {
+            const int k = along_b ? (i >> 4) & 15 : i & 15, row = along_b ? (i >> 8) * 16 + (i & 15) : i >> 4;
+            const int a = P * TB + (row >> 4), b = Q * TB + (row & 15), K = K0 + k;
+            if (K < nu) tile[k * STR + (row >> 4) * STR_A + (row & 15)] = a < nu && b < nu ? vvvo_at<LAYOUT>(vvvo, nu, x, a, b, K) : 0.0;
+        }
+    }
+    if (K0 + PK_K > nu)
+        for (int i = tid; i < PK_K * 256; i += 256) {
+            const int k = i >> 8, row = (i & 15) * 16 + ((i >> 4) & 15);
+            const int a = P * TB + (row >> 4), b = Q * TB + (row & 15), K = K0 + k;
+            if (K >= nu)
+                tile[k * STR + (row >> 4) * STR_A + (row & 15)] = a < nu && b < nu && K < nu + no
+                    ? t2[a + (long long)nu * (b + (long long)nu * ((K - nu) + (long long)no * x))] : 0.0;
+        }
+    __syncthreads();
+    const long long panel = (((long long)x * nb + P) * nb + Q) * (256LL * kp);
+    for (int i = tid; i < PK_K * 128; i += 256) {
+        const int lane = i & 63, kb = (i >> 6) & 3, pr = i >> 8;      // outer pair pr
+        if (K0 / 4 + kb >= kp / 4) continue;
+        const double *r = tile + (kb * 4 + (lane >> 4)) * STR;
+        const int in = lane & 15;
+        const long long o = panel + ((long long)pr * (kp / 4) + K0 / 4 + kb) * 128 + lane * 2;
+        *reinterpret_cast<double2 *>(axr + o) = make_double2(r[2 * pr * STR_A + in], r[(2 * pr + 1) * STR_A + in]);
+        *reinterpret_cast<double2 *>(axc + o) = make_double2(r[in * STR_A + 2 * pr], r[in * STR_A + 2 * pr + 1]);
+    }
+}
+
+// BX[y,z](g,K) = T2(g,K,y,z) for K < nu, -VM(K-nu,g,z,y) after, [y][z][g block][K][16]
+__device__ __forceinline__ void pack_bx(const double *__restrict__ t2, const double *__restrict__ vm,
+                                        double *__restrict__ bx, int no, int nu, int nb, int kp, int wg, int nwg)
 {
     const long long total = (long long)no * no * nb * kp * 16;
-    for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
-         idx += (long long)gridDim.x * blockDim.x) {
-        long long r = idx;
-        const int gl = r & 15; r >>= 4;
-        const int K = r % kp; r /= kp;
-        const int gb = r % nb; r /= nb;
-        const int z = r % no; r /= no;
-        const int y = (int)r;
-        const int g = gb * TB + gl;
+    for (long long idx = wg * 256LL + threadIdx.x; idx < total; idx += nwg * 256LL) {
+        const int gl = (int)(idx & 15);
+        const long long r = idx >> 4, pg = r / kp;
+        const int K = (int)(r - pg * kp), yz = (int)(pg / nb), g = (int)(pg - (long long)yz * nb) * TB + gl;
+        const int y = yz / no, z = yz % no;
         double v = 0.0;
         if (g < nu) {
-            if (K < nu)
-                v = t2[g + (long long)nu * (K + (long long)nu * (y + (long long)no * z))];
-            else if (K < nu + no)
-                v = -vm[(K - nu) + (long long)no * (g + (long long)nu * (z + (long long)no * y))];
+            if (K < nu) v = t2[g + (long long)nu * (K + (long long)nu * (y + (long long)no * z))];
+            else if (K < nu + no) v = -vm[(K - nu) + (long long)no * (g + (long long)nu * (z + (long long)no * y))];
         }
-        bx[idx] = (T)v;
+        bx[idx] = v;
+    }
+}
+
+// out[q][r][x][y] = VOE(x,y,q,r), zero past nu, by 16 x 16 tiles through LDS (VOE runs along x, out along y)
+__device__ __forceinline__ void pack_voe(const double *__restrict__ voe, double *__restrict__ out, int no, int nu,
+                                         int nup, int wg, int nwg)
+{
+    __shared__ double tile[16 * 17];
+    const int nb = nup / TB, i = threadIdx.x & 15, j = threadIdx.x >> 4;
+    const long long ntile = (long long)no * no * nb * nb;
+    for (long long u = wg; u < ntile; u += nwg) {
+        const int Y = (int)(u % nb), X = (int)(u / nb % nb);
+        const long long qr = u / nb / nb;               // q no + r
+        const int q = (int)(qr / no), r = (int)(qr % no);
+        const int x = X * TB + i, y = Y * TB + j;
+        tile[i * 17 + j] = x < nu && y < nu ? voe[x + (long long)nu * (y + (long long)nu * (q + (long long)no * r))] : 0.0;
+        __syncthreads();
+        out[(qr * nup + X * TB + j) * nup + Y * TB + i] = tile[j * 17 + i];
+        __syncthreads();
+    }
+}
+
+// The rest of a problem in one launch: BX, the padded VOE, and the small arrays (eps_virtual padded
+// with finite values, since padded elements carry W = 0; eps_occupied and T1 copied).
+struct RestArgs {
+    const double *t2, *vm, *voe, *eh, *ep, *t1;
+    double *bx, *voep, *ehp, *epp, *t1p;   // the last three may be null
+    int no, nu, nup, kp, gbx, gvoe;
+};
+__global__ void __launch_bounds__(256) pack_rest_kernel(RestArgs a)
+{
+    const int wg = blockIdx.x;
+    if (wg < a.gbx) pack_bx(a.t2, a.vm, a.bx, a.no, a.nu, a.nup / TB, a.kp, wg, a.gbx);
+    else if (wg < a.gbx + a.gvoe) pack_voe(a.voe, a.voep, a.no, a.nu, a.nup, wg - a.gbx, a.gvoe);
+    else {
+        if (a.epp) for (int i = threadIdx.x; i < a.nup; i += 256) a.epp[i] = i < a.nu ? a.ep[i] : 1.0e3;
+        if (a.ehp) for (int i = threadIdx.x; i < a.no; i += 256) a.ehp[i] = a.eh[i];
+        if (a.t1p) for (int i = threadIdx.x; i < a.no * a.nu; i += 256) a.t1p[i] = a.t1[i];
     }
 }
 
@@ -121,50 +189,10 @@ __global__ void pack_bx_pair_kernel(const double *__restrict__ t2yz, const doubl
     }
 }
 
-// VVVO(d,q,p,x) = VE_x(d,p,q): the (2,3) index swap of one occupied index's cube
-__global__ void ve_to_vvvo_kernel(const double *__restrict__ ve, double *__restrict__ vvvo, int nu)
+__global__ void __launch_bounds__(256) pack_voe_kernel(const double *__restrict__ voe, double *__restrict__ out, int no,
+                                                       int nu, int nup)
 {
-    const long long n3 = (long long)nu * nu * nu;
-    for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < n3;
-         idx += (long long)gridDim.x * blockDim.x) {
-        const long long d = idx % nu, q = (idx / nu) % nu, p = idx / ((long long)nu * nu);
-        vvvo[idx] = ve[d + nu * (p + (long long)nu * q)];
-    }
-}
-
-__global__ void pack_voe_kernel(const double *__restrict__ voe, double *__restrict__ out, int no,
-                                int nu, int nup)
-{
-    const long long total = (long long)no * no * nup * nup;
-    for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
-         idx += (long long)gridDim.x * blockDim.x) {
-        long long r = idx;
-        const int y = r % nup; r /= nup;
-        const int x = r % nup; r /= nup;
-        const int rr = r % no; r /= no;
-        const int q = (int)r;
-        double v = 0.0;
-        if (x < nu && y < nu)
-            v = voe[x + (long long)nu * (y + (long long)nu * (q + (long long)no * rr))];
-        out[idx] = v;
-    }
-}
-
-// Distributed (nutr, nu*no) layout -> VVVO(nu,nu,nu,no): column c + nu*x holds the
-// lower-packed symmetric (p,q) pair block, row p*(p+1)/2 + q for q <= p (0-based),
-// as DDCC_T_GETVE / CPYTSQ expand it (src/triples-ijk/common_functions.f:43-60,106-125).
-__global__ void unpack_vvvo_kernel(const double *__restrict__ packed, double *__restrict__ full, int no, int nu)
-{
-    const long long nutr = (long long)nu * (nu + 1) / 2;
-    const long long total = (long long)nu * nu * nu * no;
-    for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
-         idx += (long long)gridDim.x * blockDim.x) {
-        const int p = idx % nu;
-        const int q = (idx / nu) % nu;
-        const long long col = idx / ((long long)nu * nu);   // c + nu*x
-        const int hi = p > q ? p : q, lo = p > q ? q : p;
-        full[idx] = packed[(long long)hi * (hi + 1) / 2 + lo + nutr * col];
-    }
+    pack_voe(voe, out, no, nu, nup, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------------
@@ -519,62 +547,114 @@ __global__ void __launch_bounds__(NTHR, 1) triples_kernel(TriplesArgs g)
 // ---------------------------------------------------------------------------------
 // finalize: deterministic reductions
 // ---------------------------------------------------------------------------------
-// v1t[t][a][p] = sum over the blocks of tuple t whose role-r block contains a
-__global__ void reduce_v1_tuple_kernel(const double *__restrict__ v1_part, const int *__restrict__ blocks,
-                                       double *__restrict__ v1t, int ntup, int nblk, int nu)
+// Index of the block orbit (A <= B <= C) in the table's order (A outermost, then B, then C).
+__device__ __forceinline__ int orbit_index(int A, int B, int C, int nb)
 {
-    const long long total = (long long)ntup * nu * 3;
-    for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
-         idx += (long long)gridDim.x * blockDim.x) {
-        const int p = idx % 3;
-        const int a = (idx / 3) % nu;
-        const long long t = idx / (3LL * nu);
-        const int ab = a / TB, al = a % TB;
+    auto t2 = [](int n) { return n * (n + 1) / 2; };
+    auto t3 = [](int n) { return n * (n + 1) * (n + 2) / 6; };
+    return t3(nb) - t3(nb - A) + t2(nb - A) - t2(nb - B) + (C - B);
+}
+
+constexpr int RV_GRP = 5;             // groups of 48 lanes (virtual index of the block, tuple position)
+constexpr int RE_CHUNKS = 256;        // most work groups of the energy sum
+
+// Work groups 0 .. ntup nb - 1: v1t[t][a][p] for the 16 indices a of block ab, the sum over the orbits
+// holding ab in some role.  Those are the orbits {ab, X, Y} of the pairs X <= Y, so the work group
+// walks the pairs, RV_GRP at a time (with one lane per (t,a,p) walking all orbits, a few thousand
+// lanes took serial chains of nblk loads: 111 us at no=4, nu=167 for 5 MB of partials, now 10).
+// Work groups after them: the compensated sum of one chunk of the energy partials, left in the
+// chunk's first element.  Every order is fixed.
+__global__ void __launch_bounds__(256) reduce_partials_kernel(const double *__restrict__ v1_part, double *e_part,
+                                                              double *__restrict__ v1t, int ntup, int nblk, int nu,
+                                                              int nb, long long nitems, long long chunk)
+{
+    __shared__ double sh[256];
+    const int tid = threadIdx.x;
+    const long long wg = blockIdx.x;
+    if (wg < (long long)ntup * nb) {
+        const long long t = wg / nb;
+        const int ab = (int)(wg % nb), grp = tid / 48, e = tid % 48;
         double s = 0.0;
-        for (int q = 0; q < nblk; ++q) {
-            const int4 bp = reinterpret_cast<const int4 *>(blocks)[q];
-            const double *vp = v1_part + (t * nblk + q) * 144;
-            if (bp.x == ab) s += vp[al * 3 + p];
-            if (bp.y == ab) s += vp[48 + al * 3 + p];
-            if (bp.z == ab) s += vp[96 + al * 3 + p];
+        if (grp < RV_GRP) {
+            const double *vt = v1_part + t * nblk * 144 + e;
+            int X = 0, Y = grp;
+            for (;;) {
+                while (X < nb && Y >= nb) { ++X; Y += X - nb; }   // row X of the pair list holds Y = X .. nb-1
+                if (X >= nb) break;
+                const int lo = ab < X ? ab : X, hi = ab > Y ? ab : Y, mid = ab + X + Y - lo - hi;
+                const double *vp = vt + (long long)orbit_index(lo, mid, hi, nb) * 144;
+                if (lo == ab) s += vp[0];
+                if (mid == ab) s += vp[48];
+                if (hi == ab) s += vp[96];
+                Y += RV_GRP;
+            }
         }
-        v1t[idx] = s;
+        sh[tid] = s;
+        __syncthreads();
+        const int a = ab * TB + e / 3;
+        if (tid < 48 && a < nu) {
+            double r = sh[tid];
+#pragma unroll
+            for (int q = 1; q < RV_GRP; ++q) r += sh[q * 48 + tid];
+            v1t[(t * nu + a) * 3 + e % 3] = r;
+        }
+    } else {
+        const long long beg = (wg - (long long)ntup * nb) * chunk;
+        const long long end = beg + chunk < nitems ? beg + chunk : nitems;
+        double s = 0.0, c = 0.0;
+        for (long long i = beg + tid; i < end; i += 256) {
+            const double y = e_part[i], tt = s + y;
+            c += (fabs(s) >= fabs(y)) ? ((s - tt) + y) : ((y - tt) + s);
+            s = tt;
+        }
+        sh[tid] = s + c;
+        __syncthreads();
+        for (int w = 128; w >= 1; w >>= 1) {
+            if (tid < w) sh[tid] += sh[tid + w];
+            __syncthreads();
+        }
+        if (tid == 0) e_part[beg] = sh[0];
     }
 }
 
-// v1(a,o) (column-major nu x no) = sum over tuples and positions p with tuple[p] == o
-__global__ void reduce_v1_kernel(const double *__restrict__ v1t, const int *__restrict__ tuples,
-                                 double *__restrict__ v1, int ntup, int nu, int no)
+// v1(a,o) (column-major nu x no) = sum over tuples and positions p with tuple[p] == o: work group per
+// o and 64 indices a, four groups of lanes over the tuples, whose table entries pass through LDS.
+__global__ void __launch_bounds__(256) reduce_v1_kernel(const double *__restrict__ v1t, const int *__restrict__ tuples,
+                                                        double *__restrict__ v1, int ntup, int nu, int no)
 {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= nu * no) return;
-    const int a = idx % nu, o = idx / nu;
+    __shared__ int4 tab[256];
+    __shared__ double sh[256];
+    const int tid = threadIdx.x, grp = tid >> 6;
+    const int na = (nu + 63) / 64, o = blockIdx.x / na, a = (blockIdx.x % na) * 64 + (tid & 63);
     double s = 0.0;
-    for (int t = 0; t < ntup; ++t) {
-        const int4 tp = reinterpret_cast<const int4 *>(tuples)[t];
-        const double *r = v1t + ((long long)t * nu + a) * 3;
-        if (tp.x == o) s += r[0];
-        if (tp.y == o) s += r[1];
-        if (tp.z == o) s += r[2];
+    for (int t0 = 0; t0 < ntup; t0 += 256) {
+        const int n = ntup - t0 < 256 ? ntup - t0 : 256;
+        if (tid < n) tab[tid] = reinterpret_cast<const int4 *>(tuples)[t0 + tid];
+        __syncthreads();
+        if (a < nu)
+            for (int t = grp; t < n; t += 4) {
+                const int4 tp = tab[t];
+                const double *r = v1t + ((long long)(t0 + t) * nu + a) * 3;
+                if (tp.x == o) s += r[0];
+                if (tp.y == o) s += r[1];
+                if (tp.z == o) s += r[2];
+            }
+        __syncthreads();
     }
-    v1[idx] = s;
+    sh[tid] = s;
+    __syncthreads();
+    if (grp == 0 && a < nu) v1[a + (long long)nu * o] = (sh[tid] + sh[tid + 64]) + (sh[tid + 128] + sh[tid + 192]);
 }
 
-// out[0] = etd = sum e_part (compensated, fixed order); out[1] = ets = 2 sum T1(o,a) v1(a,o)
-__global__ void __launch_bounds__(1024) finalize_energy_kernel(const double *__restrict__ e_part, long long n,
-                                                               const double *__restrict__ t1,
+// out[0] = etd = sum of the chunk sums e_part[0], e_part[chunk], ...; out[1] = ets = 2 sum T1(o,a) v1(a,o)
+// (both compensated, fixed order)
+__global__ void __launch_bounds__(1024) finalize_energy_kernel(const double *__restrict__ e_part, int nchunk,
+                                                               long long chunk, const double *__restrict__ t1,
                                                                const double *__restrict__ v1, int no, int nu,
                                                                double *__restrict__ out)
 {
     __shared__ double sh[2][1024];
     const int tid = threadIdx.x;
-    double s = 0.0, c = 0.0;
-    for (long long i = tid; i < n; i += 1024) {
-        const double y = e_part[i];
-        const double tt = s + y;
-        c += (fabs(s) >= fabs(y)) ? ((s - tt) + y) : ((y - tt) + s);
-        s = tt;
-    }
     double s2 = 0.0, c2 = 0.0;
     for (int i = tid; i < no * nu; i += 1024) {
         const int a = i % nu, o = i / nu;
@@ -583,7 +663,7 @@ __global__ void __launch_bounds__(1024) finalize_energy_kernel(const double *__r
         c2 += (fabs(s2) >= fabs(y)) ? ((s2 - tt) + y) : ((y - tt) + s2);
         s2 = tt;
     }
-    sh[0][tid] = s + c;
+    sh[0][tid] = tid < nchunk ? e_part[tid * chunk] : 0.0;
     sh[1][tid] = s2 + c2;
     __syncthreads();
     for (int w = 512; w >= 1; w >>= 1) {
@@ -650,12 +730,27 @@ __global__ void __launch_bounds__(256) t1wt3_kernel(const double *__restrict__ w
 
 __global__ void zero_counter_kernel(unsigned int *c) { *c = 0u; }
 
-// flag |= 1 when any of the n doubles is NaN or infinite (one atomic per wave at most)
-__global__ void nonfinite_kernel(const double *__restrict__ p, long long n, unsigned int *__restrict__ flag)
+// flag |= 1 when any of the doubles of the arrays is NaN or infinite (one atomic per wave at most),
+// all arrays in one launch
+struct ScanArgs {
+    const double *p[7];
+    long long n[7];
+    int narr;
+};
+__global__ void __launch_bounds__(256) nonfinite_kernel(ScanArgs a, unsigned int *__restrict__ flag)
 {
     int bad = 0;
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-        bad |= !isfinite(p[i]);
+    const long long step = (long long)gridDim.x * blockDim.x, first = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    for (int q = 0; q < a.narr; ++q) {
+        const double *__restrict__ p = a.p[q];
+        const long long n = a.n[q];
+        long long i = first;
+        for (; i + 3 * step < n; i += 4 * step) {   // four loads in flight
+            const double x0 = p[i], x1 = p[i + step], x2 = p[i + 2 * step], x3 = p[i + 3 * step];
+            bad |= !isfinite(x0) | !isfinite(x1) | !isfinite(x2) | !isfinite(x3);
+        }
+        for (; i < n; i += step) bad |= !isfinite(p[i]);
+    }
     if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(flag, 1u);
 }
 
@@ -761,38 +856,43 @@ int ccx_hip_cu_count(int *n)
 const char *ccx_hip_last_error(void) { return hipGetErrorString(hipGetLastError()); }
 
 
-// form 0: FP64 slabs (double); form 1: FP32 slabs (float).  voep is written only when non-null.
-int ccx_hip_pack(int form, const double *vvvo, const double *t2, const double *vm, const double *voe, void *axr,
-                 void *axc, void *bx, double *voep, int no, int nu, int nup, int kp, void *stream)
+// AX in both orientations from VVVO (layout V_FULL, V_PACKED or V_VE) and T2 of nx occupied indices
+static int launch_pack_ax(int layout, const double *vvvo, const double *t2, double *axr, double *axc, int no, int nu,
+                          int nup, int kp, int nx, hipStream_t s)
 {
-    hipStream_t s = (hipStream_t)stream;
-    const int nb = nup / TB;
-    const long long nax = (long long)no * nb * nb * kp * 256;
-    const int gbx = grid_for((long long)no * no * nb * kp * 16);
-    if (form == 0) {
-        pack_ax_kernel<0, double><<<grid_for(nax), 256, 0, s>>>(vvvo, t2, (double *)axr, no, nu, nb, kp, no);
-        pack_ax_kernel<1, double><<<grid_for(nax), 256, 0, s>>>(vvvo, t2, (double *)axc, no, nu, nb, kp, no);
-        pack_bx_kernel<double><<<gbx, 256, 0, s>>>(t2, vm, (double *)bx, no, nu, nb, kp);
-    } else {
-        pack_ax_kernel<0, float><<<grid_for(nax), 256, 0, s>>>(vvvo, t2, (float *)axr, no, nu, nb, kp, no);
-        pack_ax_kernel<1, float><<<grid_for(nax), 256, 0, s>>>(vvvo, t2, (float *)axc, no, nu, nb, kp, no);
-        pack_bx_kernel<float><<<gbx, 256, 0, s>>>(t2, vm, (float *)bx, no, nu, nb, kp);
-    }
-    if (voep) pack_voe_kernel<<<grid_for((long long)no * no * nup * nup), 256, 0, s>>>(voe, voep, no, nu, nup);
+    const int nb = nup / TB, nkc = (kp + PK_K - 1) / PK_K;
+    const long long grid = (long long)nx * nb * nb * nkc;
+    if (grid > 0x7fffffffLL) return 3;
+    if (layout == V_FULL) pack_ax_kernel<V_FULL><<<(unsigned)grid, 256, 0, s>>>(vvvo, t2, axr, axc, no, nu, nb, kp, nkc);
+    else if (layout == V_PACKED) pack_ax_kernel<V_PACKED><<<(unsigned)grid, 256, 0, s>>>(vvvo, t2, axr, axc, no, nu, nb, kp, nkc);
+    else pack_ax_kernel<V_VE><<<(unsigned)grid, 256, 0, s>>>(vvvo, t2, axr, axc, no, nu, nb, kp, nkc);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-// The FP64 panels of one occupied index (both AX orientations) from vvvo_x = VVVO(:,:,:,x) (nu^3) and
-// t2_x = T2(:,:,:,x) (nu^2 no); axr_x / axc_x point at that index's panels.
-int ccx_hip_pack_ax_one(const double *vvvo_x, const double *t2_x, double *axr_x, double *axc_x, int no, int nu,
-                        int nup, int kp, void *stream)
+// The operand slabs, the padded VOE and (where their destinations are given) the small arrays of a
+// problem, from the reference-layout arrays; vvvo_layout 0 or 1 as in ccx_load_device.
+int ccx_hip_pack(int vvvo_layout, const double *vvvo, const double *t2, const double *vm, const double *voe,
+                 const double *eh, const double *ep, const double *t1, double *axr, double *axc, double *bx,
+                 double *voep, double *ehp, double *epp, double *t1p, int no, int nu, int nup, int kp, void *stream)
 {
     hipStream_t s = (hipStream_t)stream;
     const int nb = nup / TB;
-    const long long n = (long long)nb * nb * kp * 256;
-    pack_ax_kernel<0, double><<<grid_for(n), 256, 0, s>>>(vvvo_x, t2_x, axr_x, no, nu, nb, kp, 1);
-    pack_ax_kernel<1, double><<<grid_for(n), 256, 0, s>>>(vvvo_x, t2_x, axc_x, no, nu, nb, kp, 1);
+    const int rc = launch_pack_ax(vvvo_layout, vvvo, t2, axr, axc, no, nu, nup, kp, no, s);
+    if (rc != 0) return rc;
+    const long long ntile = (long long)no * no * nb * nb;
+    RestArgs a = {t2, vm, voe, eh, ep, t1, bx, voep, ehp, epp, t1p, no, nu, nup, kp,
+                  grid_for((long long)no * no * nb * kp * 16), (int)(ntile < 65536 ? ntile : 65536)};
+    pack_rest_kernel<<<a.gbx + a.gvoe + 1, 256, 0, s>>>(a);
     return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+// The FP64 panels of one occupied index (both AX orientations) from its cube (layout 0: VE_x(d,p,q) =
+// VVVO(d,q,p,x); 1: the packed columns of x) and t2_x = T2(:,:,:,x) (nu^2 no); axr_x / axc_x point at
+// that index's panels.
+int ccx_hip_pack_ax_one(int layout, const double *cube, const double *t2_x, double *axr_x, double *axc_x, int no,
+                        int nu, int nup, int kp, void *stream)
+{
+    return launch_pack_ax(layout == 1 ? V_PACKED : V_VE, cube, t2_x, axr_x, axc_x, no, nu, nup, kp, 1, (hipStream_t)stream);
 }
 
 // The FP64 BX panels of one ordered pair (y,z) and, when voe_yz is non-null, its padded VOE block:
@@ -803,18 +903,10 @@ int ccx_hip_pack_pair(const double *t2_yz, const double *vm_zy, const double *vo
     hipStream_t s = (hipStream_t)stream;
     const int nb = nup / TB;
     pack_bx_pair_kernel<<<grid_for((long long)nb * kp * 16), 256, 0, s>>>(t2_yz, vm_zy, bx_yz, no, nu, nb, kp);
-    if (voe_yz) pack_voe_kernel<<<grid_for((long long)nup * nup), 256, 0, s>>>(voe_yz, voep_yz, 1, nu, nup);
+    if (voe_yz) pack_voe_kernel<<<nb * nb < 65536 ? nb * nb : 65536, 256, 0, s>>>(voe_yz, voep_yz, 1, nu, nup);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-int ccx_hip_ve_to_vvvo(const double *ve, double *vvvo_x, int nu, void *stream)
-{
-    ve_to_vvvo_kernel<<<grid_for((long long)nu * nu * nu), 256, 0, (hipStream_t)stream>>>(ve, vvvo_x, nu);
-    return hipGetLastError() == hipSuccess ? 0 : 1;
-}
-
-// form 0: FP64 slabs; 1: FP32 slabs in the FP32 sweep's order (K padded to kps, a multiple of
-// 48); 2: split BF16 (split[] = axr_s, axc_s, bx_s, K padded to kps, W scaled by wscale)
 // K padding of a form's slabs: FP32 48; split forms two K blocks of their MFMA (64 for bf16,
 // 256 for fp8 e4m3); FP64 4
 int ccx_hip_form_kpad(int form) { return form == 1 ? 48 : form == 3 ? 256 : form >= 2 ? 64 : 4; }
@@ -912,19 +1004,24 @@ int ccx_hip_pack_split(int form, const double *axr, const double *axc, const dou
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-int ccx_hip_finalize(const double *e_part, const double *v1_part, const int *tuples, const int *blocks,
-                     const double *t1, double *v1t, double *v1, double *out, int no, int nu, int ntup, int nblk,
-                     void *stream)
+// Sums the work items' partials (the energy partials are overwritten): out = {etd, ets}, v1(nu,no).
+int ccx_hip_finalize(double *e_part, const double *v1_part, const int *tuples, const double *t1, double *v1t,
+                     double *v1, double *out, int no, int nu, int ntup, int nblk, void *stream)
 {
     hipStream_t s = (hipStream_t)stream;
+    const int nb = (nu + TB - 1) / TB;
+    const long long nitems = (long long)ntup * nblk;
+    long long chunk = (nitems + RE_CHUNKS - 1) / RE_CHUNKS;
+    if (chunk < 1024) chunk = 1024;
+    const int nchunk = (int)((nitems + chunk - 1) / chunk);
     if (ntup > 0) {
-        reduce_v1_tuple_kernel<<<grid_for((long long)ntup * nu * 3), 256, 0, s>>>(v1_part, blocks, v1t, ntup,
-                                                                                  nblk, nu);
-        reduce_v1_kernel<<<(nu * no + 255) / 256, 256, 0, s>>>(v1t, tuples, v1, ntup, nu, no);
+        reduce_partials_kernel<<<(unsigned)((long long)ntup * nb + nchunk), 256, 0, s>>>(v1_part, e_part, v1t, ntup, nblk,
+                                                                                         nu, nb, nitems, chunk);
+        reduce_v1_kernel<<<no * ((nu + 63) / 64), 256, 0, s>>>(v1t, tuples, v1, ntup, nu, no);
     } else {
         if (hipMemsetAsync(v1, 0, sizeof(double) * nu * no, s) != hipSuccess) return 1;
     }
-    finalize_energy_kernel<<<1, 1024, 0, s>>>(e_part, (long long)ntup * nblk, t1, v1, no, nu, out);
+    finalize_energy_kernel<<<1, 1024, 0, s>>>(e_part, nchunk, chunk, t1, v1, no, nu, out);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
@@ -950,27 +1047,35 @@ int ccx_hip_pack_f32v(const double *axr, const double *axc, const double *bx, fl
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-// *nonfinite = 1 when any element of the arrays p[0..narr) (n[q] doubles each) is NaN or infinite
+int ccx_hip_zero_flag(unsigned int *d_flag, void *stream)
+{
+    zero_counter_kernel<<<1, 1, 0, (hipStream_t)stream>>>(d_flag);
+    return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+// *nonfinite = 1 when any element of the arrays p[0..narr) (n[q] doubles each, at most 7 arrays) is NaN
+// or infinite.  *d_flag is zero before the call; it is left non-zero when *nonfinite is.
 int ccx_hip_nonfinite(const double *const *p, const size_t *n, int narr, unsigned int *d_flag, int *nonfinite,
                       void *stream)
 {
     hipStream_t s = (hipStream_t)stream;
-    zero_counter_kernel<<<1, 1, 0, s>>>(d_flag);
-    for (int q = 0; q < narr; ++q)
-        if (n[q] > 0) nonfinite_kernel<<<grid_for((long long)n[q]), 256, 0, s>>>(p[q], (long long)n[q], d_flag);
+    if (narr > 7) return 3;
+    ScanArgs a;
+    long long most = 1;
+    a.narr = narr;
+    for (int q = 0; q < narr; ++q) {
+        a.p[q] = p[q];
+        a.n[q] = (long long)n[q];
+        if (a.n[q] > most) most = a.n[q];
+    }
+    const int grid = grid_for((most + 3) / 4);
+    nonfinite_kernel<<<grid < 4096 ? grid : 4096, 256, 0, s>>>(a, d_flag);
     unsigned int h = 0;
     if (hipGetLastError() != hipSuccess || hipMemcpyAsync(&h, d_flag, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         return 1;
     *nonfinite = h != 0;
     return 0;
-}
-
-int ccx_hip_unpack_vvvo(const double *packed, double *full, int no, int nu, void *stream)
-{
-    unpack_vvvo_kernel<<<grid_for((long long)nu * nu * nu * no), 256, 0, (hipStream_t)stream>>>(packed, full, no,
-                                                                                                 nu);
-    return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
 int ccx_hip_event_create(void **ev)

@@ -71,13 +71,6 @@ __global__ void static_tables_kernel(int no, int nb, int *__restrict__ tuples, i
             }
 }
 
-// eps_virtual padded to nup with finite values (padded virtual indices carry W = 0)
-__global__ void static_pad_ep_kernel(const double *__restrict__ ep, double *__restrict__ epp, int nu, int nup)
-{
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a < nup) epp[a] = a < nu ? ep[a] : 1.0e3;
-}
-
 __global__ void static_fill_zero_kernel(double *__restrict__ p, long long n)
 {
     for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < n; q += (long long)gridDim.x * blockDim.x)
@@ -151,6 +144,7 @@ extern "C" int ccx_energy_static(int64_t no, int64_t nu, const double *eh, const
     const size_t n[7] = {(size_t)no, (size_t)nu, (size_t)(no * nu), (size_t)(nu * nu * no * no),
                          (size_t)(no * nu * no * no), (size_t)(nu * nu * no * no), (size_t)(nu * nu * nu * no)};
     int bad = 0;
+    if (ccx_hip_zero_flag(p.flag, stream) != 0) return CCX_ERR_DEVICE;
     if (ccx_hip_nonfinite(arr, n, 7, p.flag, &bad, stream) != 0) return CCX_ERR_DEVICE;
     if (bad) return CCX_ERR_INPUT;
 
@@ -160,10 +154,9 @@ extern "C" int ccx_energy_static(int64_t no, int64_t nu, const double *eh, const
         return hipGetLastError() == hipSuccess ? CCX_OK : CCX_ERR_DEVICE;
     }
     static_tables_kernel<<<1, 1, 0, s>>>((int)no, (int)nb, p.tuples, p.blocks);
-    static_pad_ep_kernel<<<(int)((nup + 255) / 256), 256, 0, s>>>(ep, p.epp, (int)nu, (int)nup);
     if (hipGetLastError() != hipSuccess) return CCX_ERR_DEVICE;
-    if (ccx_hip_pack(0, vvvo, t2, vm, voe, p.axr, p.axc, p.bx, p.voep, (int)no, (int)nu, (int)nup, (int)kp,
-                     stream) != 0)
+    if (ccx_hip_pack(0, vvvo, t2, vm, voe, eh, ep, t1, p.axr, p.axc, p.bx, p.voep, nullptr, p.epp, nullptr, (int)no,
+                     (int)nu, (int)nup, (int)kp, stream) != 0)
         return CCX_ERR_DEVICE;
     int cus = 256;
     if (ccx_hip_cu_count(&cus) != 0 || cus < 1) cus = 256;
@@ -173,7 +166,7 @@ extern "C" int ccx_energy_static(int64_t no, int64_t nu, const double *eh, const
                         p.counter, (int)no, (int)nu, (int)nup, (int)kp, (int)ntup, (int)nblk, grid, nullptr, 0, 1.0,
                         stream) != 0)
         return CCX_ERR_DEVICE;
-    if (ccx_hip_finalize(p.epart, p.v1part, p.tuples, p.blocks, t1, p.v1t, v1, e, (int)no, (int)nu, (int)ntup,
+    if (ccx_hip_finalize(p.epart, p.v1part, p.tuples, t1, p.v1t, v1, e, (int)no, (int)nu, (int)ntup,
                          (int)nblk, stream) != 0)
         return CCX_ERR_DEVICE;
     return CCX_OK;
