@@ -9,7 +9,7 @@
 //   W_ijk(a,b,c) = sum over the 6 simultaneous permutations s of the pairs (i,a),(j,b),(k,c)
 //                  of sum_K AX[i'](a',b',K) BX[j',k'](c',K).
 // This path is a cross-check and a surface for virtual-triple callers, not the hot path.  One
-// triple alone: a work group, one lane per (i,j,k), FP64 FMA on cached slab reads (w_abc_kernel).
+// triple alone: one wave per (i,j,k), FP64 FMA on cached slab reads (w_abc_kernel).
 // The sum over all triples: each term s is the GEMM
 //   G_s[x][(y,z)] = sum_K AX[x](v_s0, v_s1, K) BX[y,z](v_s2, K),   no x no^2 x (nu+no),
 // on the FP64 matrix cores, from copies of the slabs with x and (y,z) innermost (w_abc_mfma_kernel).
@@ -20,41 +20,47 @@ namespace {
 
 constexpr int ABC_TB = 16;        // virtual block edge of the slab layouts
 constexpr int ABC_THR = 256;
+constexpr int ABC_P[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
 __constant__ int ABC_PERM[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
 
 // V3 of triple t = (abc[4t], abc[4t+1], abc[4t+2]) into w[t * no^3 ...], column-major
 // (i fastest).  V3(i,i,i) is set to 0, as zerot3 does at the end of abc_tuple_formv3
 // (src/triples-abc/abc_tuple.f90:77); E[T] does not depend on those elements.
+// One wave per element, its lanes along K: a single triple has only no^3 elements, and with one lane
+// each its time was the 6 (nu + no) dependent slab reads of a lane (142 us at no=6, nu=64).
 __global__ void __launch_bounds__(ABC_THR) w_abc_kernel(const double *__restrict__ axr, const double *__restrict__ bx,
                                                         const int *__restrict__ trip, int ntrip, int no, int nu,
                                                         int nb, int kp, double *__restrict__ w)
 {
-    const int t = blockIdx.x;
-    if (t >= ntrip) return;
-    const int v[3] = {trip[4 * t], trip[4 * t + 1], trip[4 * t + 2]};
+    const int lane = threadIdx.x & 63;
     const int no3 = no * no * no;
+    const long long total = (long long)ntrip * no3, nwave = (long long)gridDim.x * (ABC_THR / 64);
     const int kn = nu + no;
-    for (int e = threadIdx.x; e < no3; e += ABC_THR) {
+    for (long long id = blockIdx.x * (long long)(ABC_THR / 64) + (threadIdx.x >> 6); id < total; id += nwave) {
+        const int t = (int)(id / no3), e = (int)(id % no3);
+        const int v[3] = {trip[4 * t], trip[4 * t + 1], trip[4 * t + 2]};
         const int o[3] = {e % no, (e / no) % no, e / (no * no)};
         double acc = 0.0;
         if (!(o[0] == o[1] && o[1] == o[2])) {
+#pragma unroll
             for (int s = 0; s < 6; ++s) {
-                const int p0 = ABC_PERM[s][0], p1 = ABC_PERM[s][1], p2 = ABC_PERM[s][2];
+                const int p0 = ABC_P[s][0], p1 = ABC_P[s][1], p2 = ABC_P[s][2];
                 const int x = o[p0], y = o[p1], z = o[p2];
                 const int av = v[p0], bv = v[p1], cv = v[p2];
-                // row layout of AX (pack_ax_kernel<0>): panel (x, a-block, b-block), then
+                // row layout of AX (axr): panel (x, a-block, b-block), then
                 // [alpha/2][K/4][lane = (K%4)*16 + beta][alpha%2]
                 const int al = av % ABC_TB, be = bv % ABC_TB;
                 const double *ap = axr + (((long long)x * nb + av / ABC_TB) * nb + bv / ABC_TB) * (256LL * kp)
                                    + (long long)(al >> 1) * (kp / 4) * 128 + be * 2 + (al & 1);
-                // BX (pack_bx_kernel): [y][z][c-block][K][gamma]
+                // BX: [y][z][c-block][K][gamma]
                 const double *bp = bx + (((long long)y * no + z) * nb + cv / ABC_TB) * ((long long)kp * 16) + cv % ABC_TB;
                 double sum = 0.0;
-                for (int K = 0; K < kn; ++K) sum = fma(ap[(K >> 2) * 128 + (K & 3) * 32], bp[(long long)K * 16], sum);
+                for (int K = lane; K < kn; K += 64) sum = fma(ap[(K >> 2) * 128 + (K & 3) * 32], bp[(long long)K * 16], sum);
                 acc += sum;
             }
+            for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
         }
-        w[(long long)t * no3 + e] = acc;
+        if (lane == 0) w[id] = acc;
     }
 }
 
@@ -136,8 +142,23 @@ __global__ void __launch_bounds__(ABC_THR) w_abc_mfma_kernel(const double *__res
                 d4 acc[NC];
 #pragma unroll
                 for (int c = 0; c < NC; ++c) acc[c] = d4{0, 0, 0, 0};
-#pragma unroll 4
-                for (int k = 0; k < nk; ++k) {
+                // four K steps per round: their loads are issued together (the compiler does not
+                // unroll a loop with MFMAs of itself)
+                int k = 0;
+                for (; k + 4 <= nk; k += 4) {
+                    double a[4], b[4][NC];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        a[j] = pa[(k + j) * 64];
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) b[j][c] = pb[c][(k + j) * 64];
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j], b[j][c], acc[c], 0, 0, 0);
+                }
+                for (; k < nk; ++k) {
                     const double a = pa[k * 64];
 #pragma unroll
                     for (int c = 0; c < NC; ++c) acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, pb[c][k * 64], acc[c], 0, 0, 0);
@@ -222,8 +243,9 @@ int ccx_hip_w_abc(const void *axr, const void *bx, const int *trip, int ntrip, i
 {
     if (ntrip <= 0) return 0;
     if (kp % 4 != 0 || kp < nu + no) return 3;
-    w_abc_kernel<<<ntrip, ABC_THR, 0, (hipStream_t)stream>>>((const double *)axr, (const double *)bx, trip, ntrip,
-                                                             no, nu, nb, kp, w);
+    const long long groups = ((long long)ntrip * no * no * no + ABC_THR / 64 - 1) / (ABC_THR / 64);
+    w_abc_kernel<<<(int)(groups < 65536 ? groups : 65536), ABC_THR, 0, (hipStream_t)stream>>>(
+        (const double *)axr, (const double *)bx, trip, ntrip, no, nu, nb, kp, w);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
