@@ -12,6 +12,10 @@ int ccx_hip_free(void *p);
 int ccx_hip_memcpy_h2d(void *dst, const void *src, size_t bytes, void *stream);
 int ccx_hip_memcpy_d2h(void *dst, const void *src, size_t bytes, void *stream);
 int ccx_hip_memcpy_d2d(void *dst, const void *src, size_t bytes, void *stream);
+int ccx_hip_host_malloc(void **p, size_t bytes);   /* pinned */
+int ccx_hip_host_free(void *p);
+/* from pinned memory, not waited for */
+int ccx_hip_memcpy_h2d_queue(void *dst, const void *src, size_t bytes, void *stream);
 int ccx_hip_sync(void *stream);
 int ccx_hip_cu_count(int *n);
 const char *ccx_hip_last_error(void);
@@ -25,8 +29,9 @@ int ccx_hip_pack(int vvvo_layout, const double *vvvo, const double *t2, const do
                  double *voep, double *ehp, double *epp, double *t1p, int no, int nu, int nup, int kp, void *stream);
 int ccx_hip_pack_ax_one(int layout, const double *cube, const double *t2_x, double *axr_x, double *axc_x, int no,
                         int nu, int nup, int kp, void *stream);
-int ccx_hip_pack_pair(const double *t2_yz, const double *vm_zy, const double *voe_yz, double *bx_yz,
-                      double *voep_yz, int no, int nu, int nup, int kp, void *stream);
+/* one ordered pair of the per-tuple workspace: source blocks (voe may be null) and destinations */
+struct ccx_pair_pack { const double *t2, *vm, *voe; double *bx, *voep; };
+int ccx_hip_pack_pairs(const struct ccx_pair_pack *p, int n, int no, int nu, int nup, int kp, void *stream);
 int ccx_hip_triples(int form, const void *axr, const void *axc, const void *bx, const double *voep,
                     const double *eh, const double *ep, const int *tuples, const int *blocks, double *e_part,
                     double *v1_part, double *wout, unsigned int *counter, int no, int nu, int nup, int kp,

@@ -13,6 +13,8 @@
 #include "ccx_dev.h"
 
 #define TB 16
+/* largest upload buffer a context keeps between ccx_load_host calls (larger ones are freed again) */
+#define KEEP_UPLOAD ((size_t)256 << 20)
 
 struct ccx_ctx {
     int64_t no, nu, nup, nb, kp;
@@ -35,6 +37,10 @@ struct ccx_ctx {
     unsigned int *d_flag;               /* NaN/Inf flag of ccx_load_device */
     double *d_epart, *d_v1part, *d_v1t, *d_v1, *d_out;
     int *h_tuples, *h_blocks;
+    double *h_res;                      /* pinned: v1 (no nu), etd, ets of a solve, as d_v1 holds them */
+    double *d_arena;                    /* the small device arrays, one allocation */
+    double *d_up;                       /* ccx_load_host's upload buffer, kept up to KEEP_UPLOAD bytes */
+    size_t up_bytes;
     double kernel_ms, total_ms;
     void *ev[4];
 };
@@ -103,15 +109,12 @@ static int64_t build_blocks(int64_t nb, int *out)
 
 static void free_dev(ccx_ctx *c)
 {
-    double **d[] = {&c->d_axr, &c->d_axc, &c->d_bx, &c->d_voep, &c->d_eh, &c->d_ep, &c->d_t1,
-                    &c->d_epart, &c->d_v1part, &c->d_v1t, &c->d_v1, &c->d_out};
+    double **d[] = {&c->d_axr, &c->d_axc, &c->d_bx, &c->d_voep, &c->d_epart, &c->d_v1part, &c->d_v1t, &c->d_arena};
     for (size_t q = 0; q < sizeof(d) / sizeof(d[0]); ++q) {
         ccx_hip_free(*d[q]);
         *d[q] = NULL;
     }
-    ccx_hip_free(c->d_tuples);
-    ccx_hip_free(c->d_blocks);
-    ccx_hip_free(c->d_counter);
+    c->d_eh = c->d_ep = c->d_t1 = c->d_v1 = c->d_out = NULL;   /* in the arena */
     ccx_hip_free(c->d_axr32);
     ccx_hip_free(c->d_axc32);
     ccx_hip_free(c->d_bx32);
@@ -124,7 +127,7 @@ static void free_dev(ccx_ctx *c)
     ccx_hip_free(c->d_bx_e);
     c->d_axr_e = c->d_axc_e = c->d_bx_e = NULL;
     c->split_ax_bytes = c->split_bx_bytes = 0;
-    c->d_tuples = c->d_blocks = NULL;
+    c->d_tuples = c->d_blocks = NULL;   /* in the arena */
     c->d_counter = NULL;
     c->d_axr32 = c->d_axc32 = c->d_bx32 = NULL;
     c->d_axr_s = c->d_axc_s = c->d_bx_s = NULL;
@@ -167,6 +170,8 @@ int ccx_destroy(ccx_ctx *c)
     if (!c) return CCX_ERR_ARG;
     free_dev(c);
     ccx_hip_free(c->d_flag);
+    ccx_hip_free(c->d_up);
+    ccx_hip_host_free(c->h_res);
     for (int q = 0; q < 4; ++q) ccx_hip_event_destroy(c->ev[q]);
     free(c->h_tuples);
     free(c->h_blocks);
@@ -179,13 +184,6 @@ int ccx_set_stream(ccx_ctx *c, void *stream)
     if (!c) return CCX_ERR_ARG;
     c->stream = stream;
     return CCX_OK;
-}
-
-static int finite_all(const double *p, size_t n)
-{
-    for (size_t q = 0; q < n; ++q)
-        if (!isfinite(p[q])) return 0;
-    return 1;
 }
 
 #define DALLOC(ptr, count)                                                             \
@@ -207,27 +205,46 @@ static int build_from_device(ccx_ctx *c, const double *d_eh, const double *d_ep_
     if (c->d_axr) goto allocated; /* buffers depend only on the dimensions: reuse */
     DALLOC(c->d_axr, no * nb * nb * kp * 256);
     DALLOC(c->d_axc, no * nb * nb * kp * 256);
-    DALLOC(c->d_counter, 8);
     DALLOC(c->d_bx, no * no * kp * nup);
     DALLOC(c->d_voep, no * no * nup * nup);
-    DALLOC(c->d_eh, no);
-    DALLOC(c->d_ep, nup);
-    DALLOC(c->d_t1, no * nu);
-    DALLOC(c->d_tuples, 4 * (c->ntup > 0 ? c->ntup : 1));
-    DALLOC(c->d_blocks, 4 * c->nblk);
     DALLOC(c->d_epart, nitems > 0 ? nitems : 1);
     DALLOC(c->d_v1part, (nitems > 0 ? nitems : 1) * 144);
     DALLOC(c->d_v1t, (c->ntup > 0 ? c->ntup : 1) * nu * 3);
-    DALLOC(c->d_v1, no * nu);
-    DALLOC(c->d_out, 4);
+    {
+        /* doubles: counter, tuple table (16 B an entry), block table, eps_occupied, eps_virtual, T1, v1 with
+         * the energies behind it (so one copy brings both) */
+        const int64_t n[7] = {4, 2 * c->ntup, 2 * c->nblk, no, nup, no * nu, no * nu + 2};
+        int64_t off[7], total = 0;
+        for (int q = 0; q < 7; ++q) {
+            off[q] = total;
+            total += (n[q] + 31) / 32 * 32;
+        }
+        DALLOC(c->d_arena, total);
+        c->d_counter = (unsigned int *)(c->d_arena + off[0]);
+        c->d_tuples = (int *)(c->d_arena + off[1]);
+        c->d_blocks = (int *)(c->d_arena + off[2]);
+        c->d_eh = c->d_arena + off[3];
+        c->d_ep = c->d_arena + off[4];
+        c->d_t1 = c->d_arena + off[5];
+        c->d_v1 = c->d_arena + off[6];
+        c->d_out = c->d_v1 + no * nu;
+    }
+    if (!c->h_res && ccx_hip_host_malloc((void **)&c->h_res, sizeof(double) * (size_t)(no * nu + 2)) != 0) {
+        rc = CCX_ERR_ALLOC;
+        goto fail;
+    }
+    /* the schedule tables depend only on the dimensions */
+    if (ccx_hip_memcpy_h2d(c->d_tuples, c->h_tuples, sizeof(int) * 4 * (size_t)c->ntup, c->stream) != 0 ||
+        ccx_hip_memcpy_h2d(c->d_blocks, c->h_blocks, sizeof(int) * 4 * (size_t)c->nblk, c->stream) != 0) {
+        rc = CCX_ERR_DEVICE;
+        goto fail;
+    }
 allocated:
     c->loaded = 0;
     c->f32_ready = 0;
     c->split_ready = 0;
     if (ccx_hip_pack(vvvo_layout, d_vvvo, d_t2, d_vm, d_voe, d_eh, d_ep_raw, d_t1, c->d_axr, c->d_axc, c->d_bx,
                      c->d_voep, c->d_eh, c->d_ep, c->d_t1, (int)no, (int)nu, (int)nup, (int)kp, c->stream) != 0 ||
-        ccx_hip_memcpy_h2d(c->d_tuples, c->h_tuples, sizeof(int) * 4 * (size_t)c->ntup, c->stream) != 0 ||
-        ccx_hip_memcpy_h2d(c->d_blocks, c->h_blocks, sizeof(int) * 4 * (size_t)c->nblk, c->stream) != 0 ||
         ccx_hip_sync(c->stream) != 0) { rc = CCX_ERR_DEVICE; goto fail; }
     c->loaded = 1;
     return CCX_OK;
@@ -248,10 +265,13 @@ int ccx_load_device(ccx_ctx *c, const double *eh, const double *ep, const double
                              (size_t)(no * nu * no * no), (size_t)(nu * nu * no * no),
                              vvvo_layout == 0 ? (size_t)(nu * nu * nu * no) : (size_t)(nu * (nu + 1) / 2 * nu * no)};
         int bad = 0;
-        if (!c->d_flag && ccx_hip_malloc((void **)&c->d_flag, sizeof(unsigned int)) != 0) return CCX_ERR_ALLOC;
-        if (ccx_hip_zero_flag(c->d_flag, c->stream) != 0) return CCX_ERR_DEVICE;
+        /* the flag is zero between calls: cleared when allocated and after a bad input */
+        if (!c->d_flag) {
+            if (ccx_hip_malloc((void **)&c->d_flag, sizeof(unsigned int)) != 0) return CCX_ERR_ALLOC;
+            if (ccx_hip_zero_flag(c->d_flag, c->stream) != 0) return CCX_ERR_DEVICE;
+        }
         if (ccx_hip_nonfinite(arr, n, 7, c->d_flag, &bad, c->stream) != 0) return CCX_ERR_DEVICE;
-        if (bad) return CCX_ERR_INPUT;
+        if (bad) return ccx_hip_zero_flag(c->d_flag, c->stream) != 0 ? CCX_ERR_DEVICE : CCX_ERR_INPUT;
     }
     return build_from_device(c, eh, ep, t1, t2, vm, voe, vvvo, vvvo_layout);
 }
@@ -264,33 +284,34 @@ int ccx_load_host(ccx_ctx *c, const double *eh, const double *ep, const double *
     const int64_t no = c->no, nu = c->nu;
     const size_t n_t2 = (size_t)(nu * nu * no * no), n_vm = (size_t)(no * nu * no * no);
     const size_t n_vvvo = vvvo_layout == 0 ? (size_t)(nu * nu * nu * no) : (size_t)(nu * (nu + 1) / 2 * nu * no);
-    if (!finite_all(eh, (size_t)no) || !finite_all(ep, (size_t)nu) || !finite_all(t1, (size_t)(no * nu)) ||
-        !finite_all(t2, n_t2) || !finite_all(vm, n_vm) || !finite_all(voe, n_t2) || !finite_all(vvvo, n_vvvo))
-        return CCX_ERR_INPUT;
-    int rc = CCX_OK;
-    double *d_eh = NULL, *d_ep = NULL, *d_t1 = NULL, *d_t2 = NULL, *d_vm = NULL, *d_voe = NULL, *d_vvvo = NULL;
-    DALLOC(d_eh, no);
-    DALLOC(d_ep, nu);
-    DALLOC(d_t1, no * nu);
-    DALLOC(d_t2, n_t2);
-    DALLOC(d_vm, n_vm);
-    DALLOC(d_voe, n_t2);
-    DALLOC(d_vvvo, n_vvvo);
-    if (ccx_hip_memcpy_h2d(d_eh, eh, sizeof(double) * (size_t)no, c->stream) != 0 ||
-        ccx_hip_memcpy_h2d(d_ep, ep, sizeof(double) * (size_t)nu, c->stream) != 0 ||
-        ccx_hip_memcpy_h2d(d_t1, t1, sizeof(double) * (size_t)(no * nu), c->stream) != 0 ||
-        ccx_hip_memcpy_h2d(d_t2, t2, sizeof(double) * n_t2, c->stream) != 0 ||
-        ccx_hip_memcpy_h2d(d_vm, vm, sizeof(double) * n_vm, c->stream) != 0 ||
-        ccx_hip_memcpy_h2d(d_voe, voe, sizeof(double) * n_t2, c->stream) != 0 ||
-        ccx_hip_memcpy_h2d(d_vvvo, vvvo, sizeof(double) * n_vvvo, c->stream) != 0) {
-        rc = CCX_ERR_DEVICE;
-        goto fail;
+    /* NaN/Inf are looked for on the device (ccx_load_device), where the scan is a small part of the
+     * upload's time and not longer than it */
+    const double *src[7] = {eh, ep, t1, t2, vm, voe, vvvo};
+    const size_t n[7] = {(size_t)no, (size_t)nu, (size_t)(no * nu), n_t2, n_vm, n_t2, n_vvvo};
+    size_t off[7], total = 0;
+    for (int q = 0; q < 7; ++q) {   /* one buffer, the arrays at multiples of 32 doubles */
+        off[q] = total;
+        total += (n[q] + 31) / 32 * 32;
     }
-    rc = ccx_load_device(c, d_eh, d_ep, d_t1, d_t2, d_vm, d_voe, d_vvvo, vvvo_layout);
-    ccx_hip_sync(c->stream);
-fail:
-    ccx_hip_free(d_eh); ccx_hip_free(d_ep); ccx_hip_free(d_t1); ccx_hip_free(d_t2);
-    ccx_hip_free(d_vm); ccx_hip_free(d_voe); ccx_hip_free(d_vvvo);
+    total *= sizeof(double);
+    if (total > c->up_bytes) {
+        ccx_hip_free(c->d_up);
+        c->up_bytes = 0;
+        if (ccx_hip_malloc((void **)&c->d_up, total) != 0) return CCX_ERR_ALLOC;
+        c->up_bytes = total;
+    }
+    int rc = CCX_OK;
+    for (int q = 0; q < 7 && rc == CCX_OK; ++q)
+        if (ccx_hip_memcpy_h2d(c->d_up + off[q], src[q], sizeof(double) * n[q], c->stream) != 0) rc = CCX_ERR_DEVICE;
+    if (rc == CCX_OK)
+        rc = ccx_load_device(c, c->d_up + off[0], c->d_up + off[1], c->d_up + off[2], c->d_up + off[3], c->d_up + off[4],
+                             c->d_up + off[5], c->d_up + off[6], vvvo_layout);
+    if (c->up_bytes > KEEP_UPLOAD) {
+        ccx_hip_sync(c->stream);
+        ccx_hip_free(c->d_up);
+        c->d_up = NULL;
+        c->up_bytes = 0;
+    }
     return rc;
 }
 
@@ -380,7 +401,6 @@ static int energy_run(ccx_ctx *c, int form, const int *d_tup, int64_t ntup, doub
                       int v1_on_device)
 {
     const int64_t nitems = ntup * c->nblk;
-    double host_out[2] = {0.0, 0.0};
     if (form == CCX_FORM_FP32) {
         int rc = ensure_f32(c);
         if (rc != CCX_OK) return rc;
@@ -393,7 +413,6 @@ static int energy_run(ccx_ctx *c, int form, const int *d_tup, int64_t ntup, doub
     const void *axr = form == CCX_FORM_FP32 ? (const void *)c->d_axr32 : (const void *)c->d_axr;
     const void *axc = form == CCX_FORM_FP32 ? (const void *)c->d_axc32 : (const void *)c->d_axc;
     const void *bx = form == CCX_FORM_FP32 ? (const void *)c->d_bx32 : (const void *)c->d_bx;
-    if (ccx_hip_event_record(c->ev[0], c->stream) != 0) return CCX_ERR_DEVICE;
     if (ccx_hip_event_record(c->ev[1], c->stream) != 0) return CCX_ERR_DEVICE;
     if (nitems > 0 &&
         ccx_hip_triples(form, axr, axc, bx, c->d_voep, c->d_eh, c->d_ep, d_tup, c->d_blocks, c->d_epart,
@@ -406,20 +425,18 @@ static int energy_run(ccx_ctx *c, int form, const int *d_tup, int64_t ntup, doub
                          (int)c->no, (int)c->nu, (int)ntup, (int)c->nblk, c->stream) != 0)
         return CCX_ERR_DEVICE;
     if (ccx_hip_event_record(c->ev[3], c->stream) != 0) return CCX_ERR_DEVICE;
-    if (ccx_hip_memcpy_d2h(host_out, c->d_out, sizeof(double) * 2, c->stream) != 0) return CCX_ERR_DEVICE;
-    if (v1) {
-        const size_t bytes = sizeof(double) * (size_t)(c->no * c->nu);
-        int r = v1_on_device ? ccx_hip_memcpy_d2d(v1, c->d_v1, bytes, c->stream)
-                             : ccx_hip_memcpy_d2h(v1, c->d_v1, bytes, c->stream);
-        if (r != 0 || ccx_hip_sync(c->stream) != 0) return CCX_ERR_DEVICE;
-    }
+    const size_t nv = (size_t)(c->no * c->nu), first = v1 && !v1_on_device ? 0 : nv;
+    if (v1 && v1_on_device && ccx_hip_memcpy_d2d(v1, c->d_v1, sizeof(double) * nv, c->stream) != 0) return CCX_ERR_DEVICE;
+    if (ccx_hip_memcpy_d2h(c->h_res + first, c->d_v1 + first, sizeof(double) * (nv + 2 - first), c->stream) != 0)
+        return CCX_ERR_DEVICE;
+    if (first == 0) memcpy(v1, c->h_res, sizeof(double) * nv);
     float k_ms = 0.0f, t_ms = 0.0f;
-    if (ccx_hip_event_ms(c->ev[1], c->ev[2], &k_ms) != 0 || ccx_hip_event_ms(c->ev[0], c->ev[3], &t_ms) != 0)
+    if (ccx_hip_event_ms(c->ev[1], c->ev[2], &k_ms) != 0 || ccx_hip_event_ms(c->ev[1], c->ev[3], &t_ms) != 0)
         return CCX_ERR_DEVICE;
     c->kernel_ms = k_ms;
     c->total_ms = t_ms;
-    if (etd) *etd = host_out[0];
-    if (ets) *ets = host_out[1];
+    if (etd) *etd = c->h_res[nv];
+    if (ets) *ets = c->h_res[nv + 1];
     return CCX_OK;
 }
 
@@ -988,26 +1005,31 @@ void cc_triples_(double *eh, double *ep, double *v1, double *t1, double *t2, dou
 #define TE_SLOTS 3
 static struct {
     int64_t no, nu, nup, nb, kp, nblk;
-    double *axr, *axc, *bx, *voep, *eh, *ep, *t1, *epart, *v1part, *v1t, *v1, *out;
-    double *t2x, *vmb, *voeb, *in, *x3, *v1p;
-    int *tup, *blocks;
+    double *axr, *axc, *bx, *voep, *ep, *t1, *epart, *v1part, *v1t, *v1;
+    double *t2x, *voeb, *in, *x3, *v1p;
+    int *blocks;
     unsigned int *counter;
-    double *h_ep;
+    double *small, *h_small;   /* the small inputs of a call, on the device and pinned: see te_tuple */
+    double *h_res;             /* pinned: v1 of the slots, etd, ets */
     int ready;
 } g_te;
 
 static void te_free(void)
 {
-    double *d[] = {g_te.axr, g_te.axc, g_te.bx, g_te.voep, g_te.eh, g_te.ep, g_te.t1, g_te.epart, g_te.v1part,
-                   g_te.v1t, g_te.v1, g_te.out, g_te.t2x, g_te.vmb, g_te.voeb, g_te.in, g_te.x3,
-                   g_te.v1p};
+    double *d[] = {g_te.axr, g_te.axc, g_te.bx, g_te.voep, g_te.ep, g_te.t1, g_te.epart, g_te.v1part, g_te.v1t,
+                   g_te.v1, g_te.t2x, g_te.voeb, g_te.in, g_te.x3, g_te.v1p, g_te.small};
     for (size_t q = 0; q < sizeof(d) / sizeof(d[0]); ++q) ccx_hip_free(d[q]);
-    ccx_hip_free(g_te.tup);
     ccx_hip_free(g_te.blocks);
     ccx_hip_free(g_te.counter);
-    free(g_te.h_ep);
+    ccx_hip_host_free(g_te.h_small);
+    ccx_hip_host_free(g_te.h_res);
     memset(&g_te, 0, sizeof(g_te));
 }
+
+/* Layout of a call's small inputs, in doubles: eps_virtual padded to nup; eps_occupied of the slots
+ * (four, the last unused) and the tuple table entry (four ints, two doubles; two unused); then for each of the six ordered position pairs VM (no nu)
+ * and VOE (nu^2). */
+static int64_t te_small_doubles(int64_t no, int64_t nu, int64_t nup) { return nup + 8 + 6 * (no * nu + nu * nu); }
 
 /* the workspace for (no, nu), allocated on first use and whenever the dimensions change */
 static int te_ensure(int64_t no, int64_t nu)
@@ -1026,37 +1048,32 @@ static int te_ensure(int64_t no, int64_t nu)
     DALLOC(g_te.axc, S * nb * nb * kp * 256);
     DALLOC(g_te.bx, S * S * nb * kp * 16);
     DALLOC(g_te.voep, S * S * nup * nup);
-    DALLOC(g_te.eh, S);
     DALLOC(g_te.ep, nup);
     DALLOC(g_te.t1, S * nu);
     DALLOC(g_te.epart, nblk);
     DALLOC(g_te.v1part, nblk * 144);
     DALLOC(g_te.v1t, 3 * nu);
-    DALLOC(g_te.v1, S * nu);
-    DALLOC(g_te.out, 4);
+    DALLOC(g_te.v1, S * nu + 2);
     DALLOC(g_te.t2x, S * nu * nu * no);
-    DALLOC(g_te.vmb, S * S * no * nu);
     DALLOC(g_te.voeb, S * S * nu * nu);
+    DALLOC(g_te.small, te_small_doubles(no, nu, nup));
     DALLOC(g_te.in, nu3);
     DALLOC(g_te.x3, nu);
     DALLOC(g_te.v1p, 3 * nu);
-    DALLOC(g_te.tup, 4);
     DALLOC(g_te.blocks, 4 * nblk);
     DALLOC(g_te.counter, 8);
-    g_te.h_ep = (double *)malloc(sizeof(double) * (size_t)nup);
     h_blk = (int *)malloc(sizeof(int) * 4 * (size_t)nblk);
-    if (!g_te.h_ep || !h_blk) { rc = CCX_ERR_ALLOC; goto fail; }
+    if (!h_blk || ccx_hip_host_malloc((void **)&g_te.h_small, sizeof(double) * (size_t)te_small_doubles(no, nu, nup)) != 0 ||
+        ccx_hip_host_malloc((void **)&g_te.h_res, sizeof(double) * (size_t)(S * nu + 2)) != 0) { rc = CCX_ERR_ALLOC; goto fail; }
     build_blocks(nb, h_blk);
     /* everything a call does not overwrite stays zero and finite */
     if (ccx_hip_zero(g_te.voep, sizeof(double) * (size_t)(S * S * nup * nup), NULL) != 0 ||
-        ccx_hip_zero(g_te.eh, sizeof(double) * (size_t)S, NULL) != 0 ||
         ccx_hip_zero(g_te.t1, sizeof(double) * (size_t)(S * nu), NULL) != 0 ||
         ccx_hip_memcpy_h2d(g_te.blocks, h_blk, sizeof(int) * 4 * (size_t)nblk, NULL) != 0) {
         rc = CCX_ERR_DEVICE;
         goto fail;
     }
-    for (int64_t a = 0; a < nup; ++a) g_te.h_ep[a] = 1.0e3;
-    if (ccx_hip_memcpy_h2d(g_te.ep, g_te.h_ep, sizeof(double) * (size_t)nup, NULL) != 0) { rc = CCX_ERR_DEVICE; goto fail; }
+    for (int64_t a = 0; a < nup; ++a) g_te.h_small[a] = 1.0e3;   /* eps_virtual and its padding */
     free(h_blk);
     g_te.ready = 1;
     return CCX_OK;
@@ -1110,53 +1127,60 @@ static int te_tuple(int64_t no, int64_t nu, const int64_t x[3], int kind, const 
                                 (int)nu, (int)nup, (int)kp, NULL) != 0)
             return CCX_ERR_DEVICE;
     }
-    /* BX panels and VOE blocks of the ordered position pairs (y,z), y != z, at slot pair (sy,sz) */
-    for (int y = 0; y < 3; ++y)
+    /* The small inputs go through one pinned block and one copy: as about fifteen copies with a wait
+     * each they were a third of a call at no=4, nu=87.  The last call's copy has finished: every call
+     * ends with a wait. */
+    double *h = g_te.h_small;
+    if (ep) memcpy(h, ep, sizeof(double) * (size_t)nu);   /* without ep no energy is formed: any finite values do */
+    memcpy(h + nup, h_eh, sizeof(h_eh));
+    const int tup[4] = {sl[0], sl[1], sl[2], kind};
+    memcpy(h + nup + 4, tup, sizeof(tup));
+    struct ccx_pair_pack pk[6];
+    int npair = 0;
+    for (int y = 0; y < 3; ++y)   /* BX panels and VOE blocks of the ordered position pairs, at slot pair (sy,sz) */
         for (int z = 0; z < 3; ++z) {
             if (y == z) continue;
-            const int sy = sl[y], sz = sl[z], sp = sy * TE_SLOTS + sz;
+            const int sp = sl[y] * TE_SLOTS + sl[z];
+            int seen = 0;         /* a degenerate tuple repeats slot pairs */
+            for (int q = 0; q < npair; ++q)
+                if (pk[q].bx == g_te.bx + sp * nb * kp * 16) seen = 1;
+            if (seen) continue;
             const double *vmzy = vm(ud, z, y), *voeyz = voe ? voe(ud, y, z) : NULL;
             if (!vmzy || (voe && !voeyz)) return CCX_ERR_ARG;
-            double *vmd = g_te.vmb + sp * no * nu, *voed = g_te.voeb + sp * nu2;
-            if (ccx_hip_memcpy_h2d(vmd, vmzy, sizeof(double) * (size_t)(no * nu), NULL) != 0 ||
-                (voeyz && ccx_hip_memcpy_h2d(voed, voeyz, sizeof(double) * (size_t)nu2, NULL) != 0))
-                return CCX_ERR_DEVICE;
+            const int64_t o = nup + 8 + npair * (no * nu + nu2);
+            memcpy(h + o, vmzy, sizeof(double) * (size_t)(no * nu));
+            if (voeyz) memcpy(h + o + no * nu, voeyz, sizeof(double) * (size_t)nu2);
             /* T2(:,:,x_y,x_z) sits in the T2(:,:,:,x_z) slab of slot sz */
-            const double *t2yz = g_te.t2x + sz * nu2 * no + x[y] * nu2;
-            if (ccx_hip_pack_pair(t2yz, vmd, voeyz ? voed : NULL, g_te.bx + sp * nb * kp * 16,
-                                  g_te.voep + sp * nup * nup, (int)no, (int)nu, (int)nup, (int)kp, NULL) != 0)
-                return CCX_ERR_DEVICE;
+            pk[npair].t2 = g_te.t2x + sl[z] * nu2 * no + x[y] * nu2;
+            pk[npair].vm = g_te.small + o;
+            pk[npair].voe = voeyz ? g_te.small + o + no * nu : NULL;
+            pk[npair].bx = g_te.bx + sp * nb * kp * 16;
+            pk[npair].voep = g_te.voep + sp * nup * nup;
+            ++npair;
         }
-    if (ep) {
-        memcpy(g_te.h_ep, ep, sizeof(double) * (size_t)nu);
-        if (ccx_hip_memcpy_h2d(g_te.ep, g_te.h_ep, sizeof(double) * (size_t)nup, NULL) != 0) return CCX_ERR_DEVICE;
-    }
-    const int tup[4] = {sl[0], sl[1], sl[2], kind};
-    if (ccx_hip_memcpy_h2d(g_te.eh, h_eh, sizeof(h_eh), NULL) != 0 ||
-        ccx_hip_memcpy_h2d(g_te.tup, tup, sizeof(tup), NULL) != 0)
-        return CCX_ERR_DEVICE;
+    if (ccx_hip_memcpy_h2d_queue(g_te.small, h, sizeof(double) * (size_t)(nup + 8 + npair * (no * nu + nu2)), NULL) != 0 ||
+        ccx_hip_pack_pairs(pk, npair, (int)no, (int)nu, (int)nup, (int)kp, NULL) != 0)
+        goto device;
     int cus = 256;
     if (ccx_hip_cu_count(&cus) != 0 || cus < 1) cus = 256;
     const int grid = (int)(g_te.nblk < cus ? g_te.nblk : cus);
-    if (ccx_hip_triples(0, g_te.axr, g_te.axc, g_te.bx, g_te.voep, g_te.eh, g_te.ep, g_te.tup, g_te.blocks,
+    const double *d_eh = g_te.small + nup;
+    const int *d_tup = (const int *)(g_te.small + nup + 4);   /* a multiple of 16 bytes, as the int4 load wants */
+    if (ccx_hip_triples(0, g_te.axr, g_te.axc, g_te.bx, g_te.voep, d_eh, g_te.small, d_tup, g_te.blocks,
                         g_te.epart, g_te.v1part, w ? g_te.in : NULL, g_te.counter, TE_SLOTS, (int)nu, (int)nup,
                         (int)kp, 1, (int)g_te.nblk, grid, NULL, 0, 1.0, NULL) != 0)
-        return CCX_ERR_DEVICE;
-    if (w && ccx_hip_memcpy_d2h(w, g_te.in, sizeof(double) * (size_t)nu3, NULL) != 0) return CCX_ERR_DEVICE;
+        goto device;
+    if (w && ccx_hip_memcpy_d2h(w, g_te.in, sizeof(double) * (size_t)nu3, NULL) != 0) goto device;
     if (w)
         for (int64_t a = 0; a < nu; ++a) w[a + nu * (a + nu * a)] = 0.0; /* zerot3 */
     if (voe && (etd || v1)) {
-        double out[2];
-        double *hv = (double *)malloc(sizeof(double) * (size_t)(TE_SLOTS * nu));
-        if (!hv) return CCX_ERR_ALLOC;
-        if (ccx_hip_finalize(g_te.epart, g_te.v1part, g_te.tup, g_te.t1, g_te.v1t, g_te.v1, g_te.out,
-                             TE_SLOTS, (int)nu, 1, (int)g_te.nblk, NULL) != 0 ||
-            ccx_hip_memcpy_d2h(out, g_te.out, sizeof(out), NULL) != 0 ||
-            ccx_hip_memcpy_d2h(hv, g_te.v1, sizeof(double) * (size_t)(TE_SLOTS * nu), NULL) != 0) {
-            free(hv);
-            return CCX_ERR_DEVICE;
-        }
-        if (etd) *etd += out[0];
+        const size_t nv = (size_t)(TE_SLOTS * nu);
+        double *hv = g_te.h_res;
+        if (ccx_hip_finalize(g_te.epart, g_te.v1part, d_tup, g_te.t1, g_te.v1t, g_te.v1, g_te.v1 + nv, TE_SLOTS, (int)nu,
+                             1, (int)g_te.nblk, NULL) != 0 ||
+            ccx_hip_memcpy_d2h(hv, g_te.v1, sizeof(double) * (nv + 2), NULL) != 0)
+            goto device;
+        if (etd) *etd += hv[nv];
         if (v1)   /* slot column s -> occupied column of the first position holding it */
             for (int s2 = 0; s2 < nslot; ++s2) {
                 int64_t col = -1;
@@ -1164,9 +1188,13 @@ static int te_tuple(int64_t no, int64_t nu, const int64_t x[3], int kind, const 
                     if (sl[p] == s2) col = x[p];
                 for (int64_t a = 0; a < nu; ++a) v1[a + nu * col] += hv[a + nu * s2];
             }
-        free(hv);
+    } else if (!w && ccx_hip_sync(NULL) != 0) {
+        return CCX_ERR_DEVICE;
     }
     return CCX_OK;
+device:   /* the pinned block must not be rewritten under a copy that is still queued */
+    ccx_hip_sync(NULL);
+    return CCX_ERR_DEVICE;
 }
 
 /* block lookups for the two argument styles: full VM / VOE arrays, or the six pair slices */
@@ -1238,7 +1266,7 @@ static int t1wt3_host(int64_t no, int64_t nu, int64_t ii, int64_t jj, int64_t kk
         for (int r = 0; r < 3; ++r)
             for (int64_t a = 0; a < nu; ++a) v1[a + nu * rows[r]] += vfac * v1p[3 * a + r];
     }
-done:   /* only ep[0..nu) was overwritten: the padding the tuple kernel reads stays finite */
+done:
     free(x3); free(v1p);
     return rc;
 }

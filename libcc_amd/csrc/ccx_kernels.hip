@@ -31,6 +31,9 @@
 // and holds D[l/16 + 4v][l%16], v = 0..3 (checked on the device).
 
 #include "ccx_item.h"
+extern "C" {
+#include "ccx_dev.h"
+}
 #include <stdlib.h>
 #include <string.h>
 
@@ -169,30 +172,32 @@ __global__ void __launch_bounds__(256) pack_rest_kernel(RestArgs a)
     }
 }
 
-// BX of one ordered pair (y,z): BX[y,z](g,K) = T2(g,K,y,z) for K < nu, -VM(K-nu,g,z,y) for K < nu+no;
-// t2yz = T2(:,:,y,z) (nu^2), vmzy = VM(:,:,z,y) (no*nu), bx = the pair's [nb][kp][16] panel set.
-__global__ void pack_bx_pair_kernel(const double *__restrict__ t2yz, const double *__restrict__ vmzy,
-                                    double *__restrict__ bx, int no, int nu, int nb, int kp)
+// The pairs of one tuple (at most six) in one launch: BX[y,z](g,K) = T2(g,K,y,z) for K < nu, then
+// -VM(K-nu,g,z,y), as [g block][kp][16], and the padded VOE block of each pair that has one.
+// t2 = T2(:,:,y,z) (nu^2), vm = VM(:,:,z,y) (no nu), voe = VOE(:,:,y,z).  Work groups 0 .. npb-1 of
+// a pair build BX, the others VOE; as two launches a pair these were 12 of the call's 30.
+struct PairArgs {
+    ccx_pair_pack p[6];
+    int no, nu, nup, kp, npb, npv;
+};
+__global__ void __launch_bounds__(256) pack_pairs_kernel(PairArgs a)
 {
-    const long long total = (long long)nb * kp * 16;
-    for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
-         idx += (long long)gridDim.x * blockDim.x) {
-        const int gl = (int)(idx & 15);
-        const int K = (int)((idx >> 4) % kp);
-        const int g = (int)((idx >> 4) / kp) * TB + gl;
-        double v = 0.0;
-        if (g < nu) {
-            if (K < nu) v = t2yz[g + (long long)nu * K];
-            else if (K < nu + no) v = -vmzy[(K - nu) + (long long)no * g];
-        }
-        bx[idx] = v;
+    const int per = a.npb + a.npv, wg = blockIdx.x % per;
+    const ccx_pair_pack &p = a.p[blockIdx.x / per];
+    if (wg >= a.npb) {
+        if (p.voe) pack_voe(p.voe, p.voep, 1, a.nu, a.nup, wg - a.npb, a.npv);
+        return;
     }
-}
-
-__global__ void __launch_bounds__(256) pack_voe_kernel(const double *__restrict__ voe, double *__restrict__ out, int no,
-                                                       int nu, int nup)
-{
-    pack_voe(voe, out, no, nu, nup, blockIdx.x, gridDim.x);
+    const long long total = (long long)(a.nup / TB) * a.kp * 16;
+    for (long long idx = wg * 256LL + threadIdx.x; idx < total; idx += a.npb * 256LL) {
+        const int gl = (int)(idx & 15), gk = (int)(idx >> 4), gb = gk / a.kp, K = gk - gb * a.kp, g = gb * TB + gl;
+        double v = 0.0;
+        if (g < a.nu) {
+            if (K < a.nu) v = p.t2[g + (long long)a.nu * K];
+            else if (K < a.nu + a.no) v = -p.vm[(K - a.nu) + (long long)a.no * g];
+        }
+        p.bx[idx] = v;
+    }
 }
 
 // ---------------------------------------------------------------------------------
@@ -844,6 +849,20 @@ int ccx_hip_memcpy_d2d(void *dst, const void *src, size_t bytes, void *stream)
     return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, (hipStream_t)stream) == hipSuccess ? 0 : 1;
 }
 
+int ccx_hip_memcpy_h2d_queue(void *dst, const void *src, size_t bytes, void *stream)
+{
+    if (bytes == 0) return 0;
+    return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, (hipStream_t)stream) == hipSuccess ? 0 : 1;
+}
+
+int ccx_hip_host_malloc(void **p, size_t bytes)
+{
+    *p = nullptr;
+    return hipHostMalloc(p, bytes, hipHostMallocDefault) == hipSuccess ? 0 : 1;
+}
+
+int ccx_hip_host_free(void *p) { return (p == nullptr || hipHostFree(p) == hipSuccess) ? 0 : 1; }
+
 int ccx_hip_sync(void *stream) { return hipStreamSynchronize((hipStream_t)stream) == hipSuccess ? 0 : 1; }
 
 int ccx_hip_cu_count(int *n)
@@ -895,15 +914,17 @@ int ccx_hip_pack_ax_one(int layout, const double *cube, const double *t2_x, doub
     return launch_pack_ax(layout == 1 ? V_PACKED : V_VE, cube, t2_x, axr_x, axc_x, no, nu, nup, kp, 1, (hipStream_t)stream);
 }
 
-// The FP64 BX panels of one ordered pair (y,z) and, when voe_yz is non-null, its padded VOE block:
-// t2_yz = T2(:,:,y,z), vm_zy = VM(:,:,z,y), voe_yz = VOE(:,:,y,z).
-int ccx_hip_pack_pair(const double *t2_yz, const double *vm_zy, const double *voe_yz, double *bx_yz,
-                      double *voep_yz, int no, int nu, int nup, int kp, void *stream)
+// BX panels and padded VOE blocks of n <= 6 ordered pairs (PairArgs)
+int ccx_hip_pack_pairs(const struct ccx_pair_pack *p, int n, int no, int nu, int nup, int kp, void *stream)
 {
-    hipStream_t s = (hipStream_t)stream;
+    if (n < 1 || n > 6) return 3;
     const int nb = nup / TB;
-    pack_bx_pair_kernel<<<grid_for((long long)nb * kp * 16), 256, 0, s>>>(t2_yz, vm_zy, bx_yz, no, nu, nb, kp);
-    if (voe_yz) pack_voe_kernel<<<nb * nb < 65536 ? nb * nb : 65536, 256, 0, s>>>(voe_yz, voep_yz, 1, nu, nup);
+    PairArgs a;
+    for (int q = 0; q < n; ++q) a.p[q] = p[q];
+    a.no = no; a.nu = nu; a.nup = nup; a.kp = kp;
+    a.npb = grid_for((long long)nb * kp * 16);
+    a.npv = p[0].voe ? (nb * nb < 65536 ? nb * nb : 65536) : 0;
+    pack_pairs_kernel<<<n * (a.npb + a.npv), 256, 0, (hipStream_t)stream>>>(a);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
