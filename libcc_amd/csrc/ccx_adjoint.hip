@@ -82,7 +82,7 @@ __device__ __forceinline__ double staged_w(const double *ws, int p, int bb, int 
     return ws[((p * BPW + bb) * 4 + v) * NTHR + tid];
 }
 
-__device__ void adj_epilogue(const AdjArgs &ga, double *lds, double (*red)[112], const ItemCtx &it,
+__device__ __forceinline__ void adj_epilogue(const AdjArgs &ga, double *lds, double (*red)[112], const ItemCtx &it,
                              long long item, int tl, int tkind, int mult, bool swap_bc, const double *ws, int wave,
                              int lane, int tid)
 {
@@ -106,7 +106,6 @@ __device__ void adj_epilogue(const AdjArgs &ga, double *lds, double (*red)[112],
         T[tid] = a < g.nu ? ga.t1[it.tpos[y] + (long long)g.no * a] : 0.0;
     }
     for (int idx = tid; idx < 36 * 256; idx += NTHR) D[idx] = 0.0;
-    for (int idx = lane; idx < 112; idx += 64) red[wave][idx] = 0.0;
     __syncthreads();
 
     const double dijk = g.eh[it.tpos[0]] + g.eh[it.tpos[1]] + g.eh[it.tpos[2]];
@@ -122,14 +121,22 @@ __device__ void adj_epilogue(const AdjArgs &ga, double *lds, double (*red)[112],
     // The three passes run over this thread's 8 points (rows a = row(lane,v), batches
     // b = wave*BPW+bb, column c = lane&15) with a run-time loop over v, so only one row
     // of points is live at a time.
-    // pass 1: energy and v1 partials (the forward epilogue), reduced per point:
+    // pass 1: energy and v1 partials (the forward epilogue's arithmetic): the sums over what a lane
+    // holds stay in registers, so the lanes are added up once per row for role a and once per item
+    // for roles b and c (once per point, as this pass used to do, was six times the additions).
     //   role a (rows al): over the 16 lanes of a row group  -> rw[al*3 + p]
     //   role b (rows bl): over the wave                     -> rw[48 + bb*3 + p]
     //   role c (rows cl): over the four row groups          -> rw[54 + cl*3 + p]
+    double rb[BPW][3], rc[3] = {0, 0, 0};
+#pragma unroll
+    for (int bb = 0; bb < BPW; ++bb)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) rb[bb][p] = 0.0;
 #pragma unroll 1
     for (int v = 0; v < 4; ++v) {
         const int al = Mfma<double>::row(lane, v);
         const int ag = A * TB + al;
+        double ra[3] = {0, 0, 0};
         static_for<BPW>([&](auto BB) __attribute__((always_inline)) {
             constexpr int bb = decltype(BB)::value;
             const int bl = wave * BPW + bb;
@@ -143,36 +150,38 @@ __device__ void adj_epilogue(const AdjArgs &ga, double *lds, double (*red)[112],
                 const double sq = w[0] * w[0] + w[1] * w[1] + w[2] * w[2] + w[3] * w[3] + w[4] * w[4] + w[5] * w[5];
                 esum += (6.0 * sq + 2.0 * ev * ev + 2.0 * od * od - 8.0 * ev * od) * inv;
             }
+            double d[3][3];
+            even_odd_differences(w, inv, d);
             const int el[3] = {al, bl, cl};
-            double ra[3] = {0, 0, 0}, rb[3] = {0, 0, 0}, rc[3] = {0, 0, 0};
             static_for<6>([&](auto S) __attribute__((always_inline)) {
                 constexpr int s = decltype(S)::value;
                 constexpr int r0 = PERM[s][0], r1 = PERM[s][1], r2 = PERM[s][2];
                 constexpr int bpair = pair_index(r1, r2);
                 static_for<6>([&](auto PP) __attribute__((always_inline)) {
                     constexpr int p = decltype(PP)::value;
-                    constexpr int q0 = wsrc_comp(p, s, 0), q1 = wsrc_comp(p, s, 2);
-                    constexpr int q2 = wsrc_comp(p, s, 1), q3 = wsrc_comp(p, s, 3);
                     constexpr int qr = pair_index(PERM[p][1], PERM[p][2]);
-                    const double z = 2.0 * w[q0] - 2.0 * w[q1] - w[q2] + w[q3];
-                    const double cv = z * inv * V[(qr * 6 + bpair) * VBLK + el[r1] * VSTR + el[r2]];
-                    if constexpr (r0 == 0) ra[PERM[p][0]] += cv;
-                    else if constexpr (r0 == 1) rb[PERM[p][0]] += cv;
-                    else rc[PERM[p][0]] += cv;
+                    const double z = z_term<s, p>(d), vv = V[(qr * 6 + bpair) * VBLK + el[r1] * VSTR + el[r2]];
+                    if constexpr (r0 == 0) ra[PERM[p][0]] = fma(z, vv, ra[PERM[p][0]]);
+                    else if constexpr (r0 == 1) rb[bb][PERM[p][0]] = fma(z, vv, rb[bb][PERM[p][0]]);
+                    else rc[PERM[p][0]] = fma(z, vv, rc[PERM[p][0]]);
                 });
             });
-#pragma unroll
-            for (int p = 0; p < 3; ++p) {
-                const double sa = group16_sum(ra[p]);
-                if (cl == 0) rw[al * 3 + p] += sa;
-                const double sb = wave_sum(rb[p]);
-                if (lane == 0) rw[48 + bb * 3 + p] += sb;
-                double sc = rc[p];
-                sc += __shfl_xor(sc, 16, 64);
-                sc += __shfl_xor(sc, 32, 64);
-                if (lane < 16) rw[54 + cl * 3 + p] += sc;
-            }
         });
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const double sa = group16_sum(ra[p]);
+            if (cl == 0) rw[al * 3 + p] = sa;
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+        for (int bb = 0; bb < BPW; ++bb) {
+            const double sb = wave_sum(rb[bb][p]);
+            if (lane == 0) rw[48 + bb * 3 + p] = sb;
+        }
+        const double sc = add_xor32(add_xor16(rc[p]));
+        if (lane < 16) rw[54 + cl * 3 + p] = sc;
     }
     {
         const double s = wave_sum(esum);
@@ -278,32 +287,25 @@ __device__ void adj_epilogue(const AdjArgs &ga, double *lds, double (*red)[112],
 #pragma unroll
             for (int p = 0; p < 6; ++p) w[p] = staged_w(ws, p, bb, v, tid);
             const double inv = 1.0 / (dijk - g.ep[ag] - g.ep[bg] - g.ep[cg]);
+            double d[3][3];
+            even_odd_differences(w, inv, d);
             const int el[3] = {al, bl, cl};
             static_for<6>([&](auto S) __attribute__((always_inline)) {
                 constexpr int s = decltype(S)::value;
                 constexpr int r0 = PERM[s][0], r1 = PERM[s][1], r2 = PERM[s][2];
                 static_for<6>([&](auto PP) __attribute__((always_inline)) {
                     constexpr int p = decltype(PP)::value;
-                    constexpr int q0 = wsrc_comp(p, s, 0), q1 = wsrc_comp(p, s, 2);
-                    constexpr int q2 = wsrc_comp(p, s, 1), q3 = wsrc_comp(p, s, 3);
-                    const double z = 2.0 * w[q0] - 2.0 * w[q1] - w[q2] + w[q3];
-                    const double dv = z * inv * T[(PERM[p][0] * 3 + r0) * 16 + el[r0]];
+                    const double dv = z_term<s, p>(d) * T[(PERM[p][0] * 3 + r0) * 16 + el[r0]];
                     if constexpr (s < 2) {
                         // a-axis: sum over the four row groups, then over v by the same lane
                         // (s = 0 -> target (b, c); s = 1 -> (c, b))
-                        double r = dv;
-                        r += __shfl_xor(r, 16, 64);
-                        r += __shfl_xor(r, 32, 64);
+                        const double r = add_xor32(add_xor16(dv));
                         if (lane < 16) D[(s * 6 + p) * 256 + el[r1] * 16 + el[r2]] += r;
                     } else if constexpr (s < 4) {
                         dB[s - 2][p] += dv;
                     } else {
                         // c-axis: sum over the 16 lanes of equal row (s = 4 -> (a,b); 5 -> (b,a))
-                        double r = dv;
-                        r += __shfl_xor(r, 1, 64);
-                        r += __shfl_xor(r, 2, 64);
-                        r += __shfl_xor(r, 4, 64);
-                        r += __shfl_xor(r, 8, 64);
+                        const double r = group16_sum(dv);
                         if (cl == 0) D[(s * 6 + p) * 256 + el[r1] * 16 + el[r2]] = r;
                     }
                 });
@@ -362,18 +364,22 @@ __global__ void __launch_bounds__(NTHR, 1) adj_item_kernel(AdjArgs ga)
     extern __shared__ double lds[];
     __shared__ double red[NWAVE][112];
     __shared__ long long next_item;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const TriplesArgs &g = ga.f;
     const long long nlocal = (long long)ga.tcount * g.nblk;
     for (;;) {
+        // new for every item, so that addresses are computed where they are used (triples_kernel)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63;
         if (tid == 0) next_item = (long long)atomicAdd(g.counter, 1u);
         __syncthreads();
         const long long li = next_item;
         __syncthreads();
         if (li >= nlocal) break;
-        const int tl = __builtin_amdgcn_readfirstlane((int)(li / g.nblk));
-        const int q = __builtin_amdgcn_readfirstlane((int)(li % g.nblk));
+        // block triple major within the batch, as the forward kernel's order
+        const int q = __builtin_amdgcn_readfirstlane((int)(li / ga.tcount));
+        const int tl = __builtin_amdgcn_readfirstlane((int)(li % ga.tcount));
         const int t = ga.t0 + tl;
         const long long item = (long long)t * g.nblk + q;
         int tkind, mult;

@@ -491,6 +491,29 @@ __device__ __forceinline__ void complete_orderings(double *lds, typename Mfma<T>
     }
 }
 
+// Z = 2 w[q0] - 2 w[q1] - w[q2] + w[q3] (q = sigma, sigma o (1,0,2), sigma o (0,2,1), sigma o (1,2,0) of
+// the term of placement s and ordering p) is a combination of two differences of an even and an odd
+// ordering, so with the nine differences over D at hand a term is one multiply-add.
+__device__ __forceinline__ void even_odd_differences(const double (&w)[6], double inv, double (&d)[3][3])
+{
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+#pragma unroll
+        for (int y = 0; y < 3; ++y) d[x][y] = (w[EVEN[x]] - w[ODD[y]]) * inv;
+}
+
+template <int S, int P>
+__device__ __forceinline__ double z_term(const double (&d)[3][3])
+{
+    constexpr int q0 = wsrc_comp(P, S, 0), q1 = wsrc_comp(P, S, 2), q2 = wsrc_comp(P, S, 1), q3 = wsrc_comp(P, S, 3);
+    static_assert(is_even(q0) == is_even(q3) && is_even(q1) == is_even(q2) && is_even(q0) != is_even(q1),
+                  "parities of a Z term");
+    constexpr int e0 = parity_rank(is_even(q0) ? q0 : q1), o0 = parity_rank(is_even(q0) ? q1 : q0);
+    constexpr int e1 = parity_rank(is_even(q0) ? q3 : q2), o1 = parity_rank(is_even(q0) ? q2 : q3);
+    const double z = fma(2.0, d[e0][o0], d[e1][o1]);
+    return is_even(q0) ? z : -z;
+}
+
 // Whether form FK (0 FP64, 1 FP32, 2-4 split) runs a degenerate tuple on an orbit with equal
 // blocks in the modes that use both symmetries (two orderings, or one for three equal blocks).
 // Measured at no=24, nu=216: FP64 1143 -> 1132 ms, BF16x4 1375 -> 1359, FP8x4 4116 -> 4057; FP32

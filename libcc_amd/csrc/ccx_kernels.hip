@@ -398,14 +398,8 @@ __device__ __forceinline__ void item_epilogue(const TriplesArgs &g, double *lds,
             const double ev = w[0] + w[3] + w[4], od = w[1] + w[2] + w[5];
             const double sq = w[0] * w[0] + w[1] * w[1] + w[2] * w[2] + w[3] * w[3] + w[4] * w[4] + w[5] * w[5];
             esum += (6.0 * sq + 2.0 * ev * ev + 2.0 * od * od - 8.0 * ev * od) * inv;
-            // Z = 2 w[q0] - 2 w[q1] - w[q2] + w[q3] is a combination of two differences of an even and
-            // an odd ordering, so with the nine differences over D at hand each of the 36 terms is
-            // two multiply-adds.
             double d[3][3];
-#pragma unroll
-            for (int x = 0; x < 3; ++x)
-#pragma unroll
-                for (int y = 0; y < 3; ++y) d[x][y] = (w[EVEN[x]] - w[ODD[y]]) * inv;
+            even_odd_differences(w, inv, d);
             const int el[3] = {al, bl, cl};
             static_for<6>([&](auto S) __attribute__((always_inline)) {
                 constexpr int s = decltype(S)::value;
@@ -413,17 +407,8 @@ __device__ __forceinline__ void item_epilogue(const TriplesArgs &g, double *lds,
                 constexpr int bpair = pair_index(r1, r2);
                 static_for<6>([&](auto PP) __attribute__((always_inline)) {
                     constexpr int p = decltype(PP)::value;
-                    constexpr int q0 = wsrc_comp(p, s, 0);   // sigma
-                    constexpr int q1 = wsrc_comp(p, s, 2);   // sigma o (1,0,2)
-                    constexpr int q2 = wsrc_comp(p, s, 1);   // sigma o (0,2,1)
-                    constexpr int q3 = wsrc_comp(p, s, 3);   // sigma o (1,2,0)
-                    static_assert(is_even(q0) == is_even(q3) && is_even(q1) == is_even(q2) && is_even(q0) != is_even(q1),
-                                  "parities of a Z term");
-                    constexpr int e0 = parity_rank(is_even(q0) ? q0 : q1), o0 = parity_rank(is_even(q0) ? q1 : q0);
-                    constexpr int e1 = parity_rank(is_even(q0) ? q3 : q2), o1 = parity_rank(is_even(q0) ? q2 : q3);
                     constexpr int qr = pair_index(PERM[p][1], PERM[p][2]);
-                    const double za = fma(2.0, d[e0][o0], d[e1][o1]);
-                    const double z = is_even(q0) ? za : -za;
+                    const double z = z_term<s, p>(d);
                     const double vv = lds[(qr * 6 + bpair) * VBLK + el[r1] * VSTR + el[r2]];
                     if constexpr (r0 == 0) va[v][PERM[p][0]] = fma(z, vv, va[v][PERM[p][0]]);
                     else if constexpr (r0 == 1) vb[bb][PERM[p][0]] = fma(z, vv, vb[bb][PERM[p][0]]);
