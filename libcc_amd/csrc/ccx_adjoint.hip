@@ -442,7 +442,8 @@ constexpr int GTHR = 512;                 // GEMM work group: 8 waves, 2 per SIM
 constexpr int GBPW = 2;                   // gax: rows b per wave
 constexpr int GCH = 128;                  // K columns per work group (8 MFMA tiles)
 constexpr int GCT = GCH / 16;
-constexpr int BS_STR = 17;                // padded row of the staged BX / AX slices
+constexpr int BS_STR = 17;                // padded row of the staged BX slices
+constexpr int GBX_TILES = 19;             // gbx: gamma and K tiles of a work group (two 4 KB buffers each)
 }  // namespace
 
 struct GemmArgs {
@@ -456,7 +457,7 @@ struct GemmArgs {
     const int *uoff;        // CSR offsets into ent, per ulist entry
     const int *ent;         // (tl, sigma) pairs
     double *part;           // gbx: per (entry, split, chunk, gamma group) partial tiles
-    int no, nup, nb, kp, nchunk, gt, ngg, nsplit;
+    int no, nu, nup, nb, kp, nchunk, gt, kt, ngg, nsplit;   // gbx: tiles gt x kt of a work group
     int ch0;                // gax: first K chunk of this launch (nchunk chunks from there)
 };
 
@@ -588,159 +589,163 @@ __global__ void __launch_bounds__(GTHR, 1) gax_kernel(GemmArgs a)
 //   part(g, K) = sum Wbar_t(e_u = a, e_v = b, e_wf = g) AX[t[xp]](a,b,K).
 // One work group per (entry, split, chunk, group), so pairs that collect many entries in a
 // batch spread over many work groups; gbx_reduce_kernel adds the partials of a pair in a
-// fixed order.  A panel is walked in 16 slices of fixed e_sa (sa = axis 0 when u or v is 0,
-// else axis 1), each slice staged in LDS: Wbar (16 x gamma) and AX (16 x 128 K).  Wave w
-// owns K tile w and all gamma tiles.
-template <int GT>
+// fixed order.  A panel is walked in steps of two neighbouring slices of fixed e_sa (sa = axis 0 when
+// u or v is 0, else axis 1), the pair of outer indices that the AX slab interleaves.
+//
+// Bound by the matrix cores.  A step's slices, Wbar (2 x 16 x gamma) and AX (2 x 16 x K), go straight
+// from global memory into the other of two LDS buffers while this step's MFMAs run, without
+// registers, LDS stores or padding: 16-byte units are permuted at the source so that the fragment
+// reads spread over the banks.  Wave w computes gamma tiles of quarter w & 3 (3 - (w & 3) for
+// the upper four waves, so that the two waves of a SIMD share the remainder evenly) and the half
+// w >> 2 of the K tiles.  Slices and contraction steps that hold only padding are left out.  (Staged
+// through registers, one slice a step, K chunks always 8 tiles: 5.50 ms at no=8, nu=120 and 117 ms at
+// no=14, nu=150, where kp = 164 ran 16 K tiles for 11.)
+template <int GM, int KN>   // most gamma tiles and K tiles of a wave
 __global__ void __launch_bounds__(GTHR, 1) gbx_kernel(GemmArgs a)
 {
     extern __shared__ double lds[];
-    constexpr int gstr = GT * 16 + 1;     // padded row of the staged Wbar slice
-    double *WS = lds;                     // [2][16 * gstr]
-    double *AS = lds + 2 * 16 * gstr;     // [2][GCH * BS_STR]
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    typedef __attribute__((address_space(3))) void lds_void;
+    typedef const __attribute__((address_space(1))) void g_void;
+    const int GT = a.gt, KT = a.kt;
+    const int bufd = (GT + KT) * 512;     // doubles of a buffer: [GT][slice 2][256], then [4 KT][64][2]
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int u = blockIdx.x;
     const int gg = u % a.ngg; u /= a.ngg;
     const int ch = u % a.nchunk; u /= a.nchunk;
     const int rs = u % a.nsplit; u /= a.nsplit;
     const int e = u;                      // entry (CSR position)
     const int r0_beg = rs * a.nb / a.nsplit, r0_end = (rs + 1) * a.nb / a.nsplit;
-    const int K0 = ch * GCH;
-    const int G0 = gg * GT;
-    const int ngt = (G0 + GT <= a.nb) ? GT : a.nb - G0;   // tiles past ngt are zero
-    const long long cube = (long long)a.nb * a.nb * a.nb * 4096;
-    const int nsteps = (r0_end - r0_beg) * a.nb * 16;
-    constexpr int nw = GT * 256;          // Wbar slice elements (zero past ngt tiles)
+    const int G0 = gg * GT, kb0 = ch * KT * 4;
+    const int tl = __builtin_amdgcn_readfirstlane(a.ent[2 * e]), sg = __builtin_amdgcn_readfirstlane(a.ent[2 * e + 1]);
+    const int4 tp = reinterpret_cast<const int4 *>(a.tuples)[a.t0 + tl];
+    const Sigma S = SIG[sg & 7];
+    const double wgt = (sg & 8) ? 2.0 : 1.0;   // a merged pair of a degenerate tuple
+    const int sa = (S.u == 0 || S.v == 0) ? 0 : 1, hi = sa == 0 ? 1 : 0;
+    const bool sa_u = sa == S.u;
+    const bool st_tr = (sa_u ? S.v : S.u) == hi;   // the slice's (hi, 2) axes are (o, g), else (g, o)
+    const int xo = __builtin_amdgcn_readfirstlane(S.xp == 0 ? tp.x : S.xp == 1 ? tp.y : tp.z);
+    const long long gstep = (S.wf == 0 ? (long long)a.nb * a.nb : S.wf == 1 ? a.nb : 1) * 4096;
+    const double *cube = a.wbar + tl * ((long long)a.nb * a.nb * a.nb * 4096);
+    const double *ax = (sa_u ? a.axr : a.axc) + (long long)xo * a.nb * a.nb * (256LL * a.kp);
+    const int last = a.nu - (a.nb - 1) * TB;       // real indices of the last block
 
-    d4 acc[GT];
-#pragma unroll
-    for (int i = 0; i < GT; ++i) acc[i] = d4{0, 0, 0, 0};
+    // this wave's tiles
+    const int gq = wave < 4 ? wave : 7 - wave, kh = wave >> 2;
+    const int g_beg = GT * gq / 4, gn = GT * (gq + 1) / 4 - g_beg, k_beg = KT * kh / 2, kn = KT * (kh + 1) / 2 - k_beg;
 
-    // Staging registers.  The Wbar slice is read in memory order: with the slice axis sa
-    // fixed, the block element offset is m>>4 along axis hi (1 if sa = 0, else 0) and m&15
-    // along axis 2, so a wave reads 128-byte runs whatever sigma is.
-    double2 rw[4];
-    double ra[4];
-    double rwgt = 1.0;                    // weight of the staged entry, applied when stashing
-    int st_tr;                            // 1: the slice's (hi, 2) axes are (o, g); 0: (g, o)
-    auto fetch = [&](int step) {
-        int r = step;
-        const int sidx = r & 15; r >>= 4;
-        const int R1 = r % a.nb, R0 = r0_beg + r / a.nb;
-        const int tl = a.ent[2 * e], sg = a.ent[2 * e + 1];
-        const int4 tp = reinterpret_cast<const int4 *>(a.tuples)[a.t0 + tl];
-        const int tpos[3] = {tp.x, tp.y, tp.z};
-        const Sigma S = SIG[sg & 7];
-        rwgt = (sg & 8) ? 2.0 : 1.0;      // a merged pair of a degenerate tuple
-        const int sa = (S.u == 0 || S.v == 0) ? 0 : 1;
-        const int hi = sa == 0 ? 1 : 0;
-        const int oa = (sa == S.u) ? S.v : S.u;
-        st_tr = (oa == hi) ? 1 : 0;
-        int bc[3];
-        bc[S.u] = R0; bc[S.v] = R1; bc[S.wf] = G0;
-        const long long gstep = S.wf == 0 ? (long long)a.nb * a.nb : S.wf == 1 ? a.nb : 1;
-        const double *wbase = a.wbar + tl * cube + (((long long)bc[0] * a.nb + bc[1]) * a.nb + bc[2]) * 4096 +
-                              (sa == 0 ? sidx * 256 : sidx * 16);
-        const int hstr = sa == 0 ? 16 : 256;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int idx = tid + k * GTHR;               // double2 index in the slice
-            double2 v = {0.0, 0.0};
-            if (idx < nw / 2) {
-                const int gt_l = idx >> 7, m = (idx & 127) * 2;
-                if (gt_l < ngt)
-                    v = *reinterpret_cast<const double2 *>(wbase + gt_l * gstep * 4096 + (m >> 4) * hstr + (m & 15));
-            }
-            rw[k] = v;
+    // per-lane source offsets of the direct loads (rows h of 128 B, units permuted by h & 7)
+    const int h8 = lane >> 3, un = 2 * ((lane & 7) ^ (h8 & 7));
+    const int w_hstr = sa == 0 ? 16 : 256, w_sstr = sa == 0 ? 256 : 16;
+    auto fetch = [&](int R0, int R1, int sp, int buf) __attribute__((always_inline)) {
+        double *W = lds + buf * bufd, *A = W + GT * 512;
+        const int b0 = S.u == 0 ? R0 : S.v == 0 ? R1 : G0, b1 = S.u == 1 ? R0 : S.v == 1 ? R1 : G0,
+                  b2 = S.u == 2 ? R0 : S.v == 2 ? R1 : G0;
+        const double *wb = cube + (((long long)b0 * a.nb + b1) * a.nb + b2) * 4096 + 2 * sp * w_sstr + h8 * w_hstr + un;
+#pragma unroll 1
+        for (int c = wave; c < GT * 4; c += GTHR / 64) {       // chunk: tile, slice, half of the rows
+            const int t = c >> 2, tc = G0 + t < a.nb ? t : a.nb - 1 - G0;   // tiles past the last are not used
+            __builtin_amdgcn_global_load_lds((g_void *)(wb + tc * gstep + ((c >> 1) & 1) * w_sstr + (c & 1) * 8 * w_hstr),
+                                             (lds_void *)(W + c * 128), 16, 0, 0);
         }
-        // AX slice: row layout (fixed alpha = e_u) or column layout (fixed beta = e_v); the
-        // slab interleaves the outer indices 2w, 2w+1 per lane: element (K, o) of outer index
-        // sidx sits at ((sidx/2 * kp/4 + K/4) * 64 + (K%4)*16 + o) * 2 + sidx%2 of the panel
-        const double *src = (sa == S.u ? a.axr : a.axc) +
-                            (((long long)tpos[S.xp] * a.nb + R0) * a.nb + R1) * (256LL * a.kp) +
-                            (long long)(sidx >> 1) * (32LL * a.kp) + (sidx & 1);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = tid + k * GTHR;                 // (K, o) of the 128 x 16 slice
-            const int Kl = e >> 4, o = e & 15, K = K0 + Kl;
-            ra[k] = K < a.kp ? src[((long long)(K >> 2) * 64 + (K & 3) * 16 + o) * 2] : 0.0;
-        }
-    };
-    auto stash = [&](int buf) {
-        double *W = WS + buf * 16 * gstr;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int idx = tid + k * GTHR;
-            if (idx < nw / 2) {
-                const int gt_l = idx >> 7, m = (idx & 127) * 2;
-                const int h = m >> 4, l = m & 15;     // l, l+1 along axis 2
-                if (st_tr) {                          // o = h, g = l, l+1
-                    W[h * gstr + gt_l * 16 + l] = rw[k].x;
-                    W[h * gstr + gt_l * 16 + l + 1] = rw[k].y;
-                } else {                              // o = l, l+1, g = h
-                    W[l * gstr + gt_l * 16 + h] = rw[k].x;
-                    W[(l + 1) * gstr + gt_l * 16 + h] = rw[k].y;
-                }
-            }
-        }
-        double *As = AS + buf * GCH * BS_STR;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = tid + k * GTHR;
-            As[(e >> 4) * BS_STR + (e & 15)] = ra[k] * rwgt;
+        const double *ap = ax + ((long long)R0 * a.nb + R1) * (256LL * a.kp) + (long long)sp * (32LL * a.kp);
+#pragma unroll 1
+        for (int c = wave; c < KT * 4; c += GTHR / 64) {       // chunk: K/4
+            const int kb = kb0 + c < a.kp / 4 ? kb0 + c : a.kp / 4 - 1;     // columns past kp are not used
+            const int k4 = lane >> 4, o = (lane & 15) ^ (((c & 3) << 2) | k4);
+            __builtin_amdgcn_global_load_lds((g_void *)(ap + (long long)kb * 128 + (k4 * 16 + o) * 2),
+                                             (lds_void *)(A + c * 128), 16, 0, 0);
         }
     };
 
-    if (nsteps > 0) {
-        fetch(0);
-        stash(0);
-    }
+    d4 acc[GM][KN];
+#pragma unroll
+    for (int i = 0; i < GM; ++i)
+#pragma unroll
+        for (int j = 0; j < KN; ++j) acc[i][j] = d4{0, 0, 0, 0};
+    const int m16 = lane & 15, q4 = lane >> 4;
+
+    // one step for a wave of ng gamma and nk K tiles (compile time: no MFMA behind a branch)
+    auto compute = [&](auto NG, auto NK, int buf, int nkq) __attribute__((always_inline)) {
+        constexpr int ng = decltype(NG)::value, nk = decltype(NK)::value;
+        if constexpr (ng > 0 && nk > 0) {
+            const double *W = lds + buf * bufd + g_beg * 512;
+            const double2 *A = reinterpret_cast<const double2 *>(lds + buf * bufd + GT * 512) + k_beg * 256;
+            for (int kq = 0; kq < nkq; ++kq) {
+                const int o = 4 * kq + q4;
+                const int h = st_tr ? o : m16, l = st_tr ? m16 : o;
+                const int wo = h * 16 + ((((l >> 1) ^ (h & 7)) << 1) | (l & 1));
+                const int ao = (m16 >> 2) * 64 + (m16 & 3) * 16 + (o ^ m16);
+                double2 bf[nk];
+                double af[ng][2];
+#pragma unroll
+                for (int j = 0; j < nk; ++j) bf[j] = A[j * 256 + ao];
+#pragma unroll
+                for (int i = 0; i < ng; ++i) { af[i][0] = W[i * 512 + wo]; af[i][1] = W[i * 512 + 256 + wo]; }
+#pragma unroll
+                for (int i = 0; i < ng; ++i)
+#pragma unroll
+                    for (int j = 0; j < nk; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i][0], bf[j].x, acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < ng; ++i)
+#pragma unroll
+                    for (int j = 0; j < nk; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i][1], bf[j].y, acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+    auto real = [&](int R) __attribute__((always_inline)) { return R == a.nb - 1 ? last : TB; };
+
+    int R0 = r0_beg, R1 = 0, sp = 0, buf = 0;
+    if (R0 < r0_end) fetch(R0, R1, sp, 0);
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    for (int step = 0; step < nsteps; ++step) {
-        const int buf = step & 1;
-        if (step + 1 < nsteps) fetch(step + 1);
-        const double *W = WS + buf * 16 * gstr;
-        const double *As = AS + buf * GCH * BS_STR;
-#pragma unroll
-        for (int kq = 0; kq < 4; ++kq) {
-            const int o = 4 * kq + (lane >> 4);
-            const double bf = As[(wave * 16 + (lane & 15)) * BS_STR + o];
-#pragma unroll
-            for (int i = 0; i < GT; ++i)
-                acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(W[o * gstr + i * 16 + (lane & 15)], bf, acc[i], 0, 0, 0);
-        }
-        if (step + 1 < nsteps) stash(buf ^ 1);
+    while (R0 < r0_end) {
+        const int nkq = (real(sa_u ? R1 : R0) + 3) / 4, nsp = (real(sa_u ? R0 : R1) + 1) / 2;
+        int n0 = R0, n1 = R1, ns = sp + 1;                     // the next step
+        if (ns >= nsp) { ns = 0; if (++n1 == a.nb) { n1 = 0; ++n0; } }
+        if (n0 < r0_end) fetch(n0, n1, ns, buf ^ 1);
+        typedef std::integral_constant<int, GM> G1;
+        typedef std::integral_constant<int, GM - 1> G2;
+        typedef std::integral_constant<int, KN> K1;
+        typedef std::integral_constant<int, KN - 1> K2;
+        if (gn == GM) { if (kn == KN) compute(G1{}, K1{}, buf, nkq); else compute(G1{}, K2{}, buf, nkq); }
+        else { if (kn == KN) compute(G2{}, K1{}, buf, nkq); else compute(G2{}, K2{}, buf, nkq); }
+        __builtin_amdgcn_s_waitcnt(0);     // the next step's slices have landed
         __syncthreads();
+        R0 = n0; R1 = n1; sp = ns; buf ^= 1;
     }
-    double *pt = a.part + (((long long)e * a.nsplit + rs) * a.nchunk + ch) * a.ngg * (GT * 16 * GCH) +
-                 (long long)gg * (GT * 16 * GCH);
+    double *pt = a.part + ((((long long)e * a.nsplit + rs) * a.nchunk + ch) * a.ngg + gg) * ((long long)GT * KT * 256);
 #pragma unroll
-    for (int i = 0; i < GT; ++i)
+    for (int i = 0; i < GM; ++i)
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-            pt[(i * 16 + Mfma<double>::row(lane, v)) * GCH + wave * 16 + (lane & 15)] = acc[i][v];
+        for (int j = 0; j < KN; ++j)
+            if (i < gn && j < kn)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    pt[((g_beg + i) * 16 + Mfma<double>::row(lane, v)) * (KT * 16) + (k_beg + j) * 16 + m16] = acc[i][j][v] * wgt;
 }
 
 // gbx[y][z][g][K] += sum over the entries of pair (y,z) (CSR order) and the panel splits of
 // the partial tiles
 __global__ void gbx_reduce_kernel(const double *__restrict__ part, double *__restrict__ gbx,
                                   const int *__restrict__ plist, const int *__restrict__ poff, int np, int nup,
-                                  int kp, int nchunk, int ngg, int gtr, int nsplit)
+                                  int kp, int nchunk, int ngg, int gtr, int kw, int nsplit)
 {
     const long long per = (long long)nup * kp;
     const long long total = (long long)np * per;
-    const long long tile = (long long)gtr * GCH;
+    const long long tile = (long long)gtr * kw;   // gamma rows x K columns of a partial tile
     for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < total;
          idx += (long long)gridDim.x * blockDim.x) {
         const int pi = (int)(idx / per);
         const int rem = (int)(idx % per);
         const int g = rem / kp, K = rem % kp;
-        const int ch = K / GCH, kl = K % GCH, gg = g / gtr, gl = g % gtr;
+        const int ch = K / kw, kl = K % kw, gg = g / gtr, gl = g % gtr;
         double s = 0.0;
         for (int e = poff[pi]; e < poff[pi + 1]; ++e)
             for (int rs = 0; rs < nsplit; ++rs)
-                s += part[((((long long)e * nsplit + rs) * nchunk + ch) * ngg + gg) * tile + (long long)gl * GCH + kl];
+                s += part[((((long long)e * nsplit + rs) * nchunk + ch) * ngg + gg) * tile + (long long)gl * kw + kl];
         gbx[(long long)plist[pi] * per + rem] += s;
     }
 }
@@ -851,19 +856,29 @@ static int launch_gax(const GemmArgs &a, long long grid, hipStream_t s)
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
-template <int GT>
+template <int GM, int KN>
 static int launch_gbx(const GemmArgs &a, long long grid, hipStream_t s)
 {
     static bool attr_set = false;
-    const size_t lds_bytes = sizeof(double) * (2 * 16 * (GT * 16 + 1) + 2 * GCH * BS_STR);
+    constexpr int most = sizeof(double) * 2 * 512 * GBX_TILES;
     if (!attr_set) {
-        if (hipFuncSetAttribute((const void *)gbx_kernel<GT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds_bytes) != hipSuccess)
+        if (hipFuncSetAttribute((const void *)gbx_kernel<GM, KN>, hipFuncAttributeMaxDynamicSharedMemorySize, most) != hipSuccess)
             return 2;
         attr_set = true;
     }
-    gbx_kernel<GT><<<(unsigned)grid, GTHR, lds_bytes, s>>>(a);
+    gbx_kernel<GM, KN><<<(unsigned)grid, GTHR, sizeof(double) * 2 * 512 * (a.gt + a.kt), s>>>(a);
     return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+template <int GM>
+static int launch_gbx_k(const GemmArgs &a, long long grid, hipStream_t s)
+{
+    switch ((a.kt + 1) / 2) {
+    case 1: return launch_gbx<GM, 1>(a, grid, s);
+    case 2: return launch_gbx<GM, 2>(a, grid, s);
+    case 3: return launch_gbx<GM, 3>(a, grid, s);
+    default: return launch_gbx<GM, 4>(a, grid, s);
+    }
 }
 
 extern "C" {
@@ -955,58 +970,48 @@ int ccx_hip_gax(const double *wbar, const double *bx, double *gax, const int *tu
     return rc;
 }
 
-void ccx_hip_gbx_geometry(int nup, int kp, int *nchunk, int *ngg, int *gtr)
+// Tiles of a gbx work group: K chunks of at most 8 tiles and gamma groups of at most GBX_TILES - 8,
+// each as even as the count allows, so that the two buffers of both fit the 160 KB of LDS.
+static void gbx_geometry(int nup, int kp, int *nchunk, int *ngg, int *gt, int *kt)
 {
-    const int nb = nup / TB;
-    *ngg = (nb + 13) / 14;                // gamma groups of at most 14 tiles
-    *gtr = 16 * ((nb + *ngg - 1) / *ngg); // rows of a partial tile
-    *nchunk = (kp + GCH - 1) / GCH;
+    const int nb = nup / TB, nk = (kp + 15) / 16;
+    *nchunk = (nk + 7) / 8;
+    *kt = (nk + *nchunk - 1) / *nchunk;
+    *ngg = (nb + GBX_TILES - 9) / (GBX_TILES - 8);
+    *gt = (nb + *ngg - 1) / *ngg;
 }
 
 size_t ccx_hip_gbx_part_doubles(int nup, int kp, int nent, int nsplit)
 {
-    int nchunk, ngg, gtr;
-    ccx_hip_gbx_geometry(nup, kp, &nchunk, &ngg, &gtr);
-    return (size_t)nent * nsplit * nchunk * ngg * gtr * GCH;
+    int nchunk, ngg, gt, kt;
+    gbx_geometry(nup, kp, &nchunk, &ngg, &gt, &kt);
+    return (size_t)nent * nsplit * nchunk * ngg * gt * kt * 256;
 }
 
 int ccx_hip_gbx(const double *wbar, const double *axr, const double *axc, double *gbx, double *part,
                 const int *tuples, int t0, const int *plist, const int *poff, const int *ent, int npair, int nent,
-                int nsplit, int no, int nup, int kp, void *stream)
+                int nsplit, int no, int nu, int nup, int kp, void *stream)
 {
-    const int nb = nup / TB;
-    int nchunk, ngg, gtr;
-    ccx_hip_gbx_geometry(nup, kp, &nchunk, &ngg, &gtr);
-    const int gt = gtr / 16;
     if (npair == 0 || nent == 0) return 0;
     GemmArgs a = {};
+    gbx_geometry(nup, kp, &a.nchunk, &a.ngg, &a.gt, &a.kt);
     a.wbar = wbar; a.axr = axr; a.axc = axc; a.gbx = gbx; a.part = part; a.tuples = tuples; a.t0 = t0;
     a.ulist = plist; a.uoff = poff; a.ent = ent;
-    a.no = no; a.nup = nup; a.nb = nb; a.kp = kp; a.nchunk = nchunk; a.gt = gt; a.ngg = ngg; a.nsplit = nsplit;
-    const long long grid = (long long)nent * nsplit * nchunk * ngg;
+    a.no = no; a.nu = nu; a.nup = nup; a.nb = nup / TB; a.kp = kp; a.nsplit = nsplit;
+    const long long grid = (long long)nent * nsplit * a.nchunk * a.ngg;
     hipStream_t s = (hipStream_t)stream;
     int rc;
-    switch (gt) {
-    case 1: rc = launch_gbx<1>(a, grid, s); break;
-    case 2: rc = launch_gbx<2>(a, grid, s); break;
-    case 3: rc = launch_gbx<3>(a, grid, s); break;
-    case 4: rc = launch_gbx<4>(a, grid, s); break;
-    case 5: rc = launch_gbx<5>(a, grid, s); break;
-    case 6: rc = launch_gbx<6>(a, grid, s); break;
-    case 7: rc = launch_gbx<7>(a, grid, s); break;
-    case 8: rc = launch_gbx<8>(a, grid, s); break;
-    case 9: rc = launch_gbx<9>(a, grid, s); break;
-    case 10: rc = launch_gbx<10>(a, grid, s); break;
-    case 11: rc = launch_gbx<11>(a, grid, s); break;
-    case 12: rc = launch_gbx<12>(a, grid, s); break;
-    case 13: rc = launch_gbx<13>(a, grid, s); break;
-    default: rc = launch_gbx<14>(a, grid, s); break;
+    switch ((a.gt + 3) / 4) {
+    case 1: rc = launch_gbx_k<1>(a, grid, s); break;
+    case 2: rc = launch_gbx_k<2>(a, grid, s); break;
+    default: rc = launch_gbx_k<3>(a, grid, s); break;   // gt <= GBX_TILES - 8 = 11
     }
     if (rc != 0) return rc;
     const long long total = (long long)npair * nup * kp;
     long long g2 = (total + 255) / 256;
     if (g2 > 65536) g2 = 65536;
-    gbx_reduce_kernel<<<(unsigned)g2, 256, 0, s>>>(part, gbx, plist, poff, npair, nup, kp, nchunk, ngg, gtr, nsplit);
+    gbx_reduce_kernel<<<(unsigned)g2, 256, 0, s>>>(part, gbx, plist, poff, npair, nup, kp, a.nchunk, a.ngg, a.gt * 16,
+                                                   a.kt * 16, nsplit);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 

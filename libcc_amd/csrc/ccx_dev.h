@@ -73,7 +73,7 @@ int ccx_hip_gax(const double *wbar, const double *bx, double *gax, const int *tu
 size_t ccx_hip_gbx_part_doubles(int nup, int kp, int nent, int nsplit);
 int ccx_hip_gbx(const double *wbar, const double *axr, const double *axc, double *gbx, double *part,
                 const int *tuples, int t0, const int *plist, const int *poff, const int *ent, int npair, int nent,
-                int nsplit, int no, int nup, int kp, void *stream);
+                int nsplit, int no, int nu, int nup, int kp, void *stream);
 int ccx_hip_dvoe_reduce(const double *slots, double *dvoep, const int *plist, const int *poff, const int *ent,
                         int np, int no, int nup, void *stream);
 int ccx_hip_unpack_grad(const double *gax, const double *gbx, const double *dvoep, const double *v1, double *dvvvo,

@@ -151,6 +151,19 @@ def test_autograd_function_on_device_tensors():
         np.testing.assert_allclose(gk.cpu().numpy(), 3.0 * want[k], rtol=1e-13, atol=1e-300)
 
 
+@pytest.mark.parametrize("no,nu", [(2, 17), (2, 65), (2, 126), (2, 142), (2, 175), (2, 185)], ids=lambda v: str(v))
+def test_back_contraction_tile_edges(no, nu):
+    """Gamma tiles 2, 5, 8, 9, 11 and 12 (two groups of 6), K tiles 2, 5, 8, 9 (two chunks of 5 and 4),
+    12 (two of 6); last blocks of 1, 1, 14, 14, 15 and 9 indices, so slices and contraction steps of
+    padding are left out on every axis."""
+    inp = synth.make_inputs(no, nu, 300 + nu)
+    print(f"gradient no={no} nu={nu}", flush=True)
+    want = dense.grad_tuplewise(inp)
+    got = _grad(inp)
+    for k in KEYS:
+        _close(got[k], want[k], 1e-11)
+
+
 @pytest.mark.parametrize("form", ["fp32", "bf16x3"])
 def test_autograd_function_reduced_form(form):
     """The same Function with W recomputed in a reduced form: both the 7-argument call and
