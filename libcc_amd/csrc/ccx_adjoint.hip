@@ -443,6 +443,7 @@ constexpr int GBPW = 2;                   // gax: rows b per wave
 constexpr int GCH = 128;                  // K columns per work group (8 MFMA tiles)
 constexpr int GCT = GCH / 16;
 constexpr int BS_STR = 17;                // padded row of the staged BX slices
+typedef double d2 __attribute__((ext_vector_type(2)));
 constexpr int GBX_TILES = 19;             // gbx: gamma and K tiles of a work group (two 4 KB buffers each)
 }  // namespace
 
@@ -603,11 +604,13 @@ __global__ void __launch_bounds__(GTHR, 1) gax_kernel(GemmArgs a)
 template <int GM, int KN>   // most gamma tiles and K tiles of a wave
 __global__ void __launch_bounds__(GTHR, 1) gbx_kernel(GemmArgs a)
 {
-    extern __shared__ double lds[];
+    // Two arrays, and steps in pairs so that every access names one of them: the compiler then knows
+    // that the direct loads into one do not alias the reads of the other.  In one array it puts a
+    // wait for all outstanding loads before the first read of each step, and the loads that were
+    // to run under the step's MFMAs are waited for first (5.26 ms at no=8, nu=120).
+    __shared__ __align__(16) double buf0[GBX_TILES * 512], buf1[GBX_TILES * 512];
     typedef __attribute__((address_space(3))) void lds_void;
     typedef const __attribute__((address_space(1))) void g_void;
-    const int GT = a.gt, KT = a.kt;
-    const int bufd = (GT + KT) * 512;     // doubles of a buffer: [GT][slice 2][256], then [4 KT][64][2]
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int u = blockIdx.x;
@@ -616,7 +619,10 @@ __global__ void __launch_bounds__(GTHR, 1) gbx_kernel(GemmArgs a)
     const int rs = u % a.nsplit; u /= a.nsplit;
     const int e = u;                      // entry (CSR position)
     const int r0_beg = rs * a.nb / a.nsplit, r0_end = (rs + 1) * a.nb / a.nsplit;
-    const int G0 = gg * GT, kb0 = ch * KT * 4;
+    const int nkt = (a.kp + 15) / 16;
+    const int G0 = a.nb * gg / a.ngg, GT = a.nb * (gg + 1) / a.ngg - G0;            // gt or gt - 1 tiles
+    const int k0 = nkt * ch / a.nchunk, KT = nkt * (ch + 1) / a.nchunk - k0, kb0 = k0 * 4;
+    // a buffer: Wbar [GT][slice 2][256], then AX [4 KT][64][2]
     const int tl = __builtin_amdgcn_readfirstlane(a.ent[2 * e]), sg = __builtin_amdgcn_readfirstlane(a.ent[2 * e + 1]);
     const int4 tp = reinterpret_cast<const int4 *>(a.tuples)[a.t0 + tl];
     const Sigma S = SIG[sg & 7];
@@ -637,15 +643,14 @@ __global__ void __launch_bounds__(GTHR, 1) gbx_kernel(GemmArgs a)
     // per-lane source offsets of the direct loads (rows h of 128 B, units permuted by h & 7)
     const int h8 = lane >> 3, un = 2 * ((lane & 7) ^ (h8 & 7));
     const int w_hstr = sa == 0 ? 16 : 256, w_sstr = sa == 0 ? 256 : 16;
-    auto fetch = [&](int R0, int R1, int sp, int buf) __attribute__((always_inline)) {
-        double *W = lds + buf * bufd, *A = W + GT * 512;
+    auto fetch = [&](int R0, int R1, int sp, double *W) __attribute__((always_inline)) {
+        double *A = W + GT * 512;
         const int b0 = S.u == 0 ? R0 : S.v == 0 ? R1 : G0, b1 = S.u == 1 ? R0 : S.v == 1 ? R1 : G0,
                   b2 = S.u == 2 ? R0 : S.v == 2 ? R1 : G0;
         const double *wb = cube + (((long long)b0 * a.nb + b1) * a.nb + b2) * 4096 + 2 * sp * w_sstr + h8 * w_hstr + un;
 #pragma unroll 1
         for (int c = wave; c < GT * 4; c += GTHR / 64) {       // chunk: tile, slice, half of the rows
-            const int t = c >> 2, tc = G0 + t < a.nb ? t : a.nb - 1 - G0;   // tiles past the last are not used
-            __builtin_amdgcn_global_load_lds((g_void *)(wb + tc * gstep + ((c >> 1) & 1) * w_sstr + (c & 1) * 8 * w_hstr),
+            __builtin_amdgcn_global_load_lds((g_void *)(wb + (c >> 2) * gstep + ((c >> 1) & 1) * w_sstr + (c & 1) * 8 * w_hstr),
                                              (lds_void *)(W + c * 128), 16, 0, 0);
         }
         const double *ap = ax + ((long long)R0 * a.nb + R1) * (256LL * a.kp) + (long long)sp * (32LL * a.kp);
@@ -666,22 +671,23 @@ __global__ void __launch_bounds__(GTHR, 1) gbx_kernel(GemmArgs a)
     const int m16 = lane & 15, q4 = lane >> 4;
 
     // one step for a wave of ng gamma and nk K tiles (compile time: no MFMA behind a branch)
-    auto compute = [&](auto NG, auto NK, int buf, int nkq) __attribute__((always_inline)) {
+    auto compute = [&](auto NG, auto NK, const double *lds, int nkq) __attribute__((always_inline)) {
         constexpr int ng = decltype(NG)::value, nk = decltype(NK)::value;
         if constexpr (ng > 0 && nk > 0) {
-            const double *W = lds + buf * bufd + g_beg * 512;
-            const double2 *A = reinterpret_cast<const double2 *>(lds + buf * bufd + GT * 512) + k_beg * 256;
             for (int kq = 0; kq < nkq; ++kq) {
                 const int o = 4 * kq + q4;
                 const int h = st_tr ? o : m16, l = st_tr ? m16 : o;
-                const int wo = h * 16 + ((((l >> 1) ^ (h & 7)) << 1) | (l & 1));
-                const int ao = (m16 >> 2) * 64 + (m16 & 3) * 16 + (o ^ m16);
-                double2 bf[nk];
+                int wo = g_beg * 512 + h * 16 + ((((l >> 1) ^ (h & 7)) << 1) | (l & 1));
+                int ao = (GT + k_beg) * 512 + 2 * ((m16 >> 2) * 64 + (m16 & 3) * 16 + (o ^ m16));
+                // The indices in one piece: the compiler follows a short chain of pointer additions
+                // only from the array to a read, and would split these sums into a long one.
+                asm("" : "+v"(wo), "+v"(ao));
+                d2 bf[nk];
                 double af[ng][2];
 #pragma unroll
-                for (int j = 0; j < nk; ++j) bf[j] = A[j * 256 + ao];
+                for (int j = 0; j < nk; ++j) bf[j] = *reinterpret_cast<const d2 *>(&lds[ao + j * 512]);
 #pragma unroll
-                for (int i = 0; i < ng; ++i) { af[i][0] = W[i * 512 + wo]; af[i][1] = W[i * 512 + 256 + wo]; }
+                for (int i = 0; i < ng; ++i) { af[i][0] = lds[wo + i * 512]; af[i][1] = lds[wo + i * 512 + 256]; }
 #pragma unroll
                 for (int i = 0; i < ng; ++i)
 #pragma unroll
@@ -697,26 +703,28 @@ __global__ void __launch_bounds__(GTHR, 1) gbx_kernel(GemmArgs a)
     };
     auto real = [&](int R) __attribute__((always_inline)) { return R == a.nb - 1 ? last : TB; };
 
-    int R0 = r0_beg, R1 = 0, sp = 0, buf = 0;
-    if (R0 < r0_end) fetch(R0, R1, sp, 0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    while (R0 < r0_end) {
+    int R0 = r0_beg, R1 = 0, sp = 0;
+    auto step = [&](double *next, const double *cur) __attribute__((always_inline)) {
         const int nkq = (real(sa_u ? R1 : R0) + 3) / 4, nsp = (real(sa_u ? R0 : R1) + 1) / 2;
-        int n0 = R0, n1 = R1, ns = sp + 1;                     // the next step
-        if (ns >= nsp) { ns = 0; if (++n1 == a.nb) { n1 = 0; ++n0; } }
-        if (n0 < r0_end) fetch(n0, n1, ns, buf ^ 1);
+        if (++sp >= nsp) { sp = 0; if (++R1 == a.nb) { R1 = 0; ++R0; } }   // the next step
+        if (R0 < r0_end) fetch(R0, R1, sp, next);
         typedef std::integral_constant<int, GM> G1;
         typedef std::integral_constant<int, GM - 1> G2;
         typedef std::integral_constant<int, KN> K1;
         typedef std::integral_constant<int, KN - 1> K2;
-        if (gn == GM) { if (kn == KN) compute(G1{}, K1{}, buf, nkq); else compute(G1{}, K2{}, buf, nkq); }
-        else { if (kn == KN) compute(G2{}, K1{}, buf, nkq); else compute(G2{}, K2{}, buf, nkq); }
+        if (gn == GM) { if (kn == KN) compute(G1{}, K1{}, cur, nkq); else compute(G1{}, K2{}, cur, nkq); }
+        else { if (kn == KN) compute(G2{}, K1{}, cur, nkq); else compute(G2{}, K2{}, cur, nkq); }
         __builtin_amdgcn_s_waitcnt(0);     // the next step's slices have landed
         __syncthreads();
-        R0 = n0; R1 = n1; sp = ns; buf ^= 1;
+    };
+    if (R0 < r0_end) fetch(R0, R1, sp, buf0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    while (R0 < r0_end) {
+        step(buf1, buf0);
+        if (R0 < r0_end) step(buf0, buf1);
     }
-    double *pt = a.part + ((((long long)e * a.nsplit + rs) * a.nchunk + ch) * a.ngg + gg) * ((long long)GT * KT * 256);
+    double *pt = a.part + ((((long long)e * a.nsplit + rs) * a.nchunk + ch) * a.ngg + gg) * ((long long)a.gt * a.kt * 256);
 #pragma unroll
     for (int i = 0; i < GM; ++i)
 #pragma unroll
@@ -724,7 +732,7 @@ __global__ void __launch_bounds__(GTHR, 1) gbx_kernel(GemmArgs a)
             if (i < gn && j < kn)
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    pt[((g_beg + i) * 16 + Mfma<double>::row(lane, v)) * (KT * 16) + (k_beg + j) * 16 + m16] = acc[i][j][v] * wgt;
+                    pt[((g_beg + i) * 16 + Mfma<double>::row(lane, v)) * (a.kt * 16) + (k_beg + j) * 16 + m16] = acc[i][j][v] * wgt;
 }
 
 // gbx[y][z][g][K] += sum over the entries of pair (y,z) (CSR order) and the panel splits of
@@ -741,7 +749,10 @@ __global__ void gbx_reduce_kernel(const double *__restrict__ part, double *__res
         const int pi = (int)(idx / per);
         const int rem = (int)(idx % per);
         const int g = rem / kp, K = rem % kp;
-        const int ch = K / kw, kl = K % kw, gg = g / gtr, gl = g % gtr;
+        // chunk and group of the K and the gamma tile: the last boundary at or before it (gbx_kernel)
+        const int kt = K >> 4, gt = g >> 4, nb = nup >> 4, nkt = (kp + 15) / 16;
+        const int ch = ((kt + 1) * nchunk - 1) / nkt, gg = ((gt + 1) * ngg - 1) / nb;
+        const int kl = K - (nkt * ch / nchunk) * 16, gl = g - (nb * gg / ngg) * 16;
         double s = 0.0;
         for (int e = poff[pi]; e < poff[pi + 1]; ++e)
             for (int rs = 0; rs < nsplit; ++rs)
@@ -859,14 +870,7 @@ static int launch_gax(const GemmArgs &a, long long grid, hipStream_t s)
 template <int GM, int KN>
 static int launch_gbx(const GemmArgs &a, long long grid, hipStream_t s)
 {
-    static bool attr_set = false;
-    constexpr int most = sizeof(double) * 2 * 512 * GBX_TILES;
-    if (!attr_set) {
-        if (hipFuncSetAttribute((const void *)gbx_kernel<GM, KN>, hipFuncAttributeMaxDynamicSharedMemorySize, most) != hipSuccess)
-            return 2;
-        attr_set = true;
-    }
-    gbx_kernel<GM, KN><<<(unsigned)grid, GTHR, sizeof(double) * 2 * 512 * (a.gt + a.kt), s>>>(a);
+    gbx_kernel<GM, KN><<<(unsigned)grid, GTHR, 0, s>>>(a);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 
@@ -971,7 +975,7 @@ int ccx_hip_gax(const double *wbar, const double *bx, double *gax, const int *tu
 }
 
 // Tiles of a gbx work group: K chunks of at most 8 tiles and gamma groups of at most GBX_TILES - 8,
-// each as even as the count allows, so that the two buffers of both fit the 160 KB of LDS.
+// as even as the counts allow (gt, kt: the largest), so that the two buffers of both fit the 160 KB of LDS.
 static void gbx_geometry(int nup, int kp, int *nchunk, int *ngg, int *gt, int *kt)
 {
     const int nb = nup / TB, nk = (kp + 15) / 16;
