@@ -390,13 +390,15 @@ __global__ void __launch_bounds__(NTHR, 1) adj_item_kernel(AdjArgs ga)
             f4 acc[6][BPW];
             if constexpr (FK == 2) {
                 f4 acc1[1][BPW];   // unused: the BF16 x 3 form has one accumulator
+                // the epilogue's LDS leaves no room for BX buffers of their own
+                i32x4 *b0 = reinterpret_cast<i32x4 *>(lds), *b1 = b0 + split_bx_units<2>();
                 static_assert(!pair_modes(2), "the forward kernel's modes");
-                if (tkind == 2) item_w_split<M_IJJ, 2>(g, lds, it, acc, acc1, wave, lane);
-                else if (tkind == 3) item_w_split<M_IIJ, 2>(g, lds, it, acc, acc1, wave, lane);
-                else if (mult == 1) item_w_split<M_FULL, 2>(g, lds, it, acc, acc1, wave, lane);
-                else if (mult == 6) item_w_split<M_AAA, 2>(g, lds, it, acc, acc1, wave, lane);
-                else if (it.blk[0] == it.blk[1]) item_w_split<M_AAC, 2>(g, lds, it, acc, acc1, wave, lane);
-                else item_w_split<M_ACC, 2>(g, lds, it, acc, acc1, wave, lane);
+                if (tkind == 2) item_w_split<M_IJJ, 2>(g, lds, it, acc, acc1, wave, lane, b0, b1);
+                else if (tkind == 3) item_w_split<M_IIJ, 2>(g, lds, it, acc, acc1, wave, lane, b0, b1);
+                else if (mult == 1) item_w_split<M_FULL, 2>(g, lds, it, acc, acc1, wave, lane, b0, b1);
+                else if (mult == 6) item_w_split<M_AAA, 2>(g, lds, it, acc, acc1, wave, lane, b0, b1);
+                else if (it.blk[0] == it.blk[1]) item_w_split<M_AAC, 2>(g, lds, it, acc, acc1, wave, lane, b0, b1);
+                else item_w_split<M_ACC, 2>(g, lds, it, acc, acc1, wave, lane, b0, b1);
             } else {
                 static_assert(!pair_modes(1), "the forward kernel's modes");
                 if (tkind == 2) item_w_f32v<M_IJJ>(g, lds, it, acc, wave, lane);

@@ -706,18 +706,26 @@ __device__ __forceinline__ void pin_accumulators(f4 (&acc)[N][BPW])
 // step walks the BX slices from the last to the first, reads each from LDS just before its
 // products (so one BX slice is live at a time) and issues the products with every AX slice
 // whose level fits, for every term and batch; consecutive MFMAs go to different accumulators.
+// units of 16 B of one BX buffer (six operands at most)
+template <int FK> constexpr int split_bx_units() { return 6 * SplitCfg<FK>::NS * SplitCfg<FK>::F16 * 64; }
+
 template <int PHASE, int MODE, int FK>
 __device__ __forceinline__ void run_phase_split(const TriplesArgs &g, const ItemCtx &it, f4 (&g0)[6][BPW],
-                                                f4 (&g1)[SplitCfg<FK>::TWO_ACC ? 6 : 1][BPW], i32x4 *lbx,
-                                                int wave, int lane)
+                                                f4 (&g1)[SplitCfg<FK>::TWO_ACC ? 6 : 1][BPW], i32x4 *lb0,
+                                                i32x4 *lb1, int wave, int lane)
 {
+    // BX staging: block kb in lb0 (even) or lb1 (odd).  Where they are two LDS arrays of their own the
+    // compiler knows that the direct loads into one do not alias the reads of the other; in one
+    // array it waited for every outstanding load (the next block's BX and the next AX fragments,
+    // just issued) before the first read of each K block: 175 ms at no=16, nu=181 in the BF16x3 form.
     typedef SplitCfg<FK> CF;
     constexpr int SM = slot_mask(PHASE, MODE), XM = bx_mask(PHASE, MODE);
     constexpr int NSL = __builtin_popcount(SM), NBX = __builtin_popcount(XM);
     constexpr int NS = CF::NS, F16 = CF::F16;
     constexpr int CH = NS * F16;               // 16-byte chunks per lane per fragment set
     constexpr int NCH = NBX * CH;              // BX chunks per K block
-    static_assert(2 * NCH * 1024 + 2 * NBX * 256 <= (int)(sizeof(double) * LDS_DOUBLES), "BX staging fits LDS");
+    static_assert(NCH * 64 <= split_bx_units<FK>() &&
+                  2 * split_bx_units<FK>() * 16 + 2 * NBX * 256 <= (int)(sizeof(double) * LDS_DOUBLES), "BX staging fits LDS");
     const int A = it.blk[0], B = it.blk[1], C = it.blk[2];
     int r0[2], r1[2];
     bool col[2];
@@ -746,7 +754,7 @@ __device__ __forceinline__ void run_phase_split(const TriplesArgs &g, const Item
         xq[q] = (g16 *)g.bx_s + pg * ((long long)nkb * CH * 64);
         if constexpr (CF::MX) xe[q] = (g4 *)g.bx_e + pg * ((long long)nkb * 64);
     }
-    int *lbe = reinterpret_cast<int *>(lbx + 2 * NCH * 64);   // BX block exponents, [buf][rank][lane]
+    int *lbe = reinterpret_cast<int *>(lb1 + NCH * 64);   // BX block exponents, [buf][rank][lane]
 
     // BX staging: chunk c = rank * CH + (slice * F16 + f) of K block kb goes straight from global
     // memory into LDS buffer buf (global_load_lds_dwordx4: lane l's 16 bytes land at the chunk's
@@ -771,7 +779,7 @@ __device__ __forceinline__ void run_phase_split(const TriplesArgs &g, const Item
             const int c = wave + NWAVE * r;
             if (c < NCH)
                 __builtin_amdgcn_global_load_lds((g_void *)(bx_src(c / CH) + ((long long)kb * CH + c % CH) * 64 + lane),
-                                                 (lds_void *)(lbx + (buf * NCH + c) * 64), 16, 0, 0);
+                                                 (lds_void *)((buf ? lb1 : lb0) + c * 64), 16, 0, 0);
         }
         if constexpr (CF::MX) {
             if (wave < NBX) {
@@ -834,7 +842,7 @@ __device__ __forceinline__ void run_phase_split(const TriplesArgs &g, const Item
             static_for<ST.n>([&](auto N) __attribute__((always_inline)) {
                 constexpr int n = decltype(N)::value;
                 constexpr int rank = __builtin_popcount(XM & ((1 << ST.b[n]) - 1));
-                bs[n] = split_frag_lds<FK>(lbx, (buf * NCH + rank * CH + sj * F16) * 64 + lane);
+                bs[n] = split_frag_lds<FK>(buf ? lb1 : lb0, (rank * CH + sj * F16) * 64 + lane);
             });
             static_for<NS - sj>([&](auto SI) __attribute__((always_inline)) {
                 constexpr int si = NS - 1 - sj - decltype(SI)::value;   // AX slice, highest level first
@@ -921,7 +929,7 @@ __device__ __forceinline__ void run_phase_split(const TriplesArgs &g, const Item
 template <int MODE, int FK>
 __device__ __forceinline__ void item_w_split(const TriplesArgs &g, double *lds, const ItemCtx &it,
                                              f4 (&g0)[6][BPW], f4 (&g1)[SplitCfg<FK>::TWO_ACC ? 6 : 1][BPW],
-                                             int wave, int lane)
+                                             int wave, int lane, i32x4 *lb0, i32x4 *lb1)
 {
     constexpr bool TWO = SplitCfg<FK>::TWO_ACC;
 #pragma unroll
@@ -931,12 +939,11 @@ __device__ __forceinline__ void item_w_split(const TriplesArgs &g, double *lds, 
             g0[p][bb] = f4{0, 0, 0, 0};
             if constexpr (TWO) g1[p][bb] = f4{0, 0, 0, 0};
         }
-    i32x4 *lbx = reinterpret_cast<i32x4 *>(lds);
-    run_phase_split<0, MODE, FK>(g, it, g0, g1, lbx, wave, lane);
+    run_phase_split<0, MODE, FK>(g, it, g0, g1, lb0, lb1, wave, lane);
     transpose_lb_to_l<MODE, float>(lds, g0, wave, lane);
     if constexpr (TWO) transpose_lb_to_l<MODE, float>(lds, g1, wave, lane);
-    run_phase_split<1, MODE, FK>(g, it, g0, g1, lbx, wave, lane);
-    run_phase_split<2, MODE, FK>(g, it, g0, g1, lbx, wave, lane);
+    run_phase_split<1, MODE, FK>(g, it, g0, g1, lb0, lb1, wave, lane);
+    run_phase_split<2, MODE, FK>(g, it, g0, g1, lb0, lb1, wave, lane);
     complete_orderings<MODE, float>(lds, g0, wave, lane);
     if constexpr (TWO) complete_orderings<MODE, float>(lds, g1, wave, lane);
 }

@@ -485,6 +485,11 @@ __global__ void __launch_bounds__(NTHR, 1) triples_kernel(TriplesArgs g)
     extern __shared__ double lds[];
     __shared__ double red[NWAVE][112];
     __shared__ long long next_item;
+    // BX buffers of the split sweeps (run_phase_split).  The FP8 form's, 99 KB, do not fit beside the
+    // transposition cubes and share their array.
+    constexpr bool OWN_BX = FK == 2 || FK == 4;
+    constexpr int BXU = FK >= 2 ? split_bx_units<FK >= 2 ? FK : 2>() : 1;
+    __shared__ i32x4 bx0[OWN_BX ? BXU : 1], bx1[OWN_BX ? BXU : 1];
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -516,7 +521,10 @@ __global__ void __launch_bounds__(NTHR, 1) triples_kernel(TriplesArgs g)
         f4 acc1[FK == 4 ? 6 : 1][BPW];   // two-accumulator split form: the levels above 0
         auto sweeps = [&](auto M) __attribute__((always_inline)) {
             constexpr int MODE = decltype(M)::value;
-            if constexpr (FK >= 2) item_w_split<MODE, FK>(g, lds, it, acc, acc1, wave, lane);
+            if constexpr (OWN_BX) item_w_split<MODE, FK>(g, lds, it, acc, acc1, wave, lane, bx0, bx1);
+            else if constexpr (FK >= 2)
+                item_w_split<MODE, FK>(g, lds, it, acc, acc1, wave, lane, reinterpret_cast<i32x4 *>(lds),
+                                       reinterpret_cast<i32x4 *>(lds) + BXU);
             else if constexpr (FK == 1) item_w_f32v<MODE>(g, lds, it, acc, wave, lane);
             else item_w<MODE, T>(g, lds, it, acc, wave, lane);
         };
