@@ -746,51 +746,55 @@ __device__ __forceinline__ void run_phase_split(const TriplesArgs &g, const Item
         ap[s] = (g16 *)(col[o] ? g.axc_s : g.axr_s) + (panel * 16 + 2 * wave) * ((long long)nkb * CH * 64);
         if constexpr (CF::MX) aep[s] = (g4 *)(col[o] ? g.axc_e : g.axr_e) + (panel * 16 + 2 * wave) * ((long long)nkb * 64);
     }
-    g16 *xq[6];
-    g4 *xe[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        const long long pg = (long long)(it.ys[q] * g.no + it.zs[q]) * g.nb + G;
-        xq[q] = (g16 *)g.bx_s + pg * ((long long)nkb * CH * 64);
-        if constexpr (CF::MX) xe[q] = (g4 *)g.bx_e + pg * ((long long)nkb * 64);
-    }
     int *lbe = reinterpret_cast<int *>(lb1 + NCH * 64);   // BX block exponents, [buf][rank][lane]
 
     // BX staging: chunk c = rank * CH + (slice * F16 + f) of K block kb goes straight from global
-    // memory into LDS buffer buf (global_load_lds_dwordx4: lane l's 16 bytes land at the chunk's
+    // memory into LDS buffer buf (buffer_load_dwordx4 to LDS: lane l's 16 bytes land at the chunk's
     // base + 16 l), loaded by wave c % NWAVE (wave w takes chunks w, w + NWAVE, ...); the
-    // exponent word of rank q by wave q.  No registers hold the staged data.  The rank of a chunk
-    // is wave-uniform, so its panel pointer is a uniform select.  Completion is waited for
-    // (vmcnt 0) before the barrier that publishes the buffer.
+    // exponent word of rank q by wave q.  No registers hold the staged data.  Completion is waited for
+    // (vmcnt) before the barrier that publishes the buffer.
     typedef __attribute__((address_space(3))) void lds_void;
-    typedef const __attribute__((address_space(1))) void g_void;
     constexpr int NBR = (NCH + NWAVE - 1) / NWAVE;
-    auto bx_src = [&](int rank) __attribute__((always_inline)) {
-        g16 *p = xq[nth_bit(XM, 0)];
+    // panel (y, z, G) of the BX operand of a rank, by selects on the wave-uniform rank.  (Selecting
+    // among an array of pointers in the loop became a scratch load with a wait for everything
+    // outstanding, per chunk and block.)
+    auto bx_panel = [&](int rank) __attribute__((always_inline)) {
+        int pg = 0;
         static_for<NBX>([&](auto R) __attribute__((always_inline)) {
-            constexpr int r = decltype(R)::value;
-            if (rank == r) p = xq[nth_bit(XM, r)];
+            constexpr int r = decltype(R)::value, q = nth_bit(XM, r);
+            const int v = (it.ys[q] * g.no + it.zs[q]) * g.nb + G;
+            pg = rank == r ? v : pg;
         });
-        return p;
+        return pg;
     };
+    const char *bsrc[NBR];       // this wave's chunks, at K block 0
+#pragma unroll
+    for (int r = 0; r < NBR; ++r) {
+        const int c = wave + NWAVE * r;
+        bsrc[r] = static_cast<const char *>(g.bx_s) + ((long long)bx_panel(c / CH) * nkb * CH + c % CH) * 1024;
+    }
+    const char *esrc = reinterpret_cast<const char *>(g.bx_e);
+    if constexpr (CF::MX) esrc += (long long)bx_panel(wave) * (nkb * 256);
+    // Buffer loads, not global_load_lds: that is a FLAT instruction to the compiler, after which it makes
+    // the next use of any load wait for all of them.  A chunk's resource spans its panel.
+    const int lane16 = lane * 16, lane4 = lane * 4;
+    auto rsrc = [&](const void *p, int bytes) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00027000);
+    };
+    const int panel_bytes = nkb * CH * 1024;
     auto bx_load = [&](int kb, int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < NBR; ++r) {
             const int c = wave + NWAVE * r;
             if (c < NCH)
-                __builtin_amdgcn_global_load_lds((g_void *)(bx_src(c / CH) + ((long long)kb * CH + c % CH) * 64 + lane),
-                                                 (lds_void *)((buf ? lb1 : lb0) + c * 64), 16, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rsrc(bsrc[r], panel_bytes - (c % CH) * 1024), (lds_void *)((buf ? lb1 : lb0) + c * 64), 16, lane16,
+                    kb * (CH * 1024), 0, 0);
         }
         if constexpr (CF::MX) {
-            if (wave < NBX) {
-                g4 *e = xe[nth_bit(XM, 0)];
-                static_for<NBX>([&](auto R) __attribute__((always_inline)) {
-                    constexpr int r = decltype(R)::value;
-                    if (wave == r) e = xe[nth_bit(XM, r)];
-                });
-                __builtin_amdgcn_global_load_lds((g_void *)(e + (long long)kb * 64 + lane),
-                                                 (lds_void *)(lbe + (buf * NBX + wave) * 64), 4, 0, 0);
-            }
+            if (wave < NBX)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(esrc, nkb * 256), (lds_void *)(lbe + (buf * NBX + wave) * 64),
+                                                         4, lane4, kb * 256, 0, 0);
         }
     };
     // A ring step is SPS operand slots and BS of the wave's batches: one slot of both batches.
