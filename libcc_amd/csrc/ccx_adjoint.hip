@@ -401,12 +401,13 @@ __global__ void __launch_bounds__(NTHR, 1) adj_item_kernel(AdjArgs ga)
                 else item_w_split<M_ACC, 2>(g, lds, it, acc, acc1, wave, lane, b0, b1);
             } else {
                 static_assert(!pair_modes(1), "the forward kernel's modes");
-                if (tkind == 2) item_w_f32v<M_IJJ>(g, lds, it, acc, wave, lane);
-                else if (tkind == 3) item_w_f32v<M_IIJ>(g, lds, it, acc, wave, lane);
-                else if (mult == 1) item_w_f32v<M_FULL>(g, lds, it, acc, wave, lane);
-                else if (mult == 6) item_w_f32v<M_AAA>(g, lds, it, acc, wave, lane);
-                else if (it.blk[0] == it.blk[1]) item_w_f32v<M_AAC>(g, lds, it, acc, wave, lane);
-                else item_w_f32v<M_ACC>(g, lds, it, acc, wave, lane);
+                f4 *b0 = reinterpret_cast<f4 *>(lds);
+                if (tkind == 2) item_w_f32v<M_IJJ>(g, lds, it, acc, wave, lane, b0, b0 + F32_BXU, b0 + 2 * F32_BXU);
+                else if (tkind == 3) item_w_f32v<M_IIJ>(g, lds, it, acc, wave, lane, b0, b0 + F32_BXU, b0 + 2 * F32_BXU);
+                else if (mult == 1) item_w_f32v<M_FULL>(g, lds, it, acc, wave, lane, b0, b0 + F32_BXU, b0 + 2 * F32_BXU);
+                else if (mult == 6) item_w_f32v<M_AAA>(g, lds, it, acc, wave, lane, b0, b0 + F32_BXU, b0 + 2 * F32_BXU);
+                else if (it.blk[0] == it.blk[1]) item_w_f32v<M_AAC>(g, lds, it, acc, wave, lane, b0, b0 + F32_BXU, b0 + 2 * F32_BXU);
+                else item_w_f32v<M_ACC>(g, lds, it, acc, wave, lane, b0, b0 + F32_BXU, b0 + 2 * F32_BXU);
             }
             // element (row 4 (lane >> 4) + v, column lane & 15) belongs to FP64-layout lane
             // 16 v + (lane & 15), slot lane >> 4 of the same wave

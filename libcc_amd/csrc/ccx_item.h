@@ -952,6 +952,8 @@ __device__ __forceinline__ void item_w_split(const TriplesArgs &g, double *lds, 
     if constexpr (TWO) complete_orderings<MODE, float>(lds, g1, wave, lane);
 }
 
+constexpr int F32_BXU = 6 * 64;   // units of 16 B of one BX buffer of the FP32 sweep (six operands at most)
+
 // ---- FP32 K sweep -------------------------------------------------------------------
 typedef const __attribute__((address_space(1))) f4 gf4;   // global memory, 16 B per lane
 
@@ -963,7 +965,7 @@ typedef const __attribute__((address_space(1))) f4 gf4;   // global memory, 16 B
 // ring and buffer index a compile-time constant.  4 bytes per operand element instead of 8.
 template <int PHASE, int MODE>
 __device__ __forceinline__ void run_phase_f32v(const TriplesArgs &g, const ItemCtx &it, f4 (&acc)[6][BPW],
-                                               f4 *lbx, int wave, int lane)
+                                               f4 *lb0, f4 *lb1, f4 *lb2, int wave, int lane)
 {
     constexpr int SM = slot_mask(PHASE, MODE), XM = bx_mask(PHASE, MODE);
     constexpr int NSL = __builtin_popcount(SM), NBX = __builtin_popcount(XM);
@@ -984,37 +986,37 @@ __device__ __forceinline__ void run_phase_f32v(const TriplesArgs &g, const ItemC
         const long long panel = ((long long)it.tpos[xp] * g.nb + r0[o]) * g.nb + r1[o];
         ap[s] = (gf4 *)(col[o] ? g.axc : g.axr) + panel * (16LL * nkb * 64) + (long long)wave * (2 * nkb * 64);
     }
-    gf4 *xq[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q)
-        xq[q] = (gf4 *)g.bx + ((long long)(it.ys[q] * g.no + it.zs[q]) * g.nb + G) * ((long long)nkb * 64);
-
-    f4 br;
-    auto bx_load = [&](int kb) __attribute__((always_inline)) {
-        static_for<NBX>([&](auto Cc) __attribute__((always_inline)) {
-            constexpr int c = decltype(Cc)::value;
-            if (wave == c) br = xq[nth_bit(XM, c)][kb * 64 + lane];
-        });
-    };
-    auto bx_store = [&](int buf) __attribute__((always_inline)) {
-        static_for<NBX>([&](auto Cc) __attribute__((always_inline)) {
-            constexpr int c = decltype(Cc)::value;
-            if (wave == c) lbx[(buf * NBX + c) * 64 + lane] = br;
-        });
+    // BX operand c of a block goes from global memory straight into LDS (buffer load, as in
+    // run_phase_split), loaded by wave c.  Through a register (whose next load had to wait for
+    // everything outstanding) the sweep stalled once a block: 753 ms at no=24, nu=216.
+    typedef __attribute__((address_space(3))) void lds_void;
+    int pg = 0;
+    static_for<NBX>([&](auto R) __attribute__((always_inline)) {
+        constexpr int r = decltype(R)::value, q = nth_bit(XM, r);
+        const int v = (it.ys[q] * g.no + it.zs[q]) * g.nb + G;
+        pg = wave == r ? v : pg;
+    });
+    const char *bsrc = static_cast<const char *>(g.bx) + (long long)pg * (nkb * 1024);
+    const int lane16 = lane * 16;
+    auto bx_load = [&](int kb, f4 *buf) __attribute__((always_inline)) {
+        if (wave < NBX)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(bsrc), 0, nkb * 1024, 0x00027000),
+                (lds_void *)(buf + wave * 64), 16, lane16, kb * 1024, 0, 0);
     };
     f4 ab[3][BPW];
     auto a_load = [&](int s, int kb, f4 (&d)[BPW]) __attribute__((always_inline)) {
 #pragma unroll
         for (int bb = 0; bb < BPW; ++bb) d[bb] = ap[s][(bb * nkb + kb) * 64 + lane];
     };
-    auto compute = [&](auto Sc, const f4 (&a)[BPW], int buf) __attribute__((always_inline)) {
+    auto compute = [&](auto Sc, const f4 (&a)[BPW], const f4 *buf) __attribute__((always_inline)) {
         constexpr int s = decltype(Sc)::value;
         constexpr SlotTerms ST = slot_terms(PHASE, MODE, s);
         f4 bs[ST.n > 0 ? ST.n : 1];
         static_for<ST.n>([&](auto N) __attribute__((always_inline)) {
             constexpr int n = decltype(N)::value;
             constexpr int rank = __builtin_popcount(XM & ((1 << ST.b[n]) - 1));
-            bs[n] = lbx[(buf * NBX + rank) * 64 + lane];
+            bs[n] = buf[rank * 64 + lane];
         });
         static_for<4>([&](auto J) __attribute__((always_inline)) {
             constexpr int j = decltype(J)::value;
@@ -1032,8 +1034,8 @@ __device__ __forceinline__ void run_phase_f32v(const TriplesArgs &g, const ItemC
         });
     };
 
-    bx_load(0);
-    bx_store(0);
+    bx_load(0, lb0);
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (!phase_active<PHASE>(g, it, wave)) {
         // only padding batches: stage this wave's BX chunks and meet every barrier
@@ -1041,8 +1043,8 @@ __device__ __forceinline__ void run_phase_f32v(const TriplesArgs &g, const ItemC
             static_for<3>([&](auto HB) __attribute__((always_inline)) {
                 constexpr int hb = decltype(HB)::value;
                 const int kbb = kb + hb;
-                bx_load(kbb + 1 < nkb ? kbb + 1 : nkb - 1);
-                bx_store((hb + 1) % 3);
+                bx_load(kbb + 1 < nkb ? kbb + 1 : nkb - 1, hb == 0 ? lb1 : hb == 1 ? lb2 : lb0);
+                __builtin_amdgcn_s_waitcnt(0);
                 __syncthreads();
             });
         }
@@ -1051,11 +1053,15 @@ __device__ __forceinline__ void run_phase_f32v(const TriplesArgs &g, const ItemC
     // steps t = block * NSL + slot index; the ring holds steps t, t+1, t+2
     a_load(nth_bit(SM, 0), 0, ab[0]);
     a_load(nth_bit(SM, 1 % NSL), 1 / NSL < nkb ? 1 / NSL : nkb - 1, ab[1]);
+    // the staged block was requested before this block's NSL >= 2 AX steps, of which the last two may
+    // stay in flight (loads retire in issue order): s_waitcnt vmcnt(2 BPW), nothing else
+    static_assert(NSL >= 2, "AX loads behind the staged block's");
+    constexpr int WAIT_DMA = (2 * BPW) | (7 << 4) | (15 << 8);
     for (int kb = 0; kb < nkb; kb += 3) {
         static_for<3>([&](auto HB) __attribute__((always_inline)) {
             constexpr int hb = decltype(HB)::value;
             const int kbb = kb + hb;
-            bx_load(kbb + 1 < nkb ? kbb + 1 : nkb - 1);
+            bx_load(kbb + 1 < nkb ? kbb + 1 : nkb - 1, hb == 0 ? lb1 : hb == 1 ? lb2 : lb0);
             static_for<NSL>([&](auto J) __attribute__((always_inline)) {
                 constexpr int j = decltype(J)::value;
                 constexpr int t = hb * NSL + j;
@@ -1065,10 +1071,10 @@ __device__ __forceinline__ void run_phase_f32v(const TriplesArgs &g, const ItemC
                 const int k2 = kb + t2 / NSL;
                 a_load(s2, k2 < nkb ? k2 : nkb - 1, ab[t2 % 3]);
                 __builtin_amdgcn_sched_barrier(0);
-                compute(std::integral_constant<int, s>{}, ab[t % 3], hb);
+                compute(std::integral_constant<int, s>{}, ab[t % 3], hb == 0 ? lb0 : hb == 1 ? lb1 : lb2);
                 __builtin_amdgcn_sched_barrier(0);
             });
-            bx_store((hb + 1) % 3);
+            __builtin_amdgcn_s_waitcnt(WAIT_DMA);
             __syncthreads();
         });
     }
@@ -1076,17 +1082,16 @@ __device__ __forceinline__ void run_phase_f32v(const TriplesArgs &g, const ItemC
 
 template <int MODE>
 __device__ __forceinline__ void item_w_f32v(const TriplesArgs &g, double *lds, const ItemCtx &it,
-                                            f4 (&acc)[6][BPW], int wave, int lane)
+                                            f4 (&acc)[6][BPW], int wave, int lane, f4 *lb0, f4 *lb1, f4 *lb2)
 {
 #pragma unroll
     for (int p = 0; p < 6; ++p)
 #pragma unroll
         for (int bb = 0; bb < BPW; ++bb) acc[p][bb] = f4{0, 0, 0, 0};
-    f4 *lbx = reinterpret_cast<f4 *>(lds);
-    run_phase_f32v<0, MODE>(g, it, acc, lbx, wave, lane);
+    run_phase_f32v<0, MODE>(g, it, acc, lb0, lb1, lb2, wave, lane);
     transpose_lb_to_l<MODE, float>(lds, acc, wave, lane);
-    run_phase_f32v<1, MODE>(g, it, acc, lbx, wave, lane);
-    run_phase_f32v<2, MODE>(g, it, acc, lbx, wave, lane);
+    run_phase_f32v<1, MODE>(g, it, acc, lb0, lb1, lb2, wave, lane);
+    run_phase_f32v<2, MODE>(g, it, acc, lb0, lb1, lb2, wave, lane);
     complete_orderings<MODE, float>(lds, acc, wave, lane);
 }
 

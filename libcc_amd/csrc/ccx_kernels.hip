@@ -485,11 +485,11 @@ __global__ void __launch_bounds__(NTHR, 1) triples_kernel(TriplesArgs g)
     extern __shared__ double lds[];
     __shared__ double red[NWAVE][112];
     __shared__ long long next_item;
-    // BX buffers of the split sweeps (run_phase_split).  The FP8 form's, 99 KB, do not fit beside the
+    // BX buffers of the FP32 and the split sweeps (run_phase_split).  The FP8 form's, 99 KB, do not fit beside the
     // transposition cubes and share their array.
     constexpr bool OWN_BX = FK == 2 || FK == 4;
-    constexpr int BXU = FK >= 2 ? split_bx_units<FK >= 2 ? FK : 2>() : 1;
-    __shared__ i32x4 bx0[OWN_BX ? BXU : 1], bx1[OWN_BX ? BXU : 1];
+    constexpr int BXU = FK >= 2 ? split_bx_units<FK >= 2 ? FK : 2>() : F32_BXU;
+    __shared__ i32x4 bx0[OWN_BX || FK == 1 ? BXU : 1], bx1[OWN_BX || FK == 1 ? BXU : 1], bx2[FK == 1 ? BXU : 1];
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -525,7 +525,9 @@ __global__ void __launch_bounds__(NTHR, 1) triples_kernel(TriplesArgs g)
             else if constexpr (FK >= 2)
                 item_w_split<MODE, FK>(g, lds, it, acc, acc1, wave, lane, reinterpret_cast<i32x4 *>(lds),
                                        reinterpret_cast<i32x4 *>(lds) + BXU);
-            else if constexpr (FK == 1) item_w_f32v<MODE>(g, lds, it, acc, wave, lane);
+            else if constexpr (FK == 1)
+                item_w_f32v<MODE>(g, lds, it, acc, wave, lane, reinterpret_cast<f4 *>(bx0), reinterpret_cast<f4 *>(bx1),
+                                  reinterpret_cast<f4 *>(bx2));
             else item_w<MODE, T>(g, lds, it, acc, wave, lane);
         };
         if constexpr (pair_modes(FK)) {
