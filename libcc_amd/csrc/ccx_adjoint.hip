@@ -443,8 +443,7 @@ __global__ void __launch_bounds__(NTHR, 1) adj_item_kernel(AdjArgs ga)
 namespace {
 constexpr int GTHR = 512;                 // GEMM work group: 8 waves, 2 per SIMD
 constexpr int GBPW = 2;                   // gax: rows b per wave
-constexpr int GCH = 128;                  // K columns per work group (8 MFMA tiles)
-constexpr int GCT = GCH / 16;
+constexpr int GAX_CT = 11;                // gax: most K tiles of a work group (accumulator registers)
 constexpr int BS_STR = 17;                // padded row of the staged BX slices
 typedef double d2 __attribute__((ext_vector_type(2)));
 constexpr int GBX_TILES = 19;             // gbx: gamma and K tiles of a work group (two 4 KB buffers each)
@@ -462,32 +461,35 @@ struct GemmArgs {
     const int *ent;         // (tl, sigma) pairs
     double *part;           // gbx: per (entry, split, chunk, gamma group) partial tiles
     int no, nu, nup, nb, kp, nchunk, gt, kt, ngg, nsplit;   // gbx: tiles gt x kt of a work group
-    int ch0;                // gax: first K chunk of this launch (nchunk chunks from there)
+    int k0;                 // gax: first K column of this launch (nchunk chunks from there)
 };
 
 // gAX[x](R0 16 x R1 16 rows, K chunk) += sum over entries (t,sigma) with t[xp] = x and over
 // the gamma blocks G of Wbar_t(e_u = a, e_v = b, e_wf = g) BX[t[yp],t[zp]](g, K).
 // Wave w owns rows b in {2w, 2w+1}, all 8 K tiles of the chunk.
-// NCT: K tiles of 16 the work group computes (GCT for full chunks, fewer for the last chunk
-// when kp is not a multiple of GCH, so no MFMA runs on K padding).
+// NCT: K tiles of 16 the work group computes, from column a.k0 + 16 NCT times its chunk; the launcher
+// splits K evenly, so no MFMA runs on K padding.  Contraction steps past the last virtual index, and
+// the MFMAs of waves whose two rows b lie past it, are left out.
 template <int NCT>
 __global__ void __launch_bounds__(GTHR, 1) gax_kernel(GemmArgs a)
 {
     extern __shared__ double lds[];
     double *WS = lds;                     // [2][WB_BLK]
-    double *BS = lds + 2 * WB_BLK;        // [2][GCH * BS_STR]
+    double *BS = lds + 2 * WB_BLK;        // [2][NCT * 16 * BS_STR]
+    constexpr int GCW = NCT * 16, NBL = (GCW * 8 + GTHR - 1) / GTHR;   // columns; BX loads of a thread
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int u = blockIdx.x;
-    const int ch = a.ch0 + u % a.nchunk; u /= a.nchunk;
+    const int ch = u % a.nchunk; u /= a.nchunk;
     const int R1 = u % a.nb; u /= a.nb;
     const int R0 = u % a.nb; u /= a.nb;
     const int ui = u;
     const int x = a.ulist[ui];
     const int e_beg = a.uoff[ui], e_end = a.uoff[ui + 1];
-    const int K0 = ch * GCH;
+    const int K0 = a.k0 + ch * GCW;
     const long long cube = (long long)a.nb * a.nb * a.nb * 4096;
     const int nsteps = (e_end - e_beg) * a.nb;
+    const bool rows = R1 * TB + wave * GBPW < a.nu;
 
     d4 acc[GBPW][NCT];
 #pragma unroll
@@ -495,8 +497,8 @@ __global__ void __launch_bounds__(GTHR, 1) gax_kernel(GemmArgs a)
 #pragma unroll
         for (int ct = 0; ct < NCT; ++ct) acc[bb][ct] = d4{0, 0, 0, 0};
 
-    // staging registers: Wbar block 4096 = 512 x 8, BX slice 16 x 128 = 512 x 4
-    double rw[8], rb[4];
+    // staging registers: Wbar block 4096 = 512 x 8, BX slice 16 x GCW
+    double rw[8], rb[2 * NBL];
     double rwgt = 1.0;                    // weight of the staged entry, applied when stashing
     auto fetch = [&](int step) {
         const int e = e_beg + step / a.nb, G = step % a.nb;
@@ -515,11 +517,11 @@ __global__ void __launch_bounds__(GTHR, 1) gax_kernel(GemmArgs a)
         }
         const double *bsrc = a.bx + (((long long)tpos[S.yp] * a.no + tpos[S.zp]) * a.nb + G) * (16LL * a.kp);
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int idx = 2 * (tid + k * GTHR);           // element of the 128 x 16 slice
+        for (int k = 0; k < NBL; ++k) {
+            const int idx = 2 * (tid + k * GTHR);           // element of the GCW x 16 slice
             const int Kl = idx >> 4;
             double2 v = {0.0, 0.0};
-            if (K0 + Kl < a.kp) v = reinterpret_cast<const double2 *>(bsrc + (long long)(K0 + Kl) * 16)[(idx & 15) >> 1];
+            if (Kl < GCW && K0 + Kl < a.kp) v = reinterpret_cast<const double2 *>(bsrc + (long long)(K0 + Kl) * 16)[(idx & 15) >> 1];
             rb[2 * k] = v.x; rb[2 * k + 1] = v.y;
         }
     };
@@ -532,11 +534,12 @@ __global__ void __launch_bounds__(GTHR, 1) gax_kernel(GemmArgs a)
             W[aa * WB_STR_A + b * WB_STR_B + c] = rw[2 * k];
             W[aa * WB_STR_A + b * WB_STR_B + c + 1] = rw[2 * k + 1];
         }
-        double *Bs = BS + buf * GCH * BS_STR;
+        double *Bs = BS + buf * GCW * BS_STR;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
+        for (int k = 0; k < NBL; ++k) {
             const int idx = 2 * (tid + k * GTHR);
             const int Kl = idx >> 4, gl = idx & 15;
+            if (Kl >= GCW) continue;
             Bs[Kl * BS_STR + gl] = rb[2 * k] * rwgt;
             Bs[Kl * BS_STR + gl + 1] = rb[2 * k + 1] * rwgt;
         }
@@ -555,9 +558,11 @@ __global__ void __launch_bounds__(GTHR, 1) gax_kernel(GemmArgs a)
         const int str[3] = {WB_STR_A, WB_STR_B, 1};
         const int su = str[S.u], sv = str[S.v], sw = str[S.wf];
         const double *W = WS + buf * WB_BLK;
-        const double *Bs = BS + buf * GCH * BS_STR;
+        const double *Bs = BS + buf * GCW * BS_STR;
+        const int gn = rows ? a.nu - (step % a.nb) * TB : 0;   // real gamma of this step's block
 #pragma unroll
         for (int kq = 0; kq < 4; ++kq) {
+            if (4 * kq >= gn) break;
             const int g = 4 * kq + (lane >> 4);
             double af[GBPW];
 #pragma unroll
@@ -859,7 +864,7 @@ template <int NCT>
 static int launch_gax(const GemmArgs &a, long long grid, hipStream_t s)
 {
     static bool attr_set = false;
-    const size_t lds_bytes = sizeof(double) * (2 * WB_BLK + 2 * GCH * BS_STR);
+    const size_t lds_bytes = sizeof(double) * (2 * WB_BLK + 2 * NCT * 16 * BS_STR);
     if (!attr_set) {
         if (hipFuncSetAttribute((const void *)gax_kernel<NCT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds_bytes) != hipSuccess)
@@ -868,6 +873,15 @@ static int launch_gax(const GemmArgs &a, long long grid, hipStream_t s)
     }
     gax_kernel<NCT><<<(unsigned)grid, GTHR, lds_bytes, s>>>(a);
     return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+// gax_kernel<ct> for a run-time tile count ct <= NCT
+template <int NCT>
+static int launch_gax_ct(int ct, const GemmArgs &a, long long grid, hipStream_t s)
+{
+    if (ct == NCT) return launch_gax<NCT>(a, grid, s);
+    if constexpr (NCT > 1) return launch_gax_ct<NCT - 1>(ct, a, grid, s);
+    else return 3;
 }
 
 template <int GM, int KN>
@@ -943,36 +957,29 @@ int ccx_hip_adj_items(const void *axr, const void *axc, const void *bx, const do
 }
 
 int ccx_hip_gax(const double *wbar, const double *bx, double *gax, const int *tuples, int t0, const int *xlist,
-                const int *xoff, const int *ent, int nx, int no, int nup, int kp, void *stream)
+                const int *xoff, const int *ent, int nx, int no, int nu, int nup, int kp, void *stream)
 {
     if (nx == 0) return 0;
     GemmArgs a = {};
     a.wbar = wbar; a.bx = bx; a.gax = gax; a.tuples = tuples; a.t0 = t0;
     a.ulist = xlist; a.uoff = xoff; a.ent = ent;
-    a.no = no; a.nup = nup; a.nb = nup / TB; a.kp = kp;
+    a.no = no; a.nu = nu; a.nup = nup; a.nb = nup / TB; a.kp = kp;
     hipStream_t s = (hipStream_t)stream;
-    // full K chunks, then the last partial chunk with only its K tiles
-    const int nfull = kp / GCH, tail = (kp % GCH + 15) / 16;
+    // As few chunks as GAX_CT tiles of accumulators allow, since every chunk stages the Wbar blocks
+    // again (11 of 80 ms at no=14, nu=150 with a chunk of 8 tiles and one of 3), split evenly: q tiles
+    // a chunk, one more for the first nk % n of them.
+    const int nk = (kp + 15) / 16, n = (nk + GAX_CT - 1) / GAX_CT, q = nk / n, more = nk % n;
+    const long long grid = (long long)nx * a.nb * a.nb;
     int rc = 0;
-    if (nfull > 0) {
-        a.ch0 = 0;
-        a.nchunk = nfull;
-        rc = launch_gax<GCT>(a, (long long)nx * a.nb * a.nb * nfull, s);
+    if (more > 0) {
+        a.k0 = 0;
+        a.nchunk = more;
+        rc = launch_gax_ct<GAX_CT>(q + 1, a, grid * more, s);
     }
-    if (rc == 0 && tail > 0) {
-        a.ch0 = nfull;
-        a.nchunk = 1;
-        const long long grid = (long long)nx * a.nb * a.nb;
-        switch (tail) {
-        case 1: rc = launch_gax<1>(a, grid, s); break;
-        case 2: rc = launch_gax<2>(a, grid, s); break;
-        case 3: rc = launch_gax<3>(a, grid, s); break;
-        case 4: rc = launch_gax<4>(a, grid, s); break;
-        case 5: rc = launch_gax<5>(a, grid, s); break;
-        case 6: rc = launch_gax<6>(a, grid, s); break;
-        case 7: rc = launch_gax<7>(a, grid, s); break;
-        default: rc = launch_gax<GCT>(a, grid, s); break;   // kp % GCH > 112
-        }
+    if (rc == 0) {
+        a.k0 = more * (q + 1) * 16;
+        a.nchunk = n - more;
+        rc = launch_gax_ct<GAX_CT>(q, a, grid * (n - more), s);
     }
     return rc;
 }

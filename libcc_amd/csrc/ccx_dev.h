@@ -69,7 +69,7 @@ int ccx_hip_adj_items(const void *axr, const void *axc, const void *bx, const do
                       int form, const void *const *w32, int kps, double wscale, void *stream);
 size_t ccx_hip_adj_stage_doubles(void);
 int ccx_hip_gax(const double *wbar, const double *bx, double *gax, const int *tuples, int t0, const int *xlist,
-                const int *xoff, const int *ent, int nx, int no, int nup, int kp, void *stream);
+                const int *xoff, const int *ent, int nx, int no, int nu, int nup, int kp, void *stream);
 size_t ccx_hip_gbx_part_doubles(int nup, int kp, int nent, int nsplit);
 int ccx_hip_gbx(const double *wbar, const double *axr, const double *axc, double *gbx, double *part,
                 const int *tuples, int t0, const int *plist, const int *poff, const int *ent, int npair, int nent,

@@ -826,7 +826,7 @@ int ccx_gradient_form(ccx_ctx *c, int form, double *ets, double *etd, double *dt
                               grid_size(c, (int64_t)tcount * nblk), form, form == CCX_FORM_FP64 ? NULL : w32,
                               form == CCX_FORM_FP32 ? (int)c->kpf : (int)c->kps, c->split_scale, c->stream) != 0 ||
             ccx_hip_gax(d_wbar, c->d_bx, d_gax, c->d_tuples, (int)t0, dl[0][0], dl[0][1], dl[0][2], nkeys[0], (int)no,
-                        (int)nup, (int)kp, c->stream) != 0 ||
+                        (int)nu, (int)nup, (int)kp, c->stream) != 0 ||
             ccx_hip_gbx(d_wbar, c->d_axr, c->d_axc, d_gbx, d_gpart, c->d_tuples, (int)t0, dl[1][0], dl[1][1],
                         dl[1][2], nkeys[1], nents[1], gbx_nsplit(nents[1], nb), (int)no, (int)nu, (int)nup, (int)kp,
                         c->stream) != 0 ||
