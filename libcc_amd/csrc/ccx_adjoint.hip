@@ -461,6 +461,7 @@ struct GemmArgs {
     const int *ent;         // (tl, sigma) pairs
     double *part;           // gbx: per (entry, split, chunk, gamma group) partial tiles
     int no, nu, nup, nb, kp, nchunk, gt, kt, ngg, nsplit;   // gbx: tiles gt x kt of a work group
+    int nx;                 // gax: number of keys in ulist
     int k0;                 // gax: first K column of this launch (nchunk chunks from there)
 };
 
@@ -483,7 +484,9 @@ __global__ void __launch_bounds__(GTHR, 1) gax_kernel(GemmArgs a)
     const int ch = u % a.nchunk; u /= a.nchunk;
     const int R1 = u % a.nb; u /= a.nb;
     const int R0 = u % a.nb; u /= a.nb;
-    const int ui = u;
+    // The keys are in increasing order and a batch's tuples share their largest index, whose entries
+    // outnumber the others': it goes first, so that the long work groups are not the last.
+    const int ui = a.nx - 1 - u;
     const int x = a.ulist[ui];
     const int e_beg = a.uoff[ui], e_end = a.uoff[ui + 1];
     const int K0 = a.k0 + ch * GCW;
@@ -963,7 +966,7 @@ int ccx_hip_gax(const double *wbar, const double *bx, double *gax, const int *tu
     GemmArgs a = {};
     a.wbar = wbar; a.bx = bx; a.gax = gax; a.tuples = tuples; a.t0 = t0;
     a.ulist = xlist; a.uoff = xoff; a.ent = ent;
-    a.no = no; a.nu = nu; a.nup = nup; a.nb = nup / TB; a.kp = kp;
+    a.no = no; a.nu = nu; a.nup = nup; a.nb = nup / TB; a.kp = kp; a.nx = nx;
     hipStream_t s = (hipStream_t)stream;
     // As few chunks as GAX_CT tiles of accumulators allow, since every chunk stages the Wbar blocks
     // again (11 of 80 ms at no=14, nu=150 with a chunk of 8 tiles and one of 3), split evenly: q tiles

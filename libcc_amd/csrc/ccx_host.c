@@ -15,6 +15,11 @@
 #define TB 16
 /* largest upload buffer a context keeps between ccx_load_host calls (larger ones are freed again) */
 #define KEEP_UPLOAD ((size_t)256 << 20)
+/* largest gradient workspace a context keeps between calls (until ccx_destroy): the default batch and
+ * its accumulators up to about no=24, nu=216.  Allocating and freeing it on every call took 1.5 ms of 21
+ * at no=8, nu=120 (2.7 GB) and from 4 to several hundred ms at no=14, nu=150 (17 GB), as the driver had
+ * pages ready or not. */
+#define KEEP_GRAD ((size_t)20 << 30)
 
 struct ccx_ctx {
     int64_t no, nu, nup, nb, kp;
@@ -41,6 +46,8 @@ struct ccx_ctx {
     double *d_arena;                    /* the small device arrays, one allocation */
     double *d_up;                       /* ccx_load_host's upload buffer, kept up to KEEP_UPLOAD bytes */
     size_t up_bytes;
+    double *d_grad;                     /* ccx_gradient's workspace, kept up to KEEP_GRAD bytes */
+    size_t grad_bytes;
     double kernel_ms, total_ms;
     void *ev[4];
 };
@@ -171,6 +178,7 @@ int ccx_destroy(ccx_ctx *c)
     free_dev(c);
     ccx_hip_free(c->d_flag);
     ccx_hip_free(c->d_up);
+    ccx_hip_free(c->d_grad);
     ccx_hip_host_free(c->h_res);
     for (int q = 0; q < 4; ++q) ccx_hip_event_destroy(c->ev[q]);
     free(c->h_tuples);
@@ -738,7 +746,7 @@ int ccx_gradient_form(ccx_ctx *c, int form, double *ets, double *etd, double *dt
     double host_out[2] = {0.0, 0.0};
     /* batch of tuples: Wbar cubes + dVOE slots within a memory budget (CCX_ADJ_BATCH_MB) */
     const double per_tuple = 8.0 * (double)(nup * nup * nup) + 8.0 * 6.0 * (double)(nb * nb * nb) * 256.0;
-    double budget = 16384.0;
+    double budget = 16384.0;   /* MB; with 4096 the back-contractions ran 15 % longer at no=14, nu=150 */
     const char *env = getenv("CCX_ADJ_BATCH_MB");
     if (env && atof(env) > 0) budget = atof(env);
     int64_t tb = (int64_t)(budget * 1048576.0 / per_tuple);
@@ -751,13 +759,6 @@ int ccx_gradient_form(ccx_ctx *c, int form, double *ets, double *etd, double *dt
     h_tmp = (int *)malloc(sizeof(int) * (size_t)(3 * nent + nkey));
     h_lists = (int *)malloc(sizeof(int) * (size_t)lsz);
     if (!h_tmp || !h_lists) { rc = CCX_ERR_ALLOC; goto fail; }
-    DALLOC(d_gax, no * nup * nup * kp);
-    DALLOC(d_gbx, no * no * nup * kp);
-    DALLOC(d_dvoep, no * no * nup * nup);
-    DALLOC(d_wbar, tb * nup * nup * nup);
-    DALLOC(d_slots, tb * 6 * nb * nb * nb * 256);
-    DALLOC(d_lists, lsz);
-    DALLOC(d_wstage, (int64_t)grid_size(c, tb * nblk) * (int64_t)ccx_hip_adj_stage_doubles());
     {   /* gbx partial tiles: the largest entries x splits any batch can need (a batch holds
          * 1 .. 6 tb gBX entries, fewer than 6 per tuple when degenerate tuples merge pairs,
          * and the split count grows as the entry count falls) */
@@ -767,7 +768,25 @@ int ccx_gradient_form(ccx_ctx *c, int form, double *ets, double *etd, double *dt
             if (u > umax) umax = u;
         }
         gpart_units = umax;
-        DALLOC(d_gpart, (int64_t)ccx_hip_gbx_part_doubles((int)nup, (int)kp, (int)umax, 1));
+        /* one allocation: gax, gbx, dvoep (cleared below, so adjoining), wbar, slots, wstage, gpart, lists */
+        const int64_t n[8] = {no * nup * nup * kp, no * no * nup * kp, no * no * nup * nup, tb * nup * nup * nup,
+                              tb * 6 * nb * nb * nb * 256,
+                              (int64_t)grid_size(c, tb * nblk) * (int64_t)ccx_hip_adj_stage_doubles(),
+                              (int64_t)ccx_hip_gbx_part_doubles((int)nup, (int)kp, (int)umax, 1), (lsz + 1) / 2};
+        double **dst[7] = {&d_gax, &d_gbx, &d_dvoep, &d_wbar, &d_slots, &d_wstage, &d_gpart};
+        int64_t off[8], total = 0;
+        for (int q = 0; q < 8; ++q) {
+            off[q] = total;
+            total += (n[q] + 31) / 32 * 32;
+        }
+        if (sizeof(double) * (size_t)total > c->grad_bytes) {
+            ccx_hip_free(c->d_grad);
+            c->grad_bytes = 0;
+            DALLOC(c->d_grad, total);
+            c->grad_bytes = sizeof(double) * (size_t)total;
+        }
+        for (int q = 0; q < 7; ++q) *dst[q] = c->d_grad + off[q];
+        d_lists = (int *)(c->d_grad + off[7]);
     }
     if (ccx_hip_zero(d_gax, sizeof(double) * (size_t)(no * nup * nup * kp), c->stream) != 0 ||
         ccx_hip_zero(d_gbx, sizeof(double) * (size_t)(no * no * nup * kp), c->stream) != 0 ||
@@ -872,10 +891,11 @@ int ccx_gradient_form(ccx_ctx *c, int form, double *ets, double *etd, double *dt
     if (ets) *ets = host_out[1];
 fail:
     ccx_hip_sync(c->stream);
-    ccx_hip_free(d_gax); ccx_hip_free(d_gbx); ccx_hip_free(d_dvoep); ccx_hip_free(d_wbar); ccx_hip_free(d_slots);
-    ccx_hip_free(d_lists);
-    ccx_hip_free(d_wstage);
-    ccx_hip_free(d_gpart);
+    if (c->grad_bytes > KEEP_GRAD) {
+        ccx_hip_free(c->d_grad);
+        c->d_grad = NULL;
+        c->grad_bytes = 0;
+    }
     for (int q = 0; q < 5; ++q) ccx_hip_free(d_out[q]);
     free(h_tmp);
     free(h_lists);
