@@ -880,6 +880,8 @@ __device__ __forceinline__ void run_phase_split(const TriplesArgs &g, const Item
     // that waits until at most NPF vector-memory loads are outstanding, nothing else
     constexpr int NPF = (NSL < SPS ? NSL : SPS) * BS * (NS * F16 + (CF::MX ? 1 : 0));
     static_assert(NPF < 64, "vmcnt range");
+    // the first step's loads may be issued ahead of the direct loads, the last step's may not
+    static_assert(NST >= 2, "AX loads certainly behind the staged block's");
     constexpr int WAIT_DMA = (NPF & 15) | ((NPF >> 4) << 14) | (7 << 4) | (15 << 8);
     bx_load(0, 0);
     __builtin_amdgcn_s_waitcnt(0);
@@ -1053,10 +1055,13 @@ __device__ __forceinline__ void run_phase_f32v(const TriplesArgs &g, const ItemC
     // steps t = block * NSL + slot index; the ring holds steps t, t+1, t+2
     a_load(nth_bit(SM, 0), 0, ab[0]);
     a_load(nth_bit(SM, 1 % NSL), 1 / NSL < nkb ? 1 / NSL : nkb - 1, ab[1]);
-    // the staged block was requested before this block's NSL >= 2 AX steps, of which the last two may
-    // stay in flight (loads retire in issue order): s_waitcnt vmcnt(2 BPW), nothing else
-    static_assert(NSL >= 2, "AX loads behind the staged block's");
-    constexpr int WAIT_DMA = (2 * BPW) | (7 << 4) | (15 << 8);
+    // The AX steps whose loads may stay in flight when the staged block is published (loads retire in
+    // issue order): the last two, but only steps after the block's first, whose loads the
+    // compiler may issue ahead of the direct load (no scheduling barrier lies between them).
+    // With two slots (M_AAA) that is one step.  s_waitcnt vmcnt(FLIGHT BPW), nothing else.
+    constexpr int FLIGHT = NSL > 2 ? 2 : 1;
+    static_assert(FLIGHT <= NSL - 1, "AX loads certainly behind the staged block's");
+    constexpr int WAIT_DMA = (FLIGHT * BPW) | (7 << 4) | (15 << 8);
     for (int kb = 0; kb < nkb; kb += 3) {
         static_for<3>([&](auto HB) __attribute__((always_inline)) {
             constexpr int hb = decltype(HB)::value;
