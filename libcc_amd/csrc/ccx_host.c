@@ -272,14 +272,20 @@ int ccx_load_device(ccx_ctx *c, const double *eh, const double *ep, const double
         const size_t n[7] = {(size_t)no, (size_t)nu, (size_t)(no * nu), (size_t)(nu * nu * no * no),
                              (size_t)(no * nu * no * no), (size_t)(nu * nu * no * no),
                              vvvo_layout == 0 ? (size_t)(nu * nu * nu * no) : (size_t)(nu * (nu + 1) / 2 * nu * no)};
-        int bad = 0;
-        /* the flag is zero between calls: cleared when allocated and after a bad input */
-        if (!c->d_flag) {
-            if (ccx_hip_malloc((void **)&c->d_flag, sizeof(unsigned int)) != 0) return CCX_ERR_ALLOC;
-            if (ccx_hip_zero_flag(c->d_flag, c->stream) != 0) return CCX_ERR_DEVICE;
+        const int fresh = !c->d_flag;
+        int bad = 0, rc = CCX_OK;
+        /* The flag is zero between calls.  A scan that does not end with a clean flag gives it up (freeing
+         * waits for the device), so that nothing of it, also nothing queued on this stream, meets
+         * a later load: the next one starts with a new flag. */
+        if (!c->d_flag && ccx_hip_malloc((void **)&c->d_flag, sizeof(unsigned int)) != 0) return CCX_ERR_ALLOC;
+        else if (fresh && ccx_hip_zero_flag(c->d_flag, c->stream) != 0) rc = CCX_ERR_DEVICE;
+        else if (ccx_hip_nonfinite(arr, n, 7, c->d_flag, &bad, c->stream) != 0) rc = CCX_ERR_DEVICE;
+        else if (bad) rc = CCX_ERR_INPUT;
+        if (rc != CCX_OK) {
+            ccx_hip_free(c->d_flag);
+            c->d_flag = NULL;
+            return rc;
         }
-        if (ccx_hip_nonfinite(arr, n, 7, c->d_flag, &bad, c->stream) != 0) return CCX_ERR_DEVICE;
-        if (bad) return ccx_hip_zero_flag(c->d_flag, c->stream) != 0 ? CCX_ERR_DEVICE : CCX_ERR_INPUT;
     }
     return build_from_device(c, eh, ep, t1, t2, vm, voe, vvvo, vvvo_layout);
 }
