@@ -73,7 +73,8 @@ int ccx_destroy(ccx_ctx *ctx);
 
 /* Upload inputs from host memory (reference layouts).  vvvo_layout: 0 = unpacked
  * (nu,nu,nu,no), 1 = distributed packed (nutr, nu*no).  Inputs are checked for
- * NaN/Inf (CCX_ERR_INPUT).  The context keeps an upload buffer of at most 256 MiB until ccx_destroy. */
+ * NaN/Inf (CCX_ERR_INPUT).  The context keeps an upload buffer of at most 256 MiB
+ * until ccx_destroy, or until an allocation of this library fails for want of memory. */
 int ccx_load_host(ccx_ctx *ctx, const double *eh, const double *ep, const double *t1,
                   const double *t2, const double *vm, const double *voe, const double *vvvo,
                   int vvvo_layout);
@@ -133,7 +134,9 @@ int ccx_work_stats(const ccx_ctx *ctx, int64_t *items, double *executed_flops);
  * energies.  The reference has no adjoint; the energy it differentiates is
  * src/triples-ijk/triples.F90:29-313 (W from ijk_tuple.f90:56-84, E[T] and v1 from
  * t1wt3.f90:53-102, ets = 2 T1.v1 from triples.F90:310-313).  The context keeps the call's device
- * workspace for the next one when it is at most 20 GiB, until ccx_destroy. */
+ * workspace for the next one when it is at most 20 GiB and at least half of the device's memory is free
+ * beside it, until ccx_destroy, or until an allocation of this library, for any context, fails for want
+ * of memory. */
 int ccx_gradient(ccx_ctx *ctx, double *ets, double *etd, double *dt1, double *dt2, double *dvm, double *dvoe,
                  double *dvvvo, int on_device);
 

@@ -9,6 +9,7 @@
 int ccx_hip_device_count(int *n);
 int ccx_hip_malloc(void **p, size_t bytes);
 int ccx_hip_free(void *p);
+int ccx_hip_mem_info(size_t *free_bytes, size_t *total_bytes);
 int ccx_hip_memcpy_h2d(void *dst, const void *src, size_t bytes, void *stream);
 int ccx_hip_memcpy_d2h(void *dst, const void *src, size_t bytes, void *stream);
 int ccx_hip_memcpy_d2d(void *dst, const void *src, size_t bytes, void *stream);
@@ -18,7 +19,6 @@ int ccx_hip_host_free(void *p);
 int ccx_hip_memcpy_h2d_queue(void *dst, const void *src, size_t bytes, void *stream);
 int ccx_hip_sync(void *stream);
 int ccx_hip_cu_count(int *n);
-const char *ccx_hip_last_error(void);
 int ccx_hip_lds_bytes(void);
 
 int ccx_hip_zero_flag(unsigned int *d_flag, void *stream);

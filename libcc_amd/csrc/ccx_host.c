@@ -4,6 +4,7 @@
  * reference's triples path.  All device work goes through the thin ABI in ccx_dev.h.
  */
 #include <math.h>
+#include <pthread.h>
 #include <stdio.h>
 #include <stdint.h>
 #include <stdlib.h>
@@ -15,10 +16,12 @@
 #define TB 16
 /* largest upload buffer a context keeps between ccx_load_host calls (larger ones are freed again) */
 #define KEEP_UPLOAD ((size_t)256 << 20)
-/* largest gradient workspace a context keeps between calls (until ccx_destroy): the default batch and
- * its accumulators up to about no=24, nu=216.  Allocating and freeing it on every call took 1.5 ms of 21
- * at no=8, nu=120 (2.7 GB) and from 4 to several hundred ms at no=14, nu=150 (17 GB), as the driver had
- * pages ready or not. */
+/* largest gradient workspace a context keeps between calls: the default batch and its accumulators up
+ * to about no=24, nu=216.  Allocating and freeing it on every call took 1.5 ms of 21 at no=8, nu=120
+ * (2.7 GB) and from 4 to several hundred ms at no=14, nu=150 (17 GB), as the driver had pages ready or
+ * not.  It is kept only while at least half of the device's memory is free beside it (a caller whose own data
+ * fill the device gets it back with every call), and goes back when an allocation of any
+ * context fails (dev_malloc), at the latest with ccx_destroy. */
 #define KEEP_GRAD ((size_t)20 << 30)
 
 struct ccx_ctx {
@@ -48,6 +51,8 @@ struct ccx_ctx {
     size_t up_bytes;
     double *d_grad;                     /* ccx_gradient's workspace, kept up to KEEP_GRAD bytes */
     size_t grad_bytes;
+    int up_busy, grad_busy;             /* a call is using the kept buffer (under g_keep_lock) */
+    ccx_ctx *next;                      /* in g_contexts */
     double kernel_ms, total_ms;
     void *ev[4];
 };
@@ -66,6 +71,45 @@ const char *ccx_error_string(int s)
     case CCX_ERR_SCRATCH: return "problem larger than the static scratch array";
     default: return "unknown status";
     }
+}
+
+/* ------------------------------------------------------------------ kept buffers */
+
+/* Every context, so that a failing allocation of any of them can have the buffers the others keep.
+ * The lock covers the list, the busy marks and the freeing of kept buffers; contexts may be
+ * used from different threads (one thread each). */
+static pthread_mutex_t g_keep_lock = PTHREAD_MUTEX_INITIALIZER;
+static ccx_ctx *g_contexts = NULL;
+
+static void keep_busy(int *mark, int value)
+{
+    pthread_mutex_lock(&g_keep_lock);
+    *mark = value;
+    pthread_mutex_unlock(&g_keep_lock);
+}
+
+static size_t drop_kept(double **buf, size_t *bytes)
+{
+    const size_t had = *bytes;
+    ccx_hip_free(*buf);
+    *buf = NULL;
+    *bytes = 0;
+    return had;
+}
+
+/* Device memory for the host layer: where there is none, the kept buffers that no call is using go back
+ * first. */
+static int dev_malloc(void **p, size_t bytes)
+{
+    if (ccx_hip_malloc(p, bytes) == 0) return 0;
+    size_t back = 0;
+    pthread_mutex_lock(&g_keep_lock);
+    for (ccx_ctx *c = g_contexts; c; c = c->next) {
+        if (!c->grad_busy) back += drop_kept(&c->d_grad, &c->grad_bytes);
+        if (!c->up_busy) back += drop_kept(&c->d_up, &c->up_bytes);
+    }
+    pthread_mutex_unlock(&g_keep_lock);
+    return back > 0 ? ccx_hip_malloc(p, bytes) : 1;
 }
 
 /* ------------------------------------------------------------------ schedule tables */
@@ -168,6 +212,10 @@ int ccx_create(int64_t no, int64_t nu, ccx_ctx **out)
     build_blocks(c->nb, c->h_blocks);
     for (int q = 0; q < 4; ++q)
         if (ccx_hip_event_create(&c->ev[q]) != 0) { free(c->h_tuples); free(c->h_blocks); free(c); return CCX_ERR_DEVICE; }
+    pthread_mutex_lock(&g_keep_lock);
+    c->next = g_contexts;
+    g_contexts = c;
+    pthread_mutex_unlock(&g_keep_lock);
     *out = c;
     return CCX_OK;
 }
@@ -175,6 +223,10 @@ int ccx_create(int64_t no, int64_t nu, ccx_ctx **out)
 int ccx_destroy(ccx_ctx *c)
 {
     if (!c) return CCX_ERR_ARG;
+    pthread_mutex_lock(&g_keep_lock);
+    for (ccx_ctx **q = &g_contexts; *q; q = &(*q)->next)
+        if (*q == c) { *q = c->next; break; }
+    pthread_mutex_unlock(&g_keep_lock);
     free_dev(c);
     ccx_hip_free(c->d_flag);
     ccx_hip_free(c->d_up);
@@ -196,7 +248,7 @@ int ccx_set_stream(ccx_ctx *c, void *stream)
 
 #define DALLOC(ptr, count)                                                             \
     do {                                                                               \
-        if (ccx_hip_malloc((void **)&(ptr), sizeof(*(ptr)) * (size_t)(count)) != 0) { \
+        if (dev_malloc((void **)&(ptr), sizeof(*(ptr)) * (size_t)(count)) != 0) { \
             rc = CCX_ERR_ALLOC;                                                        \
             goto fail;                                                                 \
         }                                                                              \
@@ -277,7 +329,7 @@ int ccx_load_device(ccx_ctx *c, const double *eh, const double *ep, const double
         /* The flag is zero between calls.  A scan that does not end with a clean flag gives it up (freeing
          * waits for the device), so that nothing of it, also nothing queued on this stream, meets
          * a later load: the next one starts with a new flag. */
-        if (!c->d_flag && ccx_hip_malloc((void **)&c->d_flag, sizeof(unsigned int)) != 0) return CCX_ERR_ALLOC;
+        if (!c->d_flag && dev_malloc((void **)&c->d_flag, sizeof(unsigned int)) != 0) return CCX_ERR_ALLOC;
         else if (fresh && ccx_hip_zero_flag(c->d_flag, c->stream) != 0) rc = CCX_ERR_DEVICE;
         else if (ccx_hip_nonfinite(arr, n, 7, c->d_flag, &bad, c->stream) != 0) rc = CCX_ERR_DEVICE;
         else if (bad) rc = CCX_ERR_INPUT;
@@ -308,24 +360,21 @@ int ccx_load_host(ccx_ctx *c, const double *eh, const double *ep, const double *
         total += (n[q] + 31) / 32 * 32;
     }
     total *= sizeof(double);
-    if (total > c->up_bytes) {
-        ccx_hip_free(c->d_up);
-        c->up_bytes = 0;
-        if (ccx_hip_malloc((void **)&c->d_up, total) != 0) return CCX_ERR_ALLOC;
-        c->up_bytes = total;
-    }
     int rc = CCX_OK;
+    keep_busy(&c->up_busy, 1);
+    if (total > c->up_bytes) {
+        drop_kept(&c->d_up, &c->up_bytes);
+        if (dev_malloc((void **)&c->d_up, total) != 0) rc = CCX_ERR_ALLOC;
+        else c->up_bytes = total;
+    }
     for (int q = 0; q < 7 && rc == CCX_OK; ++q)
         if (ccx_hip_memcpy_h2d(c->d_up + off[q], src[q], sizeof(double) * n[q], c->stream) != 0) rc = CCX_ERR_DEVICE;
     if (rc == CCX_OK)
         rc = ccx_load_device(c, c->d_up + off[0], c->d_up + off[1], c->d_up + off[2], c->d_up + off[3], c->d_up + off[4],
                              c->d_up + off[5], c->d_up + off[6], vvvo_layout);
-    if (c->up_bytes > KEEP_UPLOAD) {
-        ccx_hip_sync(c->stream);
-        ccx_hip_free(c->d_up);
-        c->d_up = NULL;
-        c->up_bytes = 0;
-    }
+    if (rc != CCX_OK) ccx_hip_sync(c->stream);   /* a load that succeeded has been waited for */
+    if (c->up_bytes > KEEP_UPLOAD) drop_kept(&c->d_up, &c->up_bytes);
+    keep_busy(&c->up_busy, 0);
     return rc;
 }
 
@@ -345,9 +394,9 @@ static int ensure_f32(ccx_ctx *c)
     if (c->f32_ready) return CCX_OK;
     const int64_t nax = c->no * c->nb * c->nb * 256 * c->kpf, nbx = c->no * c->no * c->nb * 16 * c->kpf;
     if (!c->d_axr32) {
-        if (ccx_hip_malloc((void **)&c->d_axr32, sizeof(float) * (size_t)nax) != 0 ||
-            ccx_hip_malloc((void **)&c->d_axc32, sizeof(float) * (size_t)nax) != 0 ||
-            ccx_hip_malloc((void **)&c->d_bx32, sizeof(float) * (size_t)nbx) != 0) {
+        if (dev_malloc((void **)&c->d_axr32, sizeof(float) * (size_t)nax) != 0 ||
+            dev_malloc((void **)&c->d_axc32, sizeof(float) * (size_t)nax) != 0 ||
+            dev_malloc((void **)&c->d_bx32, sizeof(float) * (size_t)nbx) != 0) {
             ccx_hip_free(c->d_axr32); ccx_hip_free(c->d_axc32); ccx_hip_free(c->d_bx32);
             c->d_axr32 = c->d_axc32 = c->d_bx32 = NULL;
             return CCX_ERR_ALLOC;
@@ -376,9 +425,9 @@ static int ensure_split(ccx_ctx *c, int form)
         c->d_axr_s = c->d_axc_s = c->d_bx_s = NULL;
         c->d_max = NULL;
         c->split_ax_bytes = c->split_bx_bytes = 0;
-        if (ccx_hip_malloc(&c->d_axr_s, ax_bytes) != 0 || ccx_hip_malloc(&c->d_axc_s, ax_bytes) != 0 ||
-            ccx_hip_malloc(&c->d_bx_s, bx_bytes) != 0 ||
-            ccx_hip_malloc((void **)&c->d_max, 2 * sizeof(unsigned long long)) != 0) {
+        if (dev_malloc(&c->d_axr_s, ax_bytes) != 0 || dev_malloc(&c->d_axc_s, ax_bytes) != 0 ||
+            dev_malloc(&c->d_bx_s, bx_bytes) != 0 ||
+            dev_malloc((void **)&c->d_max, 2 * sizeof(unsigned long long)) != 0) {
             ccx_hip_free(c->d_axr_s); ccx_hip_free(c->d_axc_s); ccx_hip_free(c->d_bx_s); ccx_hip_free(c->d_max);
             c->d_axr_s = c->d_axc_s = c->d_bx_s = NULL;
             c->d_max = NULL;
@@ -389,9 +438,9 @@ static int ensure_split(ccx_ctx *c, int form)
     }
     if (form == CCX_FORM_FP8X4 && !c->d_axr_e) {   /* one word per 32 elements */
         const size_t ax_w = (size_t)(c->no * c->nb * c->nb * 256 * kps / 32), bx_w = (size_t)(c->no * c->no * c->nb * 16 * kps / 32);
-        if (ccx_hip_malloc((void **)&c->d_axr_e, sizeof(int) * ax_w) != 0 ||
-            ccx_hip_malloc((void **)&c->d_axc_e, sizeof(int) * ax_w) != 0 ||
-            ccx_hip_malloc((void **)&c->d_bx_e, sizeof(int) * bx_w) != 0) {
+        if (dev_malloc((void **)&c->d_axr_e, sizeof(int) * ax_w) != 0 ||
+            dev_malloc((void **)&c->d_axc_e, sizeof(int) * ax_w) != 0 ||
+            dev_malloc((void **)&c->d_bx_e, sizeof(int) * bx_w) != 0) {
             ccx_hip_free(c->d_axr_e); ccx_hip_free(c->d_axc_e); ccx_hip_free(c->d_bx_e);
             c->d_axr_e = c->d_axc_e = c->d_bx_e = NULL;
             return CCX_ERR_ALLOC;
@@ -484,7 +533,7 @@ int ccx_energy_tuples(ccx_ctx *c, int form, int64_t n, const int64_t *ijk, doubl
     }
     int *d = NULL;
     int rc = CCX_OK;
-    if (ccx_hip_malloc((void **)&d, sizeof(int) * 4 * (size_t)(n > 0 ? n : 1)) != 0) { free(h); return CCX_ERR_ALLOC; }
+    if (dev_malloc((void **)&d, sizeof(int) * 4 * (size_t)(n > 0 ? n : 1)) != 0) { free(h); return CCX_ERR_ALLOC; }
     if (n > 0 && ccx_hip_memcpy_h2d(d, h, sizeof(int) * 4 * (size_t)n, c->stream) != 0) rc = CCX_ERR_DEVICE;
     if (rc == CCX_OK) rc = energy_run(c, form, d, n, ets, etd, v1, v1_on_device);
     ccx_hip_sync(c->stream);
@@ -598,9 +647,8 @@ int ccx_energy_abc(ccx_ctx *c, double *etd)
         DALLOC(d_x, batch);
         /* the packed copies of the matrix-core route (axt has the size of a slab, its occupied index
          * padded to 16); without room for them the triples go through w_abc_kernel */
-        if (ccx_hip_malloc((void **)&d_axt, sizeof(double) * ccx_hip_abc_a_doubles((int)c->no, (int)c->nu, (int)c->kp)) != 0 ||
-            ccx_hip_malloc((void **)&d_bxt, sizeof(double) * ccx_hip_abc_b_doubles((int)c->no, (int)c->nu, (int)c->kp)) != 0) {
-            (void)ccx_hip_last_error();   /* handled here: clears it for the launches below */
+        if (dev_malloc((void **)&d_axt, sizeof(double) * ccx_hip_abc_a_doubles((int)c->no, (int)c->nu, (int)c->kp)) != 0 ||
+            dev_malloc((void **)&d_bxt, sizeof(double) * ccx_hip_abc_b_doubles((int)c->no, (int)c->nu, (int)c->kp)) != 0) {
             ccx_hip_free(d_axt);
             d_axt = d_bxt = NULL;
         }
@@ -762,6 +810,7 @@ int ccx_gradient_form(ccx_ctx *c, int form, double *ets, double *etd, double *dt
     const int64_t nkey = no * no;
     /* host list scratch: key/tl/code arrays (3 x nent), count (nkey), and three CSR sets */
     const int64_t lsz = 3 * (nkey + (nkey + 1) + 2 * nent);
+    keep_busy(&c->grad_busy, 1);
     h_tmp = (int *)malloc(sizeof(int) * (size_t)(3 * nent + nkey));
     h_lists = (int *)malloc(sizeof(int) * (size_t)lsz);
     if (!h_tmp || !h_lists) { rc = CCX_ERR_ALLOC; goto fail; }
@@ -786,8 +835,7 @@ int ccx_gradient_form(ccx_ctx *c, int form, double *ets, double *etd, double *dt
             total += (n[q] + 31) / 32 * 32;
         }
         if (sizeof(double) * (size_t)total > c->grad_bytes) {
-            ccx_hip_free(c->d_grad);
-            c->grad_bytes = 0;
+            drop_kept(&c->d_grad, &c->grad_bytes);
             DALLOC(c->d_grad, total);
             c->grad_bytes = sizeof(double) * (size_t)total;
         }
@@ -897,12 +945,11 @@ int ccx_gradient_form(ccx_ctx *c, int form, double *ets, double *etd, double *dt
     if (ets) *ets = host_out[1];
 fail:
     ccx_hip_sync(c->stream);
-    if (c->grad_bytes > KEEP_GRAD) {
-        ccx_hip_free(c->d_grad);
-        c->d_grad = NULL;
-        c->grad_bytes = 0;
-    }
     for (int q = 0; q < 5; ++q) ccx_hip_free(d_out[q]);
+    size_t room = 0, all = 1;
+    if (c->grad_bytes > KEEP_GRAD || ccx_hip_mem_info(&room, &all) != 0 || room < all / 2)
+        drop_kept(&c->d_grad, &c->grad_bytes);
+    keep_busy(&c->grad_busy, 0);
     free(h_tmp);
     free(h_lists);
     return rc;

@@ -819,7 +819,15 @@ int ccx_hip_malloc(void **p, size_t bytes)
 {
     *p = nullptr;
     if (bytes == 0) return 0;
-    return hipMalloc(p, bytes) == hipSuccess ? 0 : 1;
+    if (hipMalloc(p, bytes) == hipSuccess) return 0;
+    *p = nullptr;
+    (void)hipGetLastError();   // reported here: the check of a later launch must not find it
+    return 1;
+}
+
+int ccx_hip_mem_info(size_t *free_bytes, size_t *total_bytes)
+{
+    return hipMemGetInfo(free_bytes, total_bytes) == hipSuccess ? 0 : 1;
 }
 
 int ccx_hip_free(void *p) { return (p == nullptr || hipFree(p) == hipSuccess) ? 0 : 1; }
@@ -853,7 +861,10 @@ int ccx_hip_memcpy_h2d_queue(void *dst, const void *src, size_t bytes, void *str
 int ccx_hip_host_malloc(void **p, size_t bytes)
 {
     *p = nullptr;
-    return hipHostMalloc(p, bytes, hipHostMallocDefault) == hipSuccess ? 0 : 1;
+    if (hipHostMalloc(p, bytes, hipHostMallocDefault) == hipSuccess) return 0;
+    *p = nullptr;
+    (void)hipGetLastError();
+    return 1;
 }
 
 int ccx_hip_host_free(void *p) { return (p == nullptr || hipHostFree(p) == hipSuccess) ? 0 : 1; }
@@ -866,8 +877,6 @@ int ccx_hip_cu_count(int *n)
     if (hipGetDevice(&dev) != hipSuccess) return 1;
     return hipDeviceGetAttribute(n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess ? 0 : 1;
 }
-
-const char *ccx_hip_last_error(void) { return hipGetErrorString(hipGetLastError()); }
 
 
 // AX in both orientations from VVVO (layout V_FULL, V_PACKED or V_VE) and T2 of nx occupied indices

@@ -7,7 +7,8 @@
 #include <stdlib.h>
 #include <string.h>
 
-long long fake_room = 1LL << 40;   /* bytes still to be had */
+long long fake_total = 1LL << 40;  /* device memory, bytes */
+long long fake_room = 1LL << 40;   /* what can still be had of it */
 int fake_fail_zero_flag, fake_fail_scan;   /* how many of the next calls fail */
 void (*fake_during_adjoint)(void);         /* called while a gradient's kernels would run */
 
@@ -100,7 +101,7 @@ int ccx_hip_event_record(void *ev, void *stream) { (void)ev; (void)stream; retur
 int ccx_hip_event_ms(void *start, void *stop, float *ms) { (void)start; (void)stop; *ms = 1.0f; return 0; }
 int ccx_hip_device_count(int *n) { *n = 1; return 0; }
 int ccx_hip_cu_count(int *n) { *n = 4; return 0; }
-const char *ccx_hip_last_error(void) { return "none"; }
+int ccx_hip_mem_info(size_t *room, size_t *total) { *room = (size_t)fake_room; *total = (size_t)fake_total; return 0; }
 int ccx_hip_form_kpad(int form) { return form == 1 ? 48 : form == 3 ? 256 : form >= 2 ? 64 : 4; }
 int ccx_hip_split_elem_bytes(int form) { return form == 2 ? 6 : 8; }
 size_t ccx_hip_adj_stage_doubles(void) { return 1024; }
