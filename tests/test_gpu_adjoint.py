@@ -151,11 +151,15 @@ def test_autograd_function_on_device_tensors():
         np.testing.assert_allclose(gk.cpu().numpy(), 3.0 * want[k], rtol=1e-13, atol=1e-300)
 
 
-@pytest.mark.parametrize("no,nu", [(2, 17), (2, 65), (2, 126), (2, 142), (2, 175), (2, 185)], ids=lambda v: str(v))
+# (3, 201) last: the CPU oracle takes about half a minute there
+@pytest.mark.parametrize("no,nu", [(2, 17), (2, 65), (2, 126), (2, 142), (2, 175), (2, 185), (2, 201), (3, 65),
+                                   (3, 126), (3, 201)], ids=lambda v: str(v))
 def test_back_contraction_tile_edges(no, nu):
-    """Gamma tiles 2, 5, 8, 9, 11 and 12 (two groups of 6), K tiles 2, 5, 8, 9 (two chunks of 5 and 4),
-    12 (two of 6); last blocks of 1, 1, 14, 14, 15 and 9 indices, so slices and contraction steps of
-    padding are left out on every axis."""
+    """Gamma tiles 2, 5, 8, 9, 11, 12 (two groups of 6) and 13 (6 and 7); gBX K chunks of 2, 5, 8, 4+5,
+    6+6 and 6+7 tiles; gAX of 2, 5, 8, 9 and 6+6 tiles in one launch and of 7+6 in two; last
+    blocks of 1, 1, 14, 14, 15, 9 and 9 indices, so slices and contraction steps of padding are left
+    out on every axis.  At no=2 every entry is a merged pair of weight 2, at no=3 the lists mix those
+    with a distinct tuple's entries of weight 1."""
     inp = synth.make_inputs(no, nu, 300 + nu)
     print(f"gradient no={no} nu={nu}", flush=True)
     want = dense.grad_tuplewise(inp)
@@ -209,3 +213,21 @@ def test_gradient_bitwise_deterministic_and_batched():
             os.environ["CCX_ADJ_BATCH_MB"] = old
     for k in KEYS:
         _close(c[k], a[k], 1e-13)
+
+
+def test_gradient_workspace_grows_and_is_reused(monkeypatch):
+    """Gradients of one context with batches of different sizes: the kept workspace is taken anew when
+    it must grow and used in part when it is larger; each result is bitwise that of a context
+    of its own with the same batch."""
+    inp = synth.make_inputs(4, 36, 1001)
+    ctx = TriplesContext(4, 36)
+    ctx.load(inp)
+    for mb in ("1", "8", "2", "64"):
+        print(f"gradient no=4 nu=36 batch {mb} MB", flush=True)
+        monkeypatch.setenv("CCX_ADJ_BATCH_MB", mb)
+        got, want = ctx.gradient(), _grad(inp)
+        for k in ("ets", "etd"):
+            assert got[k] == want[k], (mb, k)
+        for k in KEYS:
+            assert np.array_equal(got[k], want[k]), (mb, k)
+    ctx.close()

@@ -215,7 +215,7 @@ def test_workspace_grows_with_the_batch(host, monkeypatch, full_device):
     assert _room(host) >= before
 
 
-@pytest.mark.parametrize("nu,keeps", [(20, True), (260, False)], ids=["small", "282MB"])
+@pytest.mark.parametrize("nu,keeps", [(20, True), (260, False)], ids=["small", "272MiB"])
 def test_upload_buffer_is_kept_up_to_its_bound(host, nu, keeps):
     """The buffer of no=2, nu=260 is above the bound of 256 MiB: given back by every load."""
     sizes = {"eh": 2, "ep": nu, "t1": 2 * nu, "t2": 4 * nu ** 2, "vm": 8 * nu, "voe": 4 * nu ** 2, "vvvo": 2 * nu ** 3}
