@@ -89,10 +89,14 @@ int ccx_hip_nonfinite(const double *const *p, const size_t *n, int narr, unsigne
 
 /* The kernels (declared without parameters, so ccx_dev.h is not included here) */
 int ccx_hip_adj_items() { if (fake_during_adjoint) fake_during_adjoint(); return 0; }
+int fake_packed_routes;            /* virtual-triple sums that went through the packed copies */
+int ccx_hip_w_abc() { return 0; }
+int ccx_hip_abc_pack() { ++fake_packed_routes; return 0; }
+int ccx_hip_w_abc_packed() { return 0; }
 #define KERNEL(name) int name() { return 0; }
 KERNEL(ccx_hip_pack) KERNEL(ccx_hip_pack_ax_one) KERNEL(ccx_hip_pack_pairs) KERNEL(ccx_hip_triples)
 KERNEL(ccx_hip_pack_split) KERNEL(ccx_hip_pack_f32v) KERNEL(ccx_hip_finalize) KERNEL(ccx_hip_t1wt3)
-KERNEL(ccx_hip_w_abc) KERNEL(ccx_hip_abc_pack) KERNEL(ccx_hip_w_abc_packed) KERNEL(ccx_hip_x_abc)
+KERNEL(ccx_hip_x_abc)
 KERNEL(ccx_hip_gax) KERNEL(ccx_hip_gbx) KERNEL(ccx_hip_dvoe_reduce) KERNEL(ccx_hip_unpack_grad) KERNEL(ccx_hip_zero)
 
 int ccx_hip_event_create(void **ev) { *ev = NULL; return 0; }

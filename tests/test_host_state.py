@@ -226,3 +226,15 @@ def test_upload_buffer_is_kept_up_to_its_bound(host, nu, keeps):
         assert c.load(on_device=False) == OK
         assert (_room(host) < before) == keeps
     c.close()
+
+
+@pytest.mark.parametrize("no,packed", [(1, 0), (2, 1)])
+def test_one_occupied_orbital_does_not_take_the_matrix_route(host, no, packed):
+    """With one occupied orbital every cube is its one zeroed element: nothing to contract."""
+    c = Ctx(host, no, 20)
+    assert c.load() == OK
+    routes, etd = ctypes.c_int.in_dll(host, "fake_packed_routes"), ctypes.c_double()
+    before = routes.value
+    assert host.ccx_energy_abc(c.p, ctypes.byref(etd)) == OK
+    assert routes.value - before == packed
+    c.close()
