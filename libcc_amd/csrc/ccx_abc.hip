@@ -9,7 +9,8 @@
 //   W_ijk(a,b,c) = sum over the 6 simultaneous permutations s of the pairs (i,a),(j,b),(k,c)
 //                  of sum_K AX[i'](a',b',K) BX[j',k'](c',K).
 // This path is a cross-check and a surface for virtual-triple callers, not the hot path.  One
-// triple alone: one wave per (i,j,k), FP64 FMA on cached slab reads (w_abc_kernel).
+// triple alone, and lists of them where there is no room for copies of the slabs or nothing to win
+// from them: FP64 FMA on cached slab reads (w_abc_kernel).
 // The sum over all triples: each term s is the GEMM
 //   G_s[x][(y,z)] = sum_K AX[x](v_s0, v_s1, K) BX[y,z](v_s2, K),   no x no^2 x (nu+no),
 // on the FP64 matrix cores, from copies of the slabs with x and (y,z) innermost (w_abc_mfma_kernel).
@@ -20,23 +21,27 @@ namespace {
 
 constexpr int ABC_TB = 16;        // virtual block edge of the slab layouts
 constexpr int ABC_THR = 256;
+constexpr long long ABC_LANES = 24576;   // elements from which a lane each is the faster (ccx_hip_w_abc)
 constexpr int ABC_P[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
 __constant__ int ABC_PERM[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
 
 // V3 of triple t = (abc[4t], abc[4t+1], abc[4t+2]) into w[t * no^3 ...], column-major
 // (i fastest).  V3(i,i,i) is set to 0, as zerot3 does at the end of abc_tuple_formv3
 // (src/triples-abc/abc_tuple.f90:77); E[T] does not depend on those elements.
-// One wave per element, its lanes along K: a single triple has only no^3 elements, and with one lane
-// each its time was the 6 (nu + no) dependent slab reads of a lane (142 us at no=6, nu=64).
+// LPE lanes per element along K.  64 where the elements alone do not fill the chip: a single triple has
+// only no^3 of them, and with one lane each its time was the 6 (nu + no) dependent slab reads of
+// a lane (142 us at no=6, nu=64).  One for long lists: neighbouring lanes then read neighbouring x at
+// one K, where a wave along K fetches a line per lane and element.
+template <int LPE>
 __global__ void __launch_bounds__(ABC_THR) w_abc_kernel(const double *__restrict__ axr, const double *__restrict__ bx,
                                                         const int *__restrict__ trip, int ntrip, int no, int nu,
                                                         int nb, int kp, double *__restrict__ w)
 {
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x % LPE;
     const int no3 = no * no * no;
-    const long long total = (long long)ntrip * no3, nwave = (long long)gridDim.x * (ABC_THR / 64);
+    const long long total = (long long)ntrip * no3, step = (long long)gridDim.x * (ABC_THR / LPE);
     const int kn = nu + no;
-    for (long long id = blockIdx.x * (long long)(ABC_THR / 64) + (threadIdx.x >> 6); id < total; id += nwave) {
+    for (long long id = blockIdx.x * (long long)(ABC_THR / LPE) + threadIdx.x / LPE; id < total; id += step) {
         const int t = (int)(id / no3), e = (int)(id % no3);
         const int v[3] = {trip[4 * t], trip[4 * t + 1], trip[4 * t + 2]};
         const int o[3] = {e % no, (e / no) % no, e / (no * no)};
@@ -55,10 +60,11 @@ __global__ void __launch_bounds__(ABC_THR) w_abc_kernel(const double *__restrict
                 // BX: [y][z][c-block][K][gamma]
                 const double *bp = bx + (((long long)y * no + z) * nb + cv / ABC_TB) * ((long long)kp * 16) + cv % ABC_TB;
                 double sum = 0.0;
-                for (int K = lane; K < kn; K += 64) sum = fma(ap[(K >> 2) * 128 + (K & 3) * 32], bp[(long long)K * 16], sum);
+                for (int K = lane; K < kn; K += LPE) sum = fma(ap[(K >> 2) * 128 + (K & 3) * 32], bp[(long long)K * 16], sum);
                 acc += sum;
             }
-            for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
+#pragma unroll
+            for (int d = LPE / 2; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
         }
         if (lane == 0) w[id] = acc;
     }
@@ -243,9 +249,15 @@ int ccx_hip_w_abc(const void *axr, const void *bx, const int *trip, int ntrip, i
 {
     if (ntrip <= 0) return 0;
     if (kp % 4 != 0 || kp < nu + no) return 3;
-    const long long groups = ((long long)ntrip * no * no * no + ABC_THR / 64 - 1) / (ABC_THR / 64);
-    w_abc_kernel<<<(int)(groups < 65536 ? groups : 65536), ABC_THR, 0, (hipStream_t)stream>>>(
-        (const double *)axr, (const double *)bx, trip, ntrip, no, nu, nb, kp, w);
+    // A lane per element once those lanes fill the chip: 16384 elements (no=16, nu=40) took 61 us with a lane
+    // and 48 us with a wave each, 27648 (no=3, nu=120) 112 and 150 us, 16.8 M (no=16) 13.5 and 51.9 ms.
+    const long long total = (long long)ntrip * no * no * no;
+    const int lpe = total >= ABC_LANES ? 1 : 64;
+    const long long groups = (total * lpe + ABC_THR - 1) / ABC_THR;
+    const int grid = (int)(groups < 65536 ? groups : 65536);
+    const double *a = (const double *)axr, *b = (const double *)bx;
+    if (lpe == 1) w_abc_kernel<1><<<grid, ABC_THR, 0, (hipStream_t)stream>>>(a, b, trip, ntrip, no, nu, nb, kp, w);
+    else w_abc_kernel<64><<<grid, ABC_THR, 0, (hipStream_t)stream>>>(a, b, trip, ntrip, no, nu, nb, kp, w);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }
 

@@ -646,10 +646,10 @@ int ccx_energy_abc(ccx_ctx *c, double *etd)
         DALLOC(d_w, no3 * batch);
         DALLOC(d_x, batch);
         /* The packed copies of the matrix-core route (axt has the size of a slab, its occupied index
-         * padded to 16); without room for them the triples go through w_abc_kernel.  So they do at no=1,
-         * where a cube is its one zeroed element and w_abc_kernel contracts nothing (no=1, nu=200:
-         * 10.5 ms against 44.9); at no=2 the matrix cores win (nu=200: 46 ms against 98). */
-        if (c->no > 1 &&
+         * padded to 16); without room for them the triples go through w_abc_kernel.  So they do up to
+         * no=2, where the padding costs more than the matrix cores win: no=2, nu=200 34 ms
+         * against 46.7 with copies, no=3, nu=120 15.2 against 5.1. */
+        if (c->no > 2 &&
             (dev_malloc((void **)&d_axt, sizeof(double) * ccx_hip_abc_a_doubles((int)c->no, (int)c->nu, (int)c->kp)) != 0 ||
              dev_malloc((void **)&d_bxt, sizeof(double) * ccx_hip_abc_b_doubles((int)c->no, (int)c->nu, (int)c->kp)) != 0)) {
             ccx_hip_free(d_axt);

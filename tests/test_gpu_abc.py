@@ -81,6 +81,44 @@ def test_energy_abc_tile_edges(no, nu):
     ctx.close()
 
 
+# Lists of triples on the unpacked slabs, the route without room for the packed copies: below and above
+# the element count (24576) from which a lane, not a wave, takes an element
+@pytest.mark.parametrize("no,nu,ntrip", [(3, 17, 1), (3, 17, 910), (3, 17, 911), (2, 33, 5000), (5, 12, 5), (5, 12, 352),
+                                         (17, 5, 4), (17, 5, 30)], ids=lambda v: str(v))
+def test_w_abc_lists(no, nu, ntrip):
+    import torch
+
+    inp = synth.make_inputs(no, nu, 60 + no)
+    nup, kp = -(-nu // 16) * 16, -(-(nu + no) // 4) * 4
+    nb = nup // 16
+    dev = {k: torch.from_numpy(np.asfortranarray(v).ravel(order="F").copy()).cuda()
+           for k, v in inp.items() if isinstance(v, np.ndarray)}
+    slab = {k: torch.zeros(n, dtype=torch.float64, device="cuda") for k, n in {
+        "axr": no * nb * nb * kp * 256, "axc": no * nb * nb * kp * 256, "bx": no * no * nb * kp * 16,
+        "voe": no * no * nup * nup, "eh": no, "ep": nup, "t1": no * nu}.items()}
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    L = lib()
+    torch.cuda.synchronize()
+    assert L.ccx_hip_pack(0, *[p(dev[k]) for k in ("vvvo", "t2", "vm", "voe", "eh", "ep", "t1")],
+                          *[p(slab[k]) for k in ("axr", "axc", "bx", "voe", "eh", "ep", "t1")], no, nu, nup, kp, None) == 0
+    trip = [(a, b, c, 1) for a in range(nu) for b in range(a + 1) for c in range(b + 1) if not a == b == c][:ntrip]
+    assert len(trip) == ntrip
+    tr = torch.tensor(trip, dtype=torch.int32, device="cuda")
+    w = torch.full((ntrip * no ** 3,), float("nan"), dtype=torch.float64, device="cuda")
+    print(f"w_abc list no={no} nu={nu} ntrip={ntrip}", flush=True)
+    torch.cuda.synchronize()
+    assert L.ccx_hip_w_abc(p(slab["axr"]), p(slab["bx"]), p(tr), ntrip, no, nu, nb, kp, p(w), None) == 0
+    torch.cuda.synchronize()
+    got = w.cpu().numpy().reshape(ntrip, no, no, no).transpose(0, 3, 2, 1)      # i fastest
+    full = dense.w_dense(inp["t2"], inp["vm"], inp["vvvo"])                     # [i, j, k, a, b, c]
+    t = np.array(trip)
+    want = full[:, :, :, t[:, 0], t[:, 1], t[:, 2]].transpose(3, 0, 1, 2).copy()
+    i = np.arange(no)
+    want[:, i, i, i] = 0.0
+    # 6 (nu + no) products in another order
+    assert np.abs(got - want).max() <= 1e-12 * np.abs(want).max()
+
+
 def test_abc_errors():
     ctx = TriplesContext(2, 5)
     v3 = np.zeros(8)

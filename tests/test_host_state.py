@@ -228,9 +228,10 @@ def test_upload_buffer_is_kept_up_to_its_bound(host, nu, keeps):
     c.close()
 
 
-@pytest.mark.parametrize("no,packed", [(1, 0), (2, 1)])
-def test_one_occupied_orbital_does_not_take_the_matrix_route(host, no, packed):
-    """With one occupied orbital every cube is its one zeroed element: nothing to contract."""
+@pytest.mark.parametrize("no,packed", [(1, 0), (2, 0), (3, 1)])
+def test_virtual_triple_route(host, no, packed):
+    """The matrix cores take 16 occupied indices at a time: not for one (whose cubes are their one
+    zeroed element) or two."""
     c = Ctx(host, no, 20)
     assert c.load() == OK
     routes, etd = ctypes.c_int.in_dll(host, "fake_packed_routes"), ctypes.c_double()
