@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(NTHR, 1) adj_item_kernel(AdjArgs ga)
 namespace {
 constexpr int GTHR = 512;                 // GEMM work group: 8 waves, 2 per SIMD
 constexpr int GBPW = 2;                   // gax: rows b per wave
-constexpr int GAX_CT = 11;                // gax: most K tiles of a work group (accumulator registers)
+constexpr int GAX_CT = 12;                // gax: most K tiles of a work group (ccx_hip_gax)
 constexpr int BS_STR = 17;                // padded row of the staged BX slices
 typedef double d2 __attribute__((ext_vector_type(2)));
 constexpr int GBX_TILES = 19;             // gbx: gamma and K tiles of a work group (two 4 KB buffers each)
@@ -467,7 +467,7 @@ struct GemmArgs {
 
 // gAX[x](R0 16 x R1 16 rows, K chunk) += sum over entries (t,sigma) with t[xp] = x and over
 // the gamma blocks G of Wbar_t(e_u = a, e_v = b, e_wf = g) BX[t[yp],t[zp]](g, K).
-// Wave w owns rows b in {2w, 2w+1}, all 8 K tiles of the chunk.
+// Wave w owns rows b in {2w, 2w+1}, all NCT K tiles of the chunk.
 // NCT: K tiles of 16 the work group computes, from column a.k0 + 16 NCT times its chunk; the launcher
 // splits K evenly, so no MFMA runs on K padding.  Contraction steps past the last virtual index, and
 // the MFMAs of waves whose two rows b lie past it, are left out.
@@ -968,9 +968,11 @@ int ccx_hip_gax(const double *wbar, const double *bx, double *gax, const int *tu
     a.ulist = xlist; a.uoff = xoff; a.ent = ent;
     a.no = no; a.nu = nu; a.nup = nup; a.nb = nup / TB; a.kp = kp; a.nx = nx;
     hipStream_t s = (hipStream_t)stream;
-    // As few chunks as GAX_CT tiles of accumulators allow, since every chunk stages the Wbar blocks
-    // again (11 of 80 ms at no=14, nu=150 with a chunk of 8 tiles and one of 3), split evenly: q tiles
-    // a chunk, one more for the first nk % n of them.
+    // As few chunks as possible, since every chunk stages the Wbar blocks again (11 of 80 ms at no=14,
+    // nu=150 with a chunk of 8 tiles and one of 3).  A chunk holds at most GAX_CT = 12 tiles: gax_kernel<12> takes 254
+    // registers and no scratch, <13> spills 76 B a lane.  With at most 11 a gradient whose K has 12 tiles (no=12, nu=176) took
+    // 243.2 ms, with 12 235.2; of 24 tiles (no=4, nu=372) 149.5 and 146.3.  Split evenly: q tiles a chunk, one
+    // more for the first nk % n of them.
     const int nk = (kp + 15) / 16, n = (nk + GAX_CT - 1) / GAX_CT, q = nk / n, more = nk % n;
     const long long grid = (long long)nx * a.nb * a.nb;
     int rc = 0;

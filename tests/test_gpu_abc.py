@@ -68,7 +68,7 @@ def test_energy_abc_matches_ijk(no, nu, seed):
 
 # Edges of the matrix-core route's tiles: no^2 below, at and above multiples of 16 pair tiles (one to
 # four tiles per wave, one or four waves per triple), no below, at and above one row tile.
-@pytest.mark.parametrize("no,nu", [(2, 7), (4, 16), (5, 18), (7, 12), (8, 17), (9, 10), (12, 6), (16, 5), (17, 4)],
+@pytest.mark.parametrize("no,nu", [(2, 7), (3, 9), (4, 16), (5, 18), (7, 12), (8, 17), (9, 10), (12, 6), (16, 5), (17, 4)],
                          ids=lambda v: str(v))
 def test_energy_abc_tile_edges(no, nu):
     inp = synth.make_inputs(no, nu, 40 + no)

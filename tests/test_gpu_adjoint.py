@@ -156,7 +156,7 @@ def test_autograd_function_on_device_tensors():
                                    (3, 126), (3, 201)], ids=lambda v: str(v))
 def test_back_contraction_tile_edges(no, nu):
     """Gamma tiles 2, 5, 8, 9, 11, 12 (two groups of 6) and 13 (6 and 7); gBX K chunks of 2, 5, 8, 4+5,
-    6+6 and 6+7 tiles; gAX of 2, 5, 8, 9 and 6+6 tiles in one launch and of 7+6 in two; last
+    6+6 and 6+7 tiles; gAX chunks of 2, 5, 8, 9 and 12 tiles in one launch and of 7+6 in two; last
     blocks of 1, 1, 14, 14, 15, 9 and 9 indices, so slices and contraction steps of padding are left
     out on every axis.  At no=2 every entry is a merged pair of weight 2, at no=3 the lists mix those
     with a distinct tuple's entries of weight 1."""
