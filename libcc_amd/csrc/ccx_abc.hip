@@ -22,8 +22,7 @@ namespace {
 constexpr int ABC_TB = 16;        // virtual block edge of the slab layouts
 constexpr int ABC_THR = 256;
 constexpr long long ABC_LANES = 24576;   // elements from which a lane each is the faster (ccx_hip_w_abc)
-constexpr int ABC_P[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
-__constant__ int ABC_PERM[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+__device__ constexpr int ABC_PERM[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
 
 // V3 of triple t = (abc[4t], abc[4t+1], abc[4t+2]) into w[t * no^3 ...], column-major
 // (i fastest).  V3(i,i,i) is set to 0, as zerot3 does at the end of abc_tuple_formv3
@@ -49,7 +48,7 @@ __global__ void __launch_bounds__(ABC_THR) w_abc_kernel(const double *__restrict
         if (!(o[0] == o[1] && o[1] == o[2])) {
 #pragma unroll
             for (int s = 0; s < 6; ++s) {
-                const int p0 = ABC_P[s][0], p1 = ABC_P[s][1], p2 = ABC_P[s][2];
+                const int p0 = ABC_PERM[s][0], p1 = ABC_PERM[s][1], p2 = ABC_PERM[s][2];
                 const int x = o[p0], y = o[p1], z = o[p2];
                 const int av = v[p0], bv = v[p1], cv = v[p2];
                 // row layout of AX (axr): panel (x, a-block, b-block), then

@@ -1103,8 +1103,8 @@ static void te_free(void)
 }
 
 /* Layout of a call's small inputs, in doubles: eps_virtual padded to nup; eps_occupied of the slots
- * (four, the last unused) and the tuple table entry (four ints, two doubles; two unused); then for each of the six ordered position pairs VM (no nu)
- * and VOE (nu^2). */
+ * (four, the last unused); the tuple table entry (four ints, two doubles) and two unused; then for each of
+ * the six ordered position pairs VM (no nu) and VOE (nu^2). */
 static int64_t te_small_doubles(int64_t no, int64_t nu, int64_t nup) { return nup + 8 + 6 * (no * nu + nu * nu); }
 
 /* the workspace for (no, nu), allocated on first use and whenever the dimensions change */

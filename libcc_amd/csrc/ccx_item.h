@@ -799,8 +799,8 @@ __device__ __forceinline__ void run_phase_split(const TriplesArgs &g, const Item
     };
     // A ring step is SPS operand slots and BS of the wave's batches: one slot of both batches.
     // Two bf16 slots per step (a longer prefetch distance) measured 4 % (BF16x3) and 12 %
-    // (BF16x4) slower at no=24, nu=216: the larger ring costs registers, and the sweep is not
-    // waiting on its loads.  The 32-byte fp8 fragments took one batch per step while the
+    // (BF16x4) slower at no=24, nu=216, but that was while every block waited for all its loads
+    // once, which hides what a longer distance does: not measured since.  The 32-byte fp8 fragments took one batch per step while the
     // compiler spilled the sweep; with the MFMAs pinned to their block (pin_accumulators) both
     // batches fit: 879 ms against 1271 ms.
     typedef split_frag_t<FK> frag_t;
