@@ -717,7 +717,9 @@ __device__ __forceinline__ void run_phase_split(const TriplesArgs &g, const Item
     // BX staging: block kb in lb0 (even) or lb1 (odd).  Where they are two LDS arrays of their own the
     // compiler knows that the direct loads into one do not alias the reads of the other; in one
     // array it waited for every outstanding load (the next block's BX and the next AX fragments,
-    // just issued) before the first read of each K block: 175 ms at no=16, nu=181 in the BF16x3 form.
+    // just issued) before the first read of each K block: 175 ms at no=16, nu=181 in the BF16x3 form, 94 now.
+    // (The adjoint's buffers are pieces of one array at constant distance, and with the buffer loads below
+    // its listing has no such wait either.)
     typedef SplitCfg<FK> CF;
     constexpr int SM = slot_mask(PHASE, MODE), XM = bx_mask(PHASE, MODE);
     constexpr int NSL = __builtin_popcount(SM), NBX = __builtin_popcount(XM);
@@ -990,7 +992,7 @@ __device__ __forceinline__ void run_phase_f32v(const TriplesArgs &g, const ItemC
     }
     // BX operand c of a block goes from global memory straight into LDS (buffer load, as in
     // run_phase_split), loaded by wave c.  Through a register (whose next load had to wait for
-    // everything outstanding) the sweep stalled once a block: 753 ms at no=24, nu=216.
+    // everything outstanding) the sweep stalled once a block: 753 ms at no=24, nu=216, 650 now.
     typedef __attribute__((address_space(3))) void lds_void;
     int pg = 0;
     static_for<NBX>([&](auto R) __attribute__((always_inline)) {

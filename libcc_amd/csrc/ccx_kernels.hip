@@ -341,7 +341,8 @@ namespace {
 // and row swaps, by their LDS shuffles.  Of 475 kcycles per item at no=24, nu=216 the point loop took
 // 15.8 and now takes 10.4 (two multiply-adds per v1 term instead of five operations), the
 // reductions 15.9 and now 7.5; the kernel went from 1137 to 1109 ms there, from 4.79 to 4.49 ms
-// at no=8, nu=120, where an item's sweeps are half as long, and FP32 from 783 to 753 ms.
+// at no=8, nu=120, where an item's sweeps are half as long (energy calls repeated on loaded slabs; 4.57 when
+// a load comes before each), and FP32 from 783 to 753 ms (650 since its BX goes straight into LDS).
 template <class T, int FK>
 __device__ __forceinline__ void item_epilogue(const TriplesArgs &g, double *lds, double (*red)[112], const ItemCtx &it,
                                               const typename Mfma<T>::acc_t (&acc)[6][BPW],
