@@ -24,7 +24,7 @@ def _solve(inp, packed):
 
 
 # no (no-1) (no+4) / 6 tuples, 2 (no=2) to 352 (no=12); the reduction takes its table 256 at a time, which
-# lies between no=10 (210 tuples, one round) and no=11 (275, two)
+# lies between no=10 (210 tuples, one pass) and no=11 (275, two)
 @pytest.mark.parametrize("no,nu", [(2, 15), (3, 16), (2, 17), (4, 30), (5, 31), (3, 33), (2, 47), (10, 5), (11, 5),
                                    (12, 18)], ids=lambda v: str(v))
 def test_layouts_agree_and_match_oracle(no, nu):
